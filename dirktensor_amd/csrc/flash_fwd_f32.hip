@@ -8,33 +8,54 @@
 // round folds its units instead (flash_items.h): an item is then the 64-query
 // tiles p and n-1-p of one (batch, head), rows 0-63 and 64-127.
 //
+// Products. Every fp32 operand x is split into three bf16 values x = h + m + l
+// (each the rounding of what the ones before it leave: 24 significand bits in
+// three times 8, so the sum is x itself), and a product x y is formed on
+// v_mfma_f32_32x32x16_bf16 from the six partial products of weight 2^-16 and
+// above (lh, hl, mm, mh, hm, hh; the three left out are below 2^-26 of x y),
+// accumulated in fp32. Six bf16 MFMAs take 192 cycles for 16 steps of k where
+// v_mfma_f32_32x32x2_f32 takes 512, and the result is nearer to the exact one:
+// over random 128-long dot products the relative error (2-norm) is 6.1e-8 with
+// the small partial products summed first, against 2.0e-7 for the fp32
+// instruction, which rounds after every second k instead of after every sixteenth.
+// Infinities and the last binade do not split (inf * 0 in a partial product is
+// NaN, and rounding to bf16 overflows), and below 2^-109 the last part falls under
+// bf16's smallest denormal. A wave whose result is not finite, whose softmax is empty
+// where it has keys, or whose queries or output lie outside [2^-100, 2^100],
+// therefore repeats its keys with the fp32 instruction, straight from memory
+// (slow_keys), and keeps that result.
+//
 // Work split: 8 waves in two groups of 4. Both groups hold the same 128 queries
 // (32 per wave) and split the key tiles: group g takes tiles g, g+2, g+4, ... At
-// the end group 1 hands its partial (max, sum, O) to group 0 through LDS and
-// group 0 merges them with the same rescale the reference applies between tiles
-// (FlashAttention.cpp:134-156). Each wave computes S^T = K Q^T for its 32
-// queries with v_mfma_f32_32x32x2_f32, so that in the accumulator layout one
-// lane holds one query (lane % 32) and 16 keys; the row max / row sum of the
-// online softmax are then a per-lane reduction plus one exchange with lane ^ 32.
-// The probabilities stay in the accumulator registers and feed the PV product
-// O^T += V^T P^T directly as the B operand (the MFMA's k index is only a
-// summation label, so V rows are read in the accumulator's key order).
+// the end the two partials (m, l, O) are merged through LDS with the same rescale
+// the reference applies between tiles (FlashAttention.cpp:134-156), each group
+// finalising half of the dims. Each wave computes S^T = K Q^T for its 32 queries,
+// so that in the accumulator layout one lane holds one query (lane % 32) and 16
+// keys; the row max / row sum of the online softmax are then a per-lane reduction
+// plus one exchange with lane ^ 32. The probabilities stay in registers, are split
+// there and feed the PV product O^T += V^T P^T as the B operand (the MFMA's k
+// index is only a summation label, so V rows are read in the accumulator's key
+// order, by the transposing ds_read_b64_tr_b16).
 //
-// K and V tiles move from HBM straight into LDS with buffer_load ... lds,
-// double-buffered: while a step computes on one stage, the group's next tile
-// streams into the other; one barrier per step. Descriptors end at the
-// sequence's last valid key, so rows past it arrive as zeros. LDS rows are 512
-// bytes (128 floats), unpadded; the 16-byte chunk c of row r is stored at chunk
-// position c ^ (r & 15), which keeps the row-wise K reads (16 rows, one chunk
-// each) and the column-block V reads (one row, 16 chunks) free of bank conflicts.
+// K and V tiles pass through registers on their way to LDS: a wave loads a quarter of its group's tile (four floats
+// per lane and row pair), one half step ahead, splits it and writes the three bf16 planes, V's under the MFMAs of the
+// S product and the next K's under those of the PV product, so the split has no phase of its own: two barriers per
+// step, K planes free and V planes ready at one, the other way round at the other. Group 1 runs half a step behind
+// group 0, and a wave in its S product and softmax has the higher issue priority, so that one group's softmax issues
+// under the other's PV product. Plane rows are padded (K's 272 bytes, V's 320) so that the row-wise K reads and the
+// transposing V reads fall in different banks and every LDS address is one register plus a constant.
+//
+// What bounds it: the matrix pipe is busy 6144 of the ~9600 cycles of a step (two waves per SIMD, 96 MFMAs each); the
+// rest is the split (without it 95 us where the kernel takes 118, B = 2, T = 1500, H = 16) and the softmax's first
+// half. Before, on v_mfma_f32_32x32x2_f32: 201 us there, and at B = 1, T = 64, 16.5 us against 13.0. Fragments
+// prefetched in finer steps, and the tiles staged as fp32 in LDS by DMA instead of through registers, took 128 and 120.
 //
 // Numerics follow the reference: S = scale * Q K^T (FlashAttention.cpp:83-91),
 // keys with k_pos > q_pos masked (:102), m = row max of the scaled scores,
 // l = sum exp(s - m) (:159-163), output O / l, and a row with l == 0 written as
-// zeros (:165-174). The online rescale uses the running max directly
-// (FA-2 form) instead of the reference's tile-local max with alpha/beta
-// factors (:134-156); both equal sum_k exp(s_k - m_final) up to rounding.
-// exp is evaluated as exp2 with log2(e) folded into the scale.
+// zeros (:165-174). The softmax runs in the log2 domain on Q scale log2(e), with
+// a reference point that moves only when a score exceeds it by 2^8; m is the true
+// row maximum and l is rescaled to it at the end.
 
 #include "flash_items.h"
 
@@ -45,22 +66,37 @@ namespace dt {
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef short shortx4 __attribute__((ext_vector_type(4)));
+typedef short shortx8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
 
 constexpr int kD = 128;                      // head_dim (model_config.h:3)
 constexpr int kBM = kItemRows;               // queries per item
 constexpr int kBN = 32;                      // keys per tile
 constexpr int kThreads = 512;                // 8 waves
-constexpr int kRowBytes = kD * 4;            // one K or V row, unpadded
-constexpr int kTileBytes = kBN * kRowBytes;  // 16 KB per tensor per tile
+constexpr int kRowK = kD * 2 + 16;           // a row of one of K's planes
+constexpr int kRowV = kD * 2 + 64;           // a row of one of V's planes
+constexpr int kPlaneK = kBN * kRowK;
+constexpr int kPlaneV = kBN * kRowV;
+constexpr int kGroupBytes = 3 * (kPlaneK + kPlaneV);  // 55.5 KB
+constexpr int kObufRow = kD * 4 + 16;        // a row of the output staging tile
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kNegInf = -__builtin_huge_valf();
+constexpr float kInf = __builtin_huge_valf();
+constexpr float kRescaleLog2 = 8.0f;
+constexpr float kWide = 0x1p100f;
 constexpr int kBufferDword3 = 0x00020000;  // raw buffer, 32-bit data format (gfx9 family)
 
-// one LDS stage: [group][K, V][tile bytes]
-typedef uint8_t Stage[2][2][kTileBytes];
-
-__device__ __forceinline__ float xor32(float v) { return __shfl_xor(v, 32, 64); }
+// LDS: the groups' planes [group](K h, m, l, V h, m, l) in the loop; at an item's end the exchange between the groups
+// (xo, xs) and the output tile
+constexpr int kXoBytes = 2 * 4 * 8 * 64 * 16;   // 64 KB
+constexpr int kXsBytes = 2 * 4 * 3 * 64 * 4;    // 6 KB
+constexpr int kLdsBytes = kXoBytes + kXsBytes + kBM * kObufRow;
+static_assert(2 * kGroupBytes <= kLdsBytes && kLdsBytes <= 160 * 1024, "LDS of one CU");
 
 template <typename F, int... Is>
 __device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, Is...>) {
@@ -71,58 +107,149 @@ template <int N, typename F>
 __device__ __forceinline__ void static_for(F&& f) {
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
-// keeps each group of MFMAs with the LDS read issued beside it: the scheduler may not move work across
+// keeps each group of MFMAs with the LDS accesses issued beside it: the scheduler may not move work across
 #define DT_BUNDLE_END __builtin_amdgcn_sched_barrier(0)
 
-// chunk position of 16-byte chunk c of an LDS row r
-__device__ __forceinline__ int pos(int r, int c) { return c ^ (r & 15); }
+__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
+    bf16x2 r = __builtin_convertvector((floatx2){lo, hi}, bf16x2);
+    return __builtin_bit_cast(uint32_t, r);
+}
+// the bf16 planes of a pair of floats: x = h + m + l exactly for finite x below 2^127
+struct Split2 {
+    uint32_t h, m, l;
+};
+__device__ __forceinline__ Split2 split2(float x0, float x1) {
+    Split2 s;
+    s.h = pack_bf16x2(x0, x1);
+    const float r0 = x0 - __uint_as_float(s.h << 16), r1 = x1 - __uint_as_float(s.h & 0xffff0000u);
+    s.m = pack_bf16x2(r0, r1);
+    s.l = pack_bf16x2(r0 - __uint_as_float(s.m << 16), r1 - __uint_as_float(s.m & 0xffff0000u));
+    return s;
+}
+// an operand's three planes
+struct Frag3 {
+    bf16x8 h, m, l;
+};
+__device__ __forceinline__ floatx16 mfma(bf16x8 a, bf16x8 b, floatx16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// Row reductions over the two lane halves (lane l and lane l ^ 32 hold the same query): v_permlane32_swap with x as
+// both operands leaves the lower half's value and the upper half's in every lane (the same order in both halves).
+__device__ __forceinline__ float max_halves(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float sum_halves(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
 
 // Buffer descriptor over [base, base + bytes): loads at or past the end return zeros.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, kBufferDword3);
 }
 
-// LDS DMA issued through inline assembly: the compiler does not track these loads, so it does not wait
-// for them before reading the other LDS stage; stage_barrier() waits for them before any wave reads the
-// stage they fill. M0 (an operand bound to M0) holds the wave-uniform LDS destination; lane i writes 16
-// bytes at M0 + 16*i.
-// The compiler cannot insert the wait states the hardware needs before these instructions (5 after a VALU
-// write of an SGPR they read, such as a v_readlane reload of the descriptor; 1 after an SALU write of M0),
-// since it does not see inside the asm: s_nop 4 provides them.
-__device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(const lds_void*)p; }
-__device__ __forceinline__ void dma16(uint32_t lds, uint32_t voff, __amdgpu_buffer_rsrc_t r) {
-    asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "{m0}"(lds) : "memory");
+__device__ __forceinline__ float4 load16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
 }
 
-// this wave's DMA and LDS accesses are complete before any wave passes
-__device__ __forceinline__ void stage_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-// LDS accesses only: vector memory requests in flight (output stores) are not waited for
+// LDS accesses only: vector memory requests in flight (the next tiles, output stores) are not waited for
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// Per-wave state of one item: O^T: o[db][i] = O[qrow][32*db + 8*(i/4) + 4*hh + i%4] (unnormalised, relative to m_s)
+struct Acc {
+    floatx16 o[4];
+    float m_t, m_s, l;  // this lane half's maximum, the reference point (the same in both halves), this half's sum
+};
+
+// The wave's keys with v_mfma_f32_32x32x2_f32, operands straight from memory: tiles kt0, kt0 + 2, ... of the queries'
+// visible ones. Taken when the split products gave a result that is not finite; scores that are -inf, +inf or NaN
+// in fp32 arithmetic come out as such here.
+__device__ __noinline__ void slow_keys(Acc& A, const float* q, const float* K, const float* V, int ldk, int ldv, int kt0,
+                                       int n_tiles, int qw0, int lim, int L, int T, int causal, float c) {
+    const int lane = threadIdx.x & 63, ln = lane & 31, hh = lane >> 5;
+    float m_run = kNegInf, l_run = 0.0f;
+    for (int db = 0; db < 4; ++db)
+        for (int i = 0; i < 16; ++i) A.o[db][i] = 0.0f;
+    for (int kt = kt0; kt < n_tiles; kt += 2) {
+        const int k0 = kt * kBN;
+        if (causal && k0 > qw0 + 31) break;
+        floatx16 st;
+        for (int i = 0; i < 16; ++i) st[i] = 0.0f;
+        // k step s of lane half hh is dim 64*hh + s; keys past L read as zeros (and are masked)
+        const float* kp = K + (int64_t)min(k0 + ln, T - 1) * ldk + 64 * hh;
+        const bool kv = k0 + ln < L;
+        for (int s = 0; s < 64; ++s) {
+            const float kx = kp[s], qx = q[64 * hh + s];
+            st = __builtin_amdgcn_mfma_f32_32x32x2f32(kv ? kx : 0.0f, qx, st, 0, 0, 0);
+        }
+        float tmax = kNegInf;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            if (k0 + 8 * (i / 4) + 4 * hh + (i % 4) > lim) st[i] = kNegInf;
+            tmax = fmaxf(tmax, st[i]);
+        }
+        const float m_new = fmaxf(m_run, max_halves(tmax) * c);
+        const float m_use = (m_new == kNegInf) ? 0.0f : m_new;
+        const float alpha = exp2f(m_run - m_use);  // 0 when m_run == -inf
+        float psum = 0.0f;
+        {
+#pragma clang fp contract(off)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                st[i] = __builtin_amdgcn_exp2f(st[i] * c - m_use);
+                psum += st[i];
+            }
+        }
+        l_run = l_run * alpha + psum;  // this half's keys
+        m_run = m_new;
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) A.o[db][i] *= alpha;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int key = k0 + 8 * (i / 4) + 4 * hh + (i % 4);
+            const float* vp = V + (int64_t)min(key, T - 1) * ldv + ln;
+#pragma unroll
+            for (int db = 0; db < 4; ++db) {
+                const float vx = vp[32 * db];
+                A.o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(key < L ? vx : 0.0f, st[i], A.o[db], 0, 0, 0);
+            }
+        }
+    }
+    A.m_t = A.m_s = m_run;
+    A.l = l_run;
+}
+
 __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a, Schedule sc) {
-    __shared__ __attribute__((aligned(1024))) Stage stage0;
-    __shared__ __attribute__((aligned(1024))) Stage stage1;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[kLdsBytes];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave >> 2;  // key-tile group
-    // 32-query block within the item (also this wave's share of a DMA tile); in a folded launch group 1's
-    // waves take the blocks in the other half, so each SIMD holds one wave of each 64-query tile
-    const int wq = (wave & 3) ^ (sc.fold ? 2 * grp : 0);
+    // 32-query block within the item, also this wave's quarter of the group's tiles. Group 1's waves take the blocks
+    // in the other half, so each SIMD (waves w and w + 4) holds one wave of each 64 queries: an item whose second
+    // 64 rows lie past the sequence's end, or see more keys than its first, still keeps all four SIMDs busy.
+    const int wq = (wave & 3) ^ (2 * grp);
     const int ln = lane & 31;   // query within the wave's 32 (MFMA n index)
-    const int hh = lane >> 5;   // lane half (MFMA k index)
+    const int hh = lane >> 5;   // lane half
 
-    // DMA: instruction n of wave wq fills LDS rows 2*(4n + wq) and 2*(4n + wq) + 1 of a tile (1 KB, 16 bytes
-    // per lane at chunk position lane % 32); the lane fetches the global chunk that the swizzle puts there.
-    uint32_t koff[4], voff[4];
-#pragma unroll
-    for (int n = 0; n < 4; ++n) {
-        const int r = 2 * (4 * n + wq) + hh;
-        const int c = pos(r, ln);  // pos is an involution: the chunk stored at position ln
-        koff[n] = (uint32_t)((r * a.ldk + 4 * c) * 4);
-        voff[n] = (uint32_t)((r * a.ldv + 4 * c) * 4);
-    }
+    // K fragment chunk cc of row ln: dims 16*cc + 8*hh .. +8
+    const uint8_t* const kfrag = lds + grp * kGroupBytes + ln * kRowK + 16 * hh;
+    // V transposing reads: lane i of 16-lane group G reads row 4*hh + i/4 (+8 for the second read) of a 16-key chunk,
+    // dims 32*db + 16*(G&1) + 4*(i&3) .. +3
+    const int i16 = lane & 15;
+    const uint8_t* const vfrag =
+        lds + grp * kGroupBytes + 3 * kPlaneK + (4 * hh + (i16 >> 2)) * kRowV + 32 * ((lane >> 4) & 1) + 8 * (i16 & 3);
+    // this wave's quarter of a tile: unit n is rows 8*n + 2*wq and 8*n + 2*wq + 1, four floats per lane
+    const int r0 = 2 * wq + hh;
+    uint8_t* const kput = lds + grp * kGroupBytes + r0 * kRowK + 8 * ln;
+    uint8_t* const vput = lds + grp * kGroupBytes + 3 * kPlaneK + r0 * kRowV + 8 * ln;
+    const uint32_t koff = (uint32_t)((r0 * a.ldk + 4 * ln) * 4);
+    const uint32_t voff = (uint32_t)((r0 * a.ldv + 4 * ln) * 4);
 
     const int T = a.T;
     const int G = gridDim.x;
@@ -159,203 +286,322 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
         const int k_end = a.causal ? min(u.qb + 64, L) : L;
         const int n_tiles = (k_end + kBN - 1) / kBN;
         const int n_steps = (n_tiles + 1) / 2;
+        const int lim = a.causal ? min(qrow, L - 1) : L - 1;  // keys > lim are masked
 
-        // K and V of tile kt of this group -> one LDS stage, straight from HBM
-        auto dma = [&](Stage& stg, int kt) {
-            const int k0 = kt * kBN;
-            const __amdgpu_buffer_rsrc_t rk = make_rsrc(Kg + (int64_t)k0 * a.ldk, (uint32_t)(L - k0) * (uint32_t)a.ldk * 4u);
-            const __amdgpu_buffer_rsrc_t rv = make_rsrc(Vg + (int64_t)k0 * a.ldv, (uint32_t)(L - k0) * (uint32_t)a.ldv * 4u);
-            const uint32_t lk = __builtin_amdgcn_readfirstlane(lds_addr(&stg[grp][0][wq * 1024]));
-            const uint32_t lv = __builtin_amdgcn_readfirstlane(lds_addr(&stg[grp][1][wq * 1024]));
-#pragma unroll
-            for (int n = 0; n < 4; ++n) dma16(lk + 4096 * n, koff[n], rk);
-#pragma unroll
-            for (int n = 0; n < 4; ++n) dma16(lv + 4096 * n, voff[n], rv);
+        // unit n of this wave's quarter of the group's tile kt of K (kv = 0) or V (kv = 1), on its way from HBM (zeros
+        // past the sequence; nothing is fetched past the last tile)
+        const __amdgpu_buffer_rsrc_t rk = make_rsrc(Kg, (uint32_t)L * (uint32_t)a.ldk * 4u);
+        const __amdgpu_buffer_rsrc_t rv = make_rsrc(Vg, (uint32_t)L * (uint32_t)a.ldv * 4u);
+        auto load = [&](int kv, int kt, int n) {
+            const uint32_t ld4 = (uint32_t)(kv ? a.ldv : a.ldk) * 4u;
+            const uint32_t row = kt < n_tiles ? (uint32_t)(kt * kBN + 8 * n) * ld4 : 0x80000000u;
+            return load16(kv ? rv : rk, (kv ? voff : koff) + row);
         };
-        // the first tile streams in while the query row loads
-        if (grp < n_tiles) dma(stage0, grp);
-
-        // Q fragment in registers: q[4*j + e] = Q[qrow][8*j + 4*hh + e] (B operand of S^T = K Q^T); all
-        // sixteen loads are in flight before the first is used
-        float q[64];
-        {
-            float4 raw[16];
-            if (qrow < T) {
-                const float* qp = Qg + (int64_t)qrow * a.ldq + 4 * hh;
+        // that unit -> the planes
+        auto put = [&](int kv, int n, float4 x) {
+            const Split2 s0 = split2(x.x, x.y), s1 = split2(x.z, x.w);
+            uint8_t* p = kv ? vput + n * 8 * kRowV : kput + n * 8 * kRowK;
+            const int plane = kv ? kPlaneV : kPlaneK;
+            *reinterpret_cast<uint2*>(p) = make_uint2(s0.h, s1.h);
+            *reinterpret_cast<uint2*>(p + plane) = make_uint2(s0.m, s1.m);
+            *reinterpret_cast<uint2*>(p + 2 * plane) = make_uint2(s0.l, s1.l);
+        };
+        float4 x[4];  // the units between HBM and the planes: K's and V's in turn
+        float4 xk[4];
 #pragma unroll
-                for (int j = 0; j < 16; ++j) raw[j] = *reinterpret_cast<const float4*>(qp + 8 * j);
+        for (int n = 0; n < 4; ++n) xk[n] = load(0, grp, n);
+
+        // Q fragment, times scale * log2 e, split: qf[cc] = Q[qrow][16*cc + 8*hh .. +8] * c
+        Frag3 qf[8];
+        bool q_wide;  // values whose products a split may not hold in full
+        {
+            const float* qp = Qg + (int64_t)min(qrow, T - 1) * a.ldq + 8 * hh;  // (rows past T: any values)
+            float4 xq[16];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) xq[j] = *reinterpret_cast<const float4*>(qp + 16 * (j >> 1) + 4 * (j & 1));
+#pragma unroll
+            for (int n = 0; n < 4; ++n) x[n] = load(1, grp, n);
+#pragma unroll
+            for (int n = 0; n < 4; ++n) put(0, n, xk[n]);  // the group's first K tile
+            float qmax = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 16; ++j)
+                qmax = fmaxf(qmax, fmaxf(fmaxf(fabsf(xq[j].x), fabsf(xq[j].y)), fmaxf(fabsf(xq[j].z), fabsf(xq[j].w))));
+            qmax = max_halves(qmax);
+            q_wide = qmax > kWide || (qmax < 1.0f / kWide && qmax > 0.0f);
+#pragma unroll
+            for (int cc = 0; cc < 8; ++cc) {
+                const float4 x0 = xq[2 * cc], x1 = xq[2 * cc + 1];
+                const Split2 s0 = split2(x0.x * c, x0.y * c), s1 = split2(x0.z * c, x0.w * c);
+                const Split2 s2 = split2(x1.x * c, x1.y * c), s3 = split2(x1.z * c, x1.w * c);
+                qf[cc].h = __builtin_bit_cast(bf16x8, make_uint4(s0.h, s1.h, s2.h, s3.h));
+                qf[cc].m = __builtin_bit_cast(bf16x8, make_uint4(s0.m, s1.m, s2.m, s3.m));
+                qf[cc].l = __builtin_bit_cast(bf16x8, make_uint4(s0.l, s1.l, s2.l, s3.l));
+            }
+        }
+        Acc A;
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) A.o[db][i] = 0.0f;
+        A.m_t = kNegInf;
+        A.m_s = kNegInf;
+        A.l = 0.0f;
+
+        lds_barrier();
+
+        // group 1 runs half a step behind group 0: one group's softmax issues under the other's PV product
+        const bool skew = n_steps >= 4;
+        if (grp && skew) lds_barrier();
+        for (int it = 0; it < n_steps; ++it) {
+            const int kt = 2 * it + grp;
+            const int k0 = kt * kBN;
+            const bool visible = kt < n_tiles && qw0 < L && !(a.causal && k0 > qw0 + 31);
+            floatx16 st;
+            uint32_t pw[3][8];  // P's planes, packed pairs
+            auto split_p = [&](int j) {
+                const Split2 s = split2(st[2 * j], st[2 * j + 1]);
+                pw[0][j] = s.h;
+                pw[1][j] = s.m;
+                pw[2][j] = s.l;
+            };
+            if (visible) {
+                // S^T, with V's planes written under it: st[i] = t[qrow][key], key = k0 + 8*(i/4) + 4*hh + i%4; the five
+                // small partial products of every chunk first, then the large one (K's h plane is read again for it).
+                // Fragments are read one chunk ahead of their MFMAs.
+                auto read_k = [&](int cc, int p) {
+                    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(kfrag + 32 * cc + p * kPlaneK));
+                };
+                auto read_k3 = [&](int cc) { return Frag3{read_k(cc, 0), read_k(cc, 1), read_k(cc, 2)}; };
+#pragma unroll
+                for (int i = 0; i < 16; ++i) st[i] = 0.0f;
+                __builtin_amdgcn_s_setprio(2);
+                Frag3 kr[2];
+                bf16x8 kh[4];
+                kr[0] = read_k3(0);
+                static_for<8>([&](auto CC) {
+                    constexpr int cc = decltype(CC)::value;
+                    if constexpr (cc + 1 < 8) kr[(cc + 1) & 1] = read_k3(cc + 1);
+                    else kh[0] = read_k(0, 0), kh[1] = read_k(1, 0);
+                    const Frag3 k = kr[cc & 1];
+                    st = mfma(k.l, qf[cc].h, st);
+                    st = mfma(k.h, qf[cc].l, st);
+                    st = mfma(k.m, qf[cc].m, st);
+                    st = mfma(k.m, qf[cc].h, st);
+                    st = mfma(k.h, qf[cc].m, st);
+                    if constexpr (cc & 1) {
+                        put(1, cc / 2, x[cc / 2]);
+                        x[cc / 2] = load(0, kt + 2, cc / 2);
+                    }
+                    DT_BUNDLE_END;
+                });
+                static_for<4>([&](auto C2) {
+                    constexpr int c2 = decltype(C2)::value;
+                    if constexpr (c2 < 3) kh[2 * ((c2 + 1) & 1)] = read_k(2 * c2 + 2, 0), kh[2 * ((c2 + 1) & 1) + 1] = read_k(2 * c2 + 3, 0);
+                    st = mfma(kh[2 * (c2 & 1)], qf[2 * c2].h, st);
+                    st = mfma(kh[2 * (c2 & 1) + 1], qf[2 * c2 + 1].h, st);
+                    DT_BUNDLE_END;
+                });
+
+                if (k0 + kBN > L || (a.causal && k0 + kBN - 1 > qw0)) {  // diagonal / ragged tail only
+                    asm volatile("");  // keeps this block a branch
+#pragma unroll
+                    for (int i = 0; i < 16; ++i)
+                        if (k0 + 8 * (i / 4) + 4 * hh + (i % 4) > lim) st[i] = kNegInf;
+                }
+                float t0 = st[0], t1 = st[1];
+#pragma unroll
+                for (int i = 2; i < 16; i += 2) {
+                    t0 = fmaxf(t0, st[i]);
+                    t1 = fmaxf(t1, st[i + 1]);
+                }
+                const float tmax = fmaxf(t0, t1);
+                A.m_t = fmaxf(A.m_t, tmax);
+                const bool grow = (A.m_s == kNegInf) ? (tmax > kNegInf) : (tmax > A.m_s + kRescaleLog2);
+                if (__builtin_amdgcn_ballot_w64(grow) != 0) {  // wave-uniform, rare after the first tile
+                    asm volatile("");  // keeps this block a branch
+                    const float m_new = max_halves(A.m_t);
+                    const float alpha = (A.m_s == kNegInf) ? 0.0f : exp2f(A.m_s - m_new);
+                    A.m_s = m_new;
+                    A.l *= alpha;
+#pragma unroll
+                    for (int db = 0; db < 4; ++db)
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) A.o[db][i] *= alpha;
+                }
+                const float ref = (A.m_s == kNegInf) ? 0.0f : A.m_s;
+                float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 16; i += 2) {
+                    st[i] = __builtin_amdgcn_exp2f(st[i] - ref);
+                    st[i + 1] = __builtin_amdgcn_exp2f(st[i + 1] - ref);
+                    s0 += st[i];
+                    s1 += st[i + 1];
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) split_p(j);  // (the second 16 keys' under the PV product)
+                A.l += s0 + s1;
+                __builtin_amdgcn_s_setprio(0);
             } else {
 #pragma unroll
-                for (int j = 0; j < 16; ++j) raw[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                q[4 * j + 0] = raw[j].x;
-                q[4 * j + 1] = raw[j].y;
-                q[4 * j + 2] = raw[j].z;
-                q[4 * j + 3] = raw[j].w;
-            }
-        }
-
-        // O^T accumulators: o[bb][i] holds O[q][d] with d = 4*m + bb, m = 8*(i/4) + 4*hh + (i%4).
-        floatx16 o[4];
-#pragma unroll
-        for (int bb = 0; bb < 4; ++bb)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) o[bb][i] = 0.0f;
-        float m_run = kNegInf;  // running max of the raw (unscaled) scores
-        float l_run = 0.0f;
-
-        // one 32-key tile of this wave's queries
-        auto compute = [&](const Stage& stg, int k0) {
-            const uint8_t* Ks = stg[grp][0];
-            const uint8_t* Vs = stg[grp][1];
-            // S^T: st[i] = S[qrow][key], key = k0 + 8*(i/4) + 4*hh + (i%4)
-            floatx16 st;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) st[i] = 0.0f;
-            // K chunk j of row ln through a four-deep register ring, three reads ahead of its MFMAs
-            auto read_k = [&](int j) {
-                return *reinterpret_cast<const float4*>(Ks + ln * kRowBytes + (pos(ln, 2 * j + hh) << 4));
-            };
-            {
-                float4 kr[4];
-                kr[0] = read_k(0);
-                kr[1] = read_k(1);
-                kr[2] = read_k(2);
-                static_for<16>([&](auto J) {
-                    constexpr int j = decltype(J)::value;
-                    if constexpr (j + 3 < 16) kr[(j + 3) & 3] = read_k(j + 3);
-                    const float4 kv = kr[j & 3];
-                    st = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, q[4 * j + 0], st, 0, 0, 0);
-                    st = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, q[4 * j + 1], st, 0, 0, 0);
-                    st = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, q[4 * j + 2], st, 0, 0, 0);
-                    st = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, q[4 * j + 3], st, 0, 0, 0);
-                    DT_BUNDLE_END;
-                });
-            }
-            // mask (diagonal / ragged tail only) and tile max
-            const bool need_mask = (a.causal && k0 + kBN - 1 > qw0) || (k0 + kBN > L);
-            float tmax = kNegInf;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                if (need_mask) {
-                    const int key = k0 + 8 * (i / 4) + 4 * hh + (i % 4);
-                    if ((a.causal && key > qrow) || key >= L) st[i] = kNegInf;
+                for (int n = 0; n < 4; ++n) {
+                    put(1, n, x[n]);
+                    x[n] = load(0, kt + 2, n);
                 }
-                tmax = fmaxf(tmax, st[i]);
             }
-            tmax = fmaxf(tmax, xor32(tmax));
-            const float m_new = fmaxf(m_run, tmax);
-            const float m_use = (m_new == kNegInf) ? 0.0f : m_new;
-            const float mc = m_use * c;
-            const float alpha = exp2f((m_run - m_use) * c);  // 0 when m_run == -inf
-            float psum = 0.0f;
-            {
-                // s*c and m*c rounded separately (no fma contraction), so the row's maximum
-                // contributes exactly exp2(0) = 1, as exp(s - m) does in the reference.
-#pragma clang fp contract(off)
+            lds_barrier();  // V's planes are written, K's are free
+
+            if (visible) {
+                // O^T += V^T P^T with the next K tile's planes written under it. Chunk ch = 4*u + db: 16 keys u, 32 dims
+                // db; k index 8*hh + e <-> key 16*u + 8*(e/4) + 4*hh + e%4. Two chunks' accumulators alternate.
+                auto read_v = [&](int ch, int p) {
+                    const uint8_t* at = vfrag + p * kPlaneV + (ch >> 2) * 16 * kRowV + 64 * (ch & 3);
+                    const shortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4*)at);
+                    const shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4*)(at + 8 * kRowV));
+                    return __builtin_bit_cast(bf16x8, (shortx8){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+                };
+                auto frag_p = [&](int p, int u) {
+                    return __builtin_bit_cast(bf16x8, make_uint4(pw[p][4 * u], pw[p][4 * u + 1], pw[p][4 * u + 2], pw[p][4 * u + 3]));
+                };
+                // fragment f = 3 * ch + (0: l, 1: m, 2: h), read 2 ahead
+                bf16x8 vr[3];
+#pragma unroll
+                for (int f = 0; f < 2; ++f) vr[f] = read_v(f / 3, 2 - f % 3);
+                static_for<24>([&](auto F) {
+                    constexpr int f = decltype(F)::value, u = f / 12, db = (f / 3) & 3;
+                    if constexpr (f + 2 < 24) vr[(f + 2) % 3] = read_v((f + 2) / 3, 2 - (f + 2) % 3);
+                    const bf16x8 v = vr[f % 3];
+                    if constexpr (f % 3 == 2) A.o[db] = mfma(v, frag_p(2, u), A.o[db]);
+                    if constexpr (f % 3 >= 1) A.o[db] = mfma(v, frag_p(1, u), A.o[db]);
+                    A.o[db] = mfma(v, frag_p(0, u), A.o[db]);
+                    if constexpr (f >= 4 && f < 8) split_p(f);
+                    if constexpr (f % 6 == 5) {
+                        put(0, f / 6, x[f / 6]);
+                        x[f / 6] = load(1, kt + 2, f / 6);
+                    }
+                    if constexpr (f % 1 == 1-1) DT_BUNDLE_END;
+                });
+            } else {
+#pragma unroll
+                for (int n = 0; n < 4; ++n) {
+                    put(0, n, x[n]);
+                    x[n] = load(1, kt + 2, n);
+                }
+            }
+            lds_barrier();  // the next K's planes are written, V's are free
+        }
+        if (!grp && skew) lds_barrier();
+
+        {
+            // a result that is not finite or below what V's split holds in full, an empty softmax over visible keys, or
+            // wide queries: the wave's keys again, in fp32
+            float z = A.l * 0.0f, omax = 0.0f;
+#pragma unroll
+            for (int db = 0; db < 4; ++db)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
-                    const float p = __builtin_amdgcn_exp2f(st[i] * c - mc);
-                    st[i] = p;
-                    psum += p;
+                    z = fmaf(A.o[db][i], 0.0f, z);
+                    omax = fmaxf(omax, fabsf(A.o[db][i]));
                 }
+            const bool keys = grp * kBN <= lim;
+            const bool bad = qrow < L && keys && (!(z == 0.0f) || !(sum_halves(A.l) > 0.0f) || q_wide ||
+                                                  (omax < 1.0f / kWide && omax > 0.0f));
+            if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+                Acc S;  // (an object of its own: A stays in registers)
+                slow_keys(S, Qg + (int64_t)min(qrow, T - 1) * a.ldq, Kg, Vg, a.ldk, a.ldv, grp, n_tiles, qw0, lim, L, T,
+                          a.causal, c);
+                A = S;
             }
-            psum += xor32(psum);
-            l_run = l_run * alpha + psum;
-            m_run = m_new;
-#pragma unroll
-            for (int bb = 0; bb < 4; ++bb)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) o[bb][i] *= alpha;
-            // O^T += V^T P^T: MFMA step s takes key 8*(s/4) + 4*hh + (s%4) of the tile from lane half hh.
-            auto read_v = [&](int s) {
-                const int key = 8 * (s / 4) + 4 * hh + (s % 4);
-                return *reinterpret_cast<const float4*>(Vs + key * kRowBytes + (pos(key, ln) << 4));
-            };
-            {
-                float4 vr[4];
-                vr[0] = read_v(0);
-                vr[1] = read_v(1);
-                vr[2] = read_v(2);
-                static_for<16>([&](auto S) {
-                    constexpr int s = decltype(S)::value;
-                    if constexpr (s + 3 < 16) vr[(s + 3) & 3] = read_v(s + 3);
-                    const float4 vv = vr[s & 3];
-                    const float p = st[s];
-                    o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.x, p, o[0], 0, 0, 0);
-                    o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.y, p, o[1], 0, 0, 0);
-                    o[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.z, p, o[2], 0, 0, 0);
-                    o[3] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.w, p, o[3], 0, 0, 0);
-                    DT_BUNDLE_END;
-                });
-            }
-        };
-        // compute from `cur` (tile kt) while the group's next tile kn streams into `nxt`
-        auto step = [&](const Stage& cur, Stage& nxt, int kt, int kn) {
-            if (kn < n_tiles) dma(nxt, kn);
-            const int k0 = kt * kBN;
-            if (kt >= n_tiles || (a.causal && k0 > qw0 + 31)) return;  // nothing of this tile is visible
-            compute(cur, k0);
-        };
-
-        stage_barrier();  // the first tile has landed
-        for (int it = 0; it < n_steps; it += 2) {
-            step(stage0, stage1, 2 * it + grp, 2 * (it + 1) + grp);
-            stage_barrier();
-            if (it + 1 >= n_steps) break;
-            step(stage1, stage0, 2 * (it + 1) + grp, 2 * (it + 2) + grp);
-            stage_barrier();
         }
 
-        // group 1 hands (O, m, l) to group 0 through LDS (no DMA is in flight now): O as 16 float4 per lane
-        float4* xo = reinterpret_cast<float4*>(&stage0[0][0][0]) + wq * (16 * 64);
-        float* xs = reinterpret_cast<float*>(&stage1[0][0][0]) + wq * (2 * 64);
-        if (grp == 1) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) xo[i * 64 + lane] = make_float4(o[0][i], o[1][i], o[2][i], o[3][i]);
-            xs[lane] = m_run;
-            xs[64 + lane] = l_run;
-        }
-        lds_barrier();
-        if (grp == 0) {
-            // finalize (FlashAttention.cpp:159-175) over both groups' keys
-            const float m1 = xs[lane];
-            const float l1 = xs[64 + lane];
-            const float m = fmaxf(m_run, m1);
-            const float m_use = (m == kNegInf) ? 0.0f : m;
-            const float a0 = exp2f((m_run - m_use) * c);  // 0 for a group that saw no valid key
-            const float a1 = exp2f((m1 - m_use) * c);
-            const float l = l_run * a0 + l1 * a1;
-            if (qrow < T) {
-                const bool valid = qrow < L && l > 0.0f;
-                float* op = Og + (int64_t)qrow * a.ldo;
+        // Merge: group g finalises dims 64g .. 64g+63 of its block's rows and hands the other half of its partial O to the
+        // other group (float4 k of lane `lane` at xo(g)[k*64 + lane]), with its (m_s, m_t, l) at xs(g). The loop's last
+        // barrier has freed the planes.
+        A.m_t = max_halves(A.m_t);
+        A.l = sum_halves(A.l);
+        auto xo = [&](int g) { return reinterpret_cast<float4*>(lds) + (g * 4 + wq) * (8 * 64); };
+        auto xs = [&](int g) { return reinterpret_cast<float*>(lds + kXoBytes) + (g * 4 + wq) * (3 * 64); };
+        uint8_t* obuf = lds + kXoBytes + kXsBytes;  // the output tile on its way to HBM
+        {
+            float4* out = xo(grp);
+            auto hand = [&](auto DB) {
+                constexpr int db = decltype(DB)::value;
 #pragma unroll
                 for (int I = 0; I < 4; ++I)
+                    out[(4 * (db & 1) + I) * 64 + lane] =
+                        make_float4(A.o[db][4 * I], A.o[db][4 * I + 1], A.o[db][4 * I + 2], A.o[db][4 * I + 3]);
+            };
+            if (grp == 0) {
+                hand(std::integral_constant<int, 2>{});
+                hand(std::integral_constant<int, 3>{});
+            } else {
+                hand(std::integral_constant<int, 0>{});
+                hand(std::integral_constant<int, 1>{});
+            }
+            float* s = xs(grp);
+            s[lane] = A.m_s;
+            s[64 + lane] = A.m_t;
+            s[128 + lane] = A.l;
+        }
+        lds_barrier();
+        {
+            // both groups form the same statistics, group 0's terms first (FlashAttention.cpp:159-175)
+            const float* so = xs(1 - grp);
+            const float os = so[lane], ot = so[64 + lane], ol = so[128 + lane];
+            const float m0s = grp ? os : A.m_s, m1s = grp ? A.m_s : os;
+            const float m0t = grp ? ot : A.m_t, m1t = grp ? A.m_t : ot;
+            const float l0 = grp ? ol : A.l, l1 = grp ? A.l : ol;
+            const float ms = fmaxf(m0s, m1s);
+            const float a0 = (m0s == kNegInf) ? 0.0f : exp2f(m0s - ms);
+            const float a1 = (m1s == kNegInf) ? 0.0f : exp2f(m1s - ms);
+            const float l = l0 * a0 + l1 * a1;
+            const float mt = fmaxf(m0t, m1t);
+            const bool valid = qrow < L && l > 0.0f;
+            const float inv = valid ? 1.0f / l : 0.0f;
+            const float4* in = xo(1 - grp);
+            uint8_t* orow = obuf + (32 * wq + ln) * kObufRow + 16 * hh;
+            auto fin = [&](auto DB) {
+                constexpr int db = decltype(DB)::value;
+#pragma unroll
+                for (int I = 0; I < 4; ++I) {
+                    const float4 y = in[(4 * (db & 1) + I) * 64 + lane];
+                    const float yv[4] = {y.x, y.y, y.z, y.w};
+                    float v[4];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        const int i = 4 * I + r;
-                        const float4 x = xo[i * 64 + lane];
-                        float4 v;
-                        if (valid) {
-                            v.x = (o[0][i] * a0 + x.x * a1) / l;
-                            v.y = (o[1][i] * a0 + x.y * a1) / l;
-                            v.z = (o[2][i] * a0 + x.z * a1) / l;
-                            v.w = (o[3][i] * a0 + x.w * a1) / l;
-                        } else {
-                            v = make_float4(0.f, 0.f, 0.f, 0.f);
-                        }
-                        *reinterpret_cast<float4*>(&op[32 * I + 16 * hh + 4 * r]) = v;
+                        const float own = A.o[db][4 * I + r];
+                        const float x = (db < 2) ? own * a0 + yv[r] * a1 : yv[r] * a0 + own * a1;
+                        const float q = x * inv;  // x / l (l >= 1), with one correction step
+                        const float e = fmaf(fmaf(-q, l, x), inv, q);
+                        v[r] = valid ? (fabsf(q) < kInf ? e : q) : 0.0f;
                     }
-                if (hh == 0) {
-                    if (a.m) a.m[stat_base + (int64_t)qrow * a.H] = valid ? m * a.scale : kNegInf;
-                    if (a.l) a.l[stat_base + (int64_t)qrow * a.H] = valid ? l : 0.0f;
+                    *reinterpret_cast<float4*>(orow + 32 * (4 * db + I)) = make_float4(v[0], v[1], v[2], v[3]);
                 }
+            };
+            if (grp == 0) {
+                fin(std::integral_constant<int, 0>{});
+                fin(std::integral_constant<int, 1>{});
+                if (qrow < T && hh == 0) {
+                    if (a.m) a.m[stat_base + (int64_t)qrow * a.H] = valid ? mt * (a.scale / c) : kNegInf;
+                    if (a.l) a.l[stat_base + (int64_t)qrow * a.H] = valid ? l * exp2f(ms - mt) : 0.0f;
+                }
+            } else {
+                fin(std::integral_constant<int, 2>{});
+                fin(std::integral_constant<int, 3>{});
             }
         }
-        // group 0 has read the exchange before the next item's DMA may overwrite it; the output stores
-        // need not have completed
+        lds_barrier();
+        // the item's 128 output rows: 32 lanes per 512-byte row, 2 rows per store instruction
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int ch = j * kThreads + tid;  // 16-byte chunk ch % 32 of row ch / 32
+            const int r = ch >> 5, cq = ch & 31;
+            const int qr = (j < 4 ? u.qa : u.qb - 64) + r;  // rows 0-63 in j < 4
+            const float4 w = *reinterpret_cast<const float4*>(obuf + r * kObufRow + 16 * cq);
+            if (qr < T) *reinterpret_cast<float4*>(&Og[(int64_t)qr * a.ldo + 4 * cq]) = w;
+        }
+        // every wave has read the output tile before the next item's DMA and planes may overwrite it; the output
+        // stores need not have completed
         lds_barrier();
     }
 }
