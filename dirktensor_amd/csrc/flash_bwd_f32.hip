@@ -1,37 +1,47 @@
 // Causal flash attention backward, fp32 exact mode, for gfx950 (CDNA4).
 //
-// Replaces flash_attention_backward (FlashAttention.cpp:185-359) with fp32
-// tensors and fp32 MFMA (v_mfma_f32_32x32x2_f32) products.
+// Replaces flash_attention_backward (FlashAttention.cpp:185-359) with fp32 tensors. As in the forward
+// (flash_fwd_f32.hip), every fp32 product runs on v_mfma_f32_32x32x16_bf16: an operand x is the exact sum of three
+// bf16 values h + m + l, and x y is formed from the six partial products of weight 2^-16 and above, small ones
+// first, accumulated in fp32. That is 192 matrix-pipe cycles per 16 steps of k against 512 on
+// v_mfma_f32_32x32x2_f32, with less rounding (it rounds every second k). Operands that a split does not hold in full
+// (infinities, the last binade, values around 2^-109 and below) are found at the end of a block, from a result that
+// is not finite or from the largest value of each operand, and the wave then repeats its block with the fp32
+// instruction, straight from memory (slow_dkdv, slow_dq).
 //
-// Same decomposition as the bf16 mode: flash_bwd_dkdv_f32 owns 128 keys of one
-// (batch, head) per workgroup (32 per wave, K and V rows in registers) and
-// streams 64-query tiles of Q, dO, lse2 and delta; flash_bwd_dq_f32 owns 128
-// queries (Q and dO rows in registers) and streams 64-key tiles of K and V.
-// Each gradient row has a single owner, so no atomics; S and dP are computed
-// in both kernels. Each workgroup owns one block; the grid lists the blocks in
-// decreasing causal cost, so the hardware's first-free-CU dispatch runs the
-// longest blocks first. With more than one block per CU and pass the dS path
-// replaces the dQ kernel: the dK/dV kernel also stores dS (fp32) and
-// flash_bwd_dq_ds forms dQ = dS K from it (5 products per tile pair instead of 7).
+// Decomposition, as in the bf16 mode: flash_bwd_dkdv owns a block of keys of one (batch, head), 32 per wave with the
+// planes of their K and V rows in registers, and streams 32-query tiles of Q and dO; flash_bwd_dq owns queries (Q and
+// dO planes in registers) and streams 32-key tiles of K and V. Each gradient row has a single owner, so no atomics; S
+// and dP are computed in both. Each workgroup owns one block; the grid lists the blocks in decreasing causal cost, so
+// the hardware's first-free-CU dispatch runs the longest blocks first. With more than one block per CU and pass the
+// dS path replaces the dQ kernel: the dK/dV kernel also stores dS (fp32) and flash_bwd_dq_ds forms dQ = dS K from it
+// (5 products per tile pair instead of 7).
 //
-// v_mfma_f32_32x32x2_f32 takes one A value per lane (row l%32, k = l/32) and
-// one B value (column l%32, k = l/32). For the products over the head
-// dimension, k step s of lane half hh is dim 64*hh + s, so a lane's register
-// operand is half of one row (64 floats) and its LDS operand is read four
-// steps at a time as a float4. For the products over queries (dK/dV) or keys
-// (dQ), the B operand is an accumulator element: step (blk, i) pairs k = hh
-// with row 32*blk + 8*(i/4) + 4*hh + i%4, the accumulator layout, and the A
-// operand is one float of that row read from LDS.
+// A workgroup is 4 waves in G groups; the groups hold the same block and take alternate tiles, each with LDS of its
+// own, and add up their partial gradients at the end. G = 1: blocks of 128 rows; G = 2: blocks of 64, twice as many
+// of half the length, where 128-row blocks would leave the longest one to set the time (the rule is at the launch).
 //
-// Tiles move from HBM straight into LDS with buffer_load ... lds, double-buffered
-// (the next tile streams in while the current one is used; one barrier per
-// tile). LDS rows are 512 bytes (128 floats), unpadded; the 16-byte chunk c of
-// row r is stored at chunk position c ^ (r & 15), so the row-wise reads of the
-// head-dimension products (16 rows, one chunk each) are conflict-free; the
-// column reads of the other products (two rows, 8 chunks each) meet in pairs
-// of banks (LDS bandwidth is far from the limit at fp32 MFMA rates). Every LDS
-// operand goes through a four-deep register ring, three reads ahead of the
-// MFMAs that consume it.
+// A streamed tile passes through registers: a thread loads four floats of a row at a time, a phase or two ahead,
+// splits them and writes the three planes under the MFMAs of another product. Per tile and wave (dK/dV):
+//   S = Q K^T      under it: Q planes of the next tile
+//   dP = dO V^T    under it: P = exp2(S c - lse2) and its split
+//   dV^T += dO^T P under it: dS = P (dP - delta) and its split      -- then a barrier: dO's planes are free
+//   dK^T += Q^T dS under it: dO planes of the next tile             -- then a barrier: the next tile is ready
+// so Q has two sets of planes and dO one (72 KB with the row statistics, 145 KB for two groups). dQ is the same with
+// K, V in the places of Q, dO, and one product less.
+//
+// What bounds it: the matrix pipe, 192 MFMAs per tile and wave for dK/dV at one wave per SIMD (K, V, dK and dV of 32 keys
+// take 320 of a lane's 512 registers), and with few blocks the longest of them. B = 1, H = 16, us per call against the
+// same decomposition on v_mfma_f32_32x32x2_f32: T = 1000 268 -> 110, T = 2048 568 -> 335, T = 4096 1540 -> 1028.
+//
+// LDS planes: 32 rows of 256 bytes, 16-byte chunk c of row r at c ^ swz(r), swz(r) = 4*(r & 3) + ((r >> 2) & 3):
+// row-wise fragment reads, transposing reads (ds_read_b64_tr_b16, in the accumulator's row order) and the split's
+// 8-byte writes are all free of bank conflicts.
+//
+// MFMA operand layouts: the A operand is a 32-row fragment, lane l holding row l%32 and k elements 8*(l/32) .. +8; the
+// B operand a 32-column fragment, lane l holding column l%32 and the same k elements; accumulator element i of lane l
+// is row 8*(i/4) + 4*(l/32) + i%4, column l%32, so an accumulator's 8 elements 8u .. 8u+7 are a B operand over 16 rows
+// in that order.
 
 #include "dt_internal.h"
 
@@ -44,18 +54,28 @@ namespace dt {
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef short shortx4 __attribute__((ext_vector_type(4)));
+typedef short shortx8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
 
 constexpr int kD = 128;
-constexpr int kTile = 64;
-constexpr int kRowBytes = kD * 4;              // one LDS row, unpadded
-constexpr int kTileBytes = kTile * kRowBytes;  // 32 KB
-constexpr int kBlk = 128;
+constexpr int kTile = 32;                        // rows per streamed tile
+constexpr int kRow = kD * 2;                     // a row of a bf16 plane
+constexpr int kPlane = kTile * kRow;             // 8 KB
+constexpr int kPlanes = 3 * kPlane;              // h, m, l
+constexpr int kBlk = 128;                        // rows owned by a workgroup of one group
 constexpr int kThreads = 256;
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kWide = 0x1p100f;
 constexpr int kBufferDword3 = 0x00020000;  // raw buffer, 32-bit data format (gfx9 family)
-typedef __attribute__((address_space(3))) void lds_void;
 
-__device__ __forceinline__ floatx16 mfma(float a, float b, floatx16 c) {
+__device__ __forceinline__ floatx16 mfma(bf16x8 a, bf16x8 b, floatx16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ floatx16 mfma_f32(float a, float b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 __device__ __forceinline__ floatx16 zero16() {
@@ -74,143 +94,209 @@ template <int N, typename F>
 __device__ __forceinline__ void static_for(F&& f) {
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
-// keeps each group of MFMAs with the LDS reads issued beside it: the scheduler may not move work across
+// keeps each group of MFMAs with the work issued beside it: the scheduler may not move work across
 #define DT_BUNDLE_END __builtin_amdgcn_sched_barrier(0)
-
-// x as an opaque value at this point: address arithmetic derived from it is done where it is used instead
-// of being hoisted out of the tile loop into long-lived registers
-__device__ __forceinline__ int fresh(int x) {
-    asm volatile("" : "+v"(x));
-    return x;
-}
-// byte offset of float x of row r in a swizzled LDS tile
-__device__ __forceinline__ int swz(int r) { return r & 15; }
 
 // Buffer descriptor over [base, base + bytes): loads at or past the end return zeros.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, kBufferDword3);
 }
-// LDS DMA issued through inline assembly: the compiler does not track these loads, so it does not wait
-// for them before reading the other LDS stage; stage_barrier() waits for them before any wave reads the
-// stage they fill. M0 (an operand bound to M0) holds the wave-uniform LDS destination; lane i writes 16
-// (or 4) bytes at M0 + 16*i (4*i).
-// The compiler cannot insert the wait states the hardware needs before these instructions (5 after a VALU
-// write of an SGPR they read, such as a v_readlane reload of the descriptor; 1 after an SALU write of M0),
-// since it does not see inside the asm: s_nop 4 provides them.
-__device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(const lds_void*)p; }
-__device__ __forceinline__ void dma16(uint32_t lds, uint32_t voff, __amdgpu_buffer_rsrc_t r) {
-    asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "{m0}"(lds) : "memory");
+__device__ __forceinline__ float4 load16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
 }
-__device__ __forceinline__ void dma4(uint32_t lds, uint32_t voff, __amdgpu_buffer_rsrc_t r) {
-    asm volatile("s_nop 4\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "{m0}"(lds) : "memory");
+__device__ __forceinline__ float load4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
 }
-// this wave's LDS DMA and LDS accesses are complete before any wave passes it
-__device__ __forceinline__ void stage_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// LDS accesses complete before any wave passes; loads in flight are not waited for
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// rows r0 .. T-1 of a [T][ld] fp32 tensor -> one LDS tile (rows past T arrive as zeros). Instruction n
-// of wave w fills LDS rows 2*(4n + w) and 2*(4n + w) + 1 (1 KB, 16 bytes per lane at chunk position
-// lane % 32); the lane fetches the chunk the swizzle puts there. The row offsets are formed here from
-// one opaque value rather than kept in registers across the tile loop.
-__device__ __forceinline__ void dma_tile(uint8_t* tile, const float* base, int r0, int T, int ld, int lane, int wave) {
-    const __amdgpu_buffer_rsrc_t r = make_rsrc(base + (int64_t)r0 * ld, (uint32_t)(T - r0) * (uint32_t)ld * 4u);
-    const uint32_t l0 = __builtin_amdgcn_readfirstlane(lds_addr(tile + wave * 1024));
-    const int r_lane = fresh(2 * wave + (lane >> 5));  // row of instruction 0; instruction n adds 8n
-    const int pos = lane & 31;
-#pragma unroll
-    for (int n = 0; n < 8; ++n) {
-        const int row = r_lane + 8 * n;
-        dma16(l0 + 4096 * n, (uint32_t)((row * ld + 4 * (pos ^ swz(row))) * 4), r);
+__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
+    bf16x2 r = __builtin_convertvector((floatx2){lo, hi}, bf16x2);
+    return __builtin_bit_cast(uint32_t, r);
+}
+// the bf16 planes of a pair of floats: x = h + m + l exactly for finite x in 2^-109 .. 2^127
+struct Split2 {
+    uint32_t h, m, l;
+};
+__device__ __forceinline__ Split2 split2(float x0, float x1) {
+    Split2 s;
+    s.h = pack_bf16x2(x0, x1);
+    const float r0 = x0 - __uint_as_float(s.h << 16), r1 = x1 - __uint_as_float(s.h & 0xffff0000u);
+    s.m = pack_bf16x2(r0, r1);
+    s.l = pack_bf16x2(r0 - __uint_as_float(s.m << 16), r1 - __uint_as_float(s.m & 0xffff0000u));
+    return s;
+}
+// an operand's three planes
+struct Frag3 {
+    bf16x8 h, m, l;
+};
+// eight accumulator elements as a B operand, packed pair by pair
+struct Words3 {
+    uint32_t w[3][8];  // [h, m, l][pair of elements]
+    __device__ __forceinline__ void put(int pair, float x0, float x1) {
+        const Split2 s = split2(x0, x1);
+        w[0][pair] = s.h;
+        w[1][pair] = s.m;
+        w[2][pair] = s.l;
     }
-}
-// 64 floats t0 .. t0+63 of a [T] row -> LDS (one wave; entries past T arrive as zeros)
-__device__ __forceinline__ void dma_stats(float* dst, const float* base, int t0, int T, int lane) {
-    const __amdgpu_buffer_rsrc_t r = make_rsrc(base + t0, (uint32_t)(T - t0) * 4u);
-    dma4(__builtin_amdgcn_readfirstlane(lds_addr(dst)), (uint32_t)lane * 4u, r);
-}
-// one row half from global memory: f[s] = X[row][64*hh + s], zeros when row >= T
-__device__ __forceinline__ void load_half_row(float (&f)[64], const float* base, int row, int T, int ld, int hh) {
-    if (row < T) {
-        const float4* p = reinterpret_cast<const float4*>(base + (int64_t)row * ld + 64 * hh);
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const float4 x = p[j];
-            f[4 * j] = x.x;
-            f[4 * j + 1] = x.y;
-            f[4 * j + 2] = x.z;
-            f[4 * j + 3] = x.w;
-        }
-    } else {
-#pragma unroll
-        for (int s = 0; s < 64; ++s) f[s] = 0.0f;
+    __device__ __forceinline__ bf16x8 frag(int p, int u) const {
+        return __builtin_bit_cast(bf16x8, make_uint4(w[p][4 * u], w[p][4 * u + 1], w[p][4 * u + 2], w[p][4 * u + 3]));
     }
+};
+// max |x| over both lane halves is within what splits hold (or all zero)
+__device__ __forceinline__ bool wide(float amax) { return amax > kWide || (amax < 1.0f / kWide && amax > 0.0f); }
+__device__ __forceinline__ float max4(float a, float4 x) {
+    return fmaxf(a, fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))));
 }
-// C[32 rows of block blk] += X[rows][64*hh + s] * f[s] over s: the product over the head dimension with
-// the LDS tile's rows as M and a register row half as the B operand. Two such products (tiles x and y,
-// register halves fx and fy) run as two interleaved accumulator chains, so consecutive MFMAs never
-// depend on each other; the LDS operands go through a three-deep register ring, two reads ahead of
-// the MFMAs that consume them.
-__device__ __forceinline__ void dot_rows2(floatx16& cx, floatx16& cy, const uint8_t* tx, const uint8_t* ty, int blk,
-                                          int ln, int hh, const float (&fx)[64], const float (&fy)[64]) {
-    cx = zero16();
-    cy = zero16();
-    // chunk 16*hh + j of row r = 32*blk + ln sits at position 16*hh + (j ^ (ln & 15))
-    const int base = fresh((32 * blk + ln) * kRowBytes + 256 * hh) | ((ln & 15) << 4);
-    auto rd = [&](const uint8_t* t, int j) { return *reinterpret_cast<const float4*>(t + (base ^ (j << 4))); };
-    float4 x[3], y[3];
-    x[0] = rd(tx, 0);
-    y[0] = rd(ty, 0);
-    x[1] = rd(tx, 1);
-    y[1] = rd(ty, 1);
-    static_for<16>([&](auto J) {
-        constexpr int j = decltype(J)::value;
-        if constexpr (j + 2 < 16) {
-            x[(j + 2) % 3] = rd(tx, j + 2);
-            y[(j + 2) % 3] = rd(ty, j + 2);
+
+__device__ __forceinline__ int swz(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
+
+// Lane addresses inside a plane.
+struct LaneAddr {
+    uint32_t raddr[8];     // row fragment chunk cc: row ln, dims 16*cc + 8*hh .. +8
+    uint32_t taddr[2][4];  // transposing read s of dim block db in a 16-row chunk (chunk u adds 4096)
+};
+__device__ __forceinline__ LaneAddr lane_addr(int lane) {
+    LaneAddr A;
+    const int ln = lane & 31, hh = lane >> 5;
+    const int g = hh ^ swz(ln);
+#pragma unroll
+    for (int cc = 0; cc < 8; ++cc) A.raddr[cc] = (uint32_t)(ln * kRow + (((2 * cc) ^ g) << 4));
+    // lane i of 16-lane group g2 reads row 4*hh + i/4 (+8 for s = 1), dims 32*db + 16*(g2 & 1) + 4*(i & 3) .. +3
+    const int i16 = lane & 15;
+    const int g2 = (lane >> 4) & 1;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const int r = 4 * hh + (i16 >> 2) + 8 * s;
+#pragma unroll
+        for (int db = 0; db < 4; ++db) {
+            const int chunk = 4 * db + 2 * g2 + ((i16 & 3) >> 1);
+            A.taddr[s][db] = (uint32_t)(r * kRow + ((chunk ^ swz(r)) << 4) + 8 * (i16 & 1));
         }
-        const float4 u = x[j % 3], v = y[j % 3];
-        cx = mfma(u.x, fx[4 * j], cx);
-        cy = mfma(v.x, fy[4 * j], cy);
-        cx = mfma(u.y, fx[4 * j + 1], cx);
-        cy = mfma(v.y, fy[4 * j + 1], cy);
-        cx = mfma(u.z, fx[4 * j + 2], cx);
-        cy = mfma(v.z, fy[4 * j + 2], cy);
-        cx = mfma(u.w, fx[4 * j + 3], cx);
-        cy = mfma(v.w, fy[4 * j + 3], cy);
-        DT_BUNDLE_END;
-    });
+    }
+    return A;
 }
-// acc[db] += sum over the 64 tile rows of tile[row][32*db + ln] * w[blk][i], row = 32*blk + 8*(i/4) + 4*hh + i%4
-// (step t = 16*blk + i reads its four LDS values, one per db, three steps ahead)
-__device__ __forceinline__ void acc_cols(floatx16 (&acc)[4], const uint8_t* tile, int ln, int hh, const floatx16 (&w)[2]) {
-    // float 32*db + ln of row r = 32*(t/16) + 8*((t%16)/4) + 4*hh + t%4 is chunk 8*db + ln/4, at position
-    // (8*db + ln/4) ^ (r & 15) = 8*(db ^ ((t/4) & 1)) + ((ln/4) ^ (4*hh + t%4))
-    const int lane_part = fresh((hh * 4) * kRowBytes + 4 * (ln & 3));
-    const int cx = fresh((ln >> 2) ^ (4 * hh));
-    auto rd = [&](int t) {
-        const int i = t & 15;
-        const int r0 = 32 * (t >> 4) + 8 * (i / 4) + (i % 4);  // row without the lane half
-        const int g = (t >> 2) & 1;
-        const uint8_t* row = tile + r0 * kRowBytes + lane_part + ((cx ^ (t & 3)) << 4);
-        return make_float4(*reinterpret_cast<const float*>(row + ((0 ^ g) << 7)),
-                           *reinterpret_cast<const float*>(row + ((1 ^ g) << 7)),
-                           *reinterpret_cast<const float*>(row + ((2 ^ g) << 7)),
-                           *reinterpret_cast<const float*>(row + ((3 ^ g) << 7)));
+
+// The product over the head dimension: rows of a tile (M) times the lane's row f (N), the five small partial products
+// of every chunk first, then the large one (whose plane is read again). Fragments are read one chunk ahead; ride(I)
+// is issued beside bundle I of 12.
+template <typename Ride>
+__device__ __forceinline__ floatx16 dot_rows(const uint8_t* tile, const LaneAddr& LA, const Frag3 (&f)[8], Ride&& ride) {
+    auto rd = [&](int cc, int p) {
+        return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(tile + LA.raddr[cc] + p * kPlane));
     };
-    float4 x[4];
-    x[0] = rd(0);
-    x[1] = rd(1);
-    x[2] = rd(2);
-    static_for<32>([&](auto Tc) {
-        constexpr int t = decltype(Tc)::value;
-        if constexpr (t + 3 < 32) x[(t + 3) & 3] = rd(t + 3);
-        const float4 v = x[t & 3];
-        const float wv = w[t >> 4][t & 15];
-        acc[0] = mfma(v.x, wv, acc[0]);
-        acc[1] = mfma(v.y, wv, acc[1]);
-        acc[2] = mfma(v.z, wv, acc[2]);
-        acc[3] = mfma(v.w, wv, acc[3]);
+    auto rd3 = [&](int cc) { return Frag3{rd(cc, 0), rd(cc, 1), rd(cc, 2)}; };
+    floatx16 c = zero16();
+    Frag3 x[2];
+    bf16x8 xh[4];
+    x[0] = rd3(0);
+    static_for<8>([&](auto CC) {
+        constexpr int cc = decltype(CC)::value;
+        if constexpr (cc + 1 < 8) x[(cc + 1) & 1] = rd3(cc + 1);
+        else xh[0] = rd(0, 0), xh[1] = rd(1, 0);
+        const Frag3 k = x[cc & 1];
+        c = mfma(k.l, f[cc].h, c);
+        c = mfma(k.h, f[cc].l, c);
+        c = mfma(k.m, f[cc].m, c);
+        c = mfma(k.m, f[cc].h, c);
+        c = mfma(k.h, f[cc].m, c);
+        ride(CC);
         DT_BUNDLE_END;
     });
+    static_for<4>([&](auto C2) {
+        constexpr int c2 = decltype(C2)::value;
+        if constexpr (c2 < 3) xh[2 * ((c2 + 1) & 1)] = rd(2 * c2 + 2, 0), xh[2 * ((c2 + 1) & 1) + 1] = rd(2 * c2 + 3, 0);
+        c = mfma(xh[2 * (c2 & 1)], f[2 * c2].h, c);
+        c = mfma(xh[2 * (c2 & 1) + 1], f[2 * c2 + 1].h, c);
+        ride(std::integral_constant<int, 8 + c2>{});
+        DT_BUNDLE_END;
+    });
+    return c;
+}
+// acc[db] += the tile's rows (k) transposed times w, over its 32 rows; ride(I) beside chunk I = 4*u + db of 8
+template <typename Ride>
+__device__ __forceinline__ void acc_cols(floatx16 (&acc)[4], const uint8_t* tile, const LaneAddr& LA, const Words3& w, Ride&& ride) {
+    auto rd = [&](int ch, int p) {
+        const uint32_t off = (uint32_t)(p * kPlane + (ch >> 2) * 16 * kRow);
+        const shortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4*)(tile + LA.taddr[0][ch & 3] + off));
+        const shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4*)(tile + LA.taddr[1][ch & 3] + off));
+        return __builtin_bit_cast(bf16x8, (shortx8){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+    };
+    auto rd3 = [&](int ch) { return Frag3{rd(ch, 0), rd(ch, 1), rd(ch, 2)}; };
+    Frag3 x[2];
+    x[0] = rd3(0);
+    static_for<8>([&](auto CH) {
+        constexpr int ch = decltype(CH)::value, u = ch >> 2, db = ch & 3;
+        if constexpr (ch + 1 < 8) x[(ch + 1) & 1] = rd3(ch + 1);
+        const Frag3 v = x[ch & 1];
+        acc[db] = mfma(v.l, w.frag(0, u), acc[db]);
+        acc[db] = mfma(v.h, w.frag(2, u), acc[db]);
+        acc[db] = mfma(v.m, w.frag(1, u), acc[db]);
+        acc[db] = mfma(v.m, w.frag(0, u), acc[db]);
+        acc[db] = mfma(v.h, w.frag(1, u), acc[db]);
+        acc[db] = mfma(v.h, w.frag(0, u), acc[db]);
+        ride(CH);
+        DT_BUNDLE_END;
+    });
+}
+
+// A group's share of the streaming: unit n (0 .. 4G-1) is the four floats 4*ln .. +3 of row (8/G)*n + 2*w + hh of a
+// tile, w the wave within its group.
+template <int G>
+struct Stream {
+    static constexpr int kUnits = 4 * G;
+    uint32_t waddr;  // of unit 0 in a plane
+    uint32_t off;    // of unit 0 in the tensor's rows, bytes
+    uint32_t ld4;    // the tensor's row stride, bytes
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ Stream(const float* base, int T, int ld, int lane, int w)
+        : off((uint32_t)((2 * w + (lane >> 5)) * ld + 4 * (lane & 31)) * 4u),
+          ld4((uint32_t)ld * 4u),
+          r(make_rsrc(base, (uint32_t)T * (uint32_t)ld * 4u)) {
+        const int row = 2 * w + (lane >> 5), ln = lane & 31;
+        waddr = (uint32_t)(row * kRow + (((ln >> 1) ^ swz(row)) << 4) + 8 * (ln & 1));
+    }
+    // byte offset of a tile's first row; a tile at or past n_tiles is not fetched (its loads return zeros, as do rows
+    // at or past T). Formed once per tile: a condition per load would end a scheduling region each time.
+    __device__ __forceinline__ uint32_t at(int tile, int row0, int n_tiles) const {
+        return (uint32_t)(row0 + min(tile, n_tiles) * kTile) * ld4 | (tile < n_tiles ? 0u : 0x80000000u);
+    }
+    __device__ __forceinline__ float4 load(uint32_t tile_at, int n) const {
+        return load16(r, off + (tile_at + (uint32_t)((8 / G) * n) * ld4));
+    }
+    __device__ __forceinline__ void put(uint8_t* planes, int n, float4 x) const {
+        const Split2 s0 = split2(x.x, x.y), s1 = split2(x.z, x.w);
+        // swz's upper bits count rows of 8/G: G = 1 flips bit 1 on odd units, G = 2 takes n mod 4
+        const uint32_t flip = G == 1 ? (uint32_t)(n & 1) << 5 : (uint32_t)(n & 3) << 4;
+        uint8_t* p = planes + ((waddr ^ flip) + (uint32_t)(n * (8 / G) * kRow));
+        *reinterpret_cast<uint2*>(p) = make_uint2(s0.h, s1.h);
+        *reinterpret_cast<uint2*>(p + kPlane) = make_uint2(s0.m, s1.m);
+        *reinterpret_cast<uint2*>(p + 2 * kPlane) = make_uint2(s0.l, s1.l);
+    }
+};
+
+// the lane's own row, split: f[cc] = X[row][16*cc + 8*hh .. +8] * mul (zeros when row >= T); its largest |x| -> amax
+__device__ __forceinline__ void load_frags(Frag3 (&f)[8], const float* base, int row, int T, int ld, int hh, float mul, float& amax) {
+    const bool in = row < T;
+    const float* p = base + (int64_t)(in ? row : 0) * ld + 8 * hh;
+    float4 x[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) x[j] = *reinterpret_cast<const float4*>(p + 16 * (j >> 1) + 4 * (j & 1));
+    if (!in) mul = 0.0f;
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) m = max4(m, x[j]);
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+    amax = in ? fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) : 0.0f;
+#pragma unroll
+    for (int cc = 0; cc < 8; ++cc) {
+        const float4 a = x[2 * cc], b = x[2 * cc + 1];
+        const Split2 s0 = split2(in ? a.x * mul : 0.0f, in ? a.y * mul : 0.0f), s1 = split2(in ? a.z * mul : 0.0f, in ? a.w * mul : 0.0f);
+        const Split2 s2 = split2(in ? b.x * mul : 0.0f, in ? b.y * mul : 0.0f), s3 = split2(in ? b.z * mul : 0.0f, in ? b.w * mul : 0.0f);
+        f[cc].h = __builtin_bit_cast(bf16x8, make_uint4(s0.h, s1.h, s2.h, s3.h));
+        f[cc].m = __builtin_bit_cast(bf16x8, make_uint4(s0.m, s1.m, s2.m, s3.m));
+        f[cc].l = __builtin_bit_cast(bf16x8, make_uint4(s0.l, s1.l, s2.l, s3.l));
+    }
 }
 // accumulator X^T (4 blocks of 32 dims x 32 rows, lane = row) * mul -> row `row` of [T][ld] at base
 __device__ __forceinline__ void store_rows(float* base, int row, int ld, int hh, const floatx16 (&x)[4], float mul) {
@@ -222,254 +308,563 @@ __device__ __forceinline__ void store_rows(float* base, int row, int ld, int hh,
             *reinterpret_cast<float4*>(p + 32 * db + 8 * g + 4 * hh) =
                 make_float4(x[db][4 * g] * mul, x[db][4 * g + 1] * mul, x[db][4 * g + 2] * mul, x[db][4 * g + 3] * mul);
 }
+// 0 for finite accumulators, NaN otherwise
+__device__ __forceinline__ float finite_probe(const floatx16 (&x)[4]) {
+    float z = 0.0f;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) z = fmaf(x[db][i], 0.0f, z);
+    return z;
+}
+
+// LDS of one group: the first operand's planes twice, the second's once, and for dK/dV the tile rows' lse2 and delta
+struct GroupLds {
+    uint8_t a[2][kPlanes];
+    uint8_t b[kPlanes];
+    float stats[2][2][kTile];
+};
+template <int G>
+union BwdLds {
+    GroupLds g[G];
+    struct {
+        float4 x[4][16][64];  // the groups' exchange (G = 2): 64 KB
+        float amax[4][2];
+    } end;
+};
+static_assert(sizeof(BwdLds<2>) <= 160 * 1024, "LDS of one CU");
+
+// The kernel's FlashBwdArgs (its first argument) where the launch put it: a reference to the parameter itself, handed
+// to a function that is not inlined, would move the parameter, and every descriptor made from it, out of scalar registers.
+__device__ __forceinline__ const FlashBwdArgs* kernel_args() {
+    return (const FlashBwdArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+}
+
+// The largest |x| of each streamed operand over the workgroup's waves (each wave saw its share of its group's tiles;
+// the whole workgroup's is as good), through LDS that nothing else uses now. Ends with a barrier.
+__device__ __forceinline__ bool wide_streams(float (&lds)[4][2], float a0, float a1, int wave, int lane) {
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1) {
+        a0 = fmaxf(a0, __shfl_xor(a0, s, 64));
+        a1 = fmaxf(a1, __shfl_xor(a1, s, 64));
+    }
+    if (lane == 0) {
+        lds[wave][0] = a0;
+        lds[wave][1] = a1;
+    }
+    lds_barrier();
+    float m0 = 0.0f, m1 = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        m0 = fmaxf(m0, lds[w][0]);
+        m1 = fmaxf(m1, lds[w][1]);
+    }
+    return wide(m0) || wide(m1);
+}
+
+// The two groups' partial sums: group g keeps own + other of `keep` and hands `give` over (group 0's terms first).
+__device__ __forceinline__ void add_groups(floatx16 (&keep)[4], const floatx16 (&give)[4], float4 (&x)[4][16][64], int grp, int wave, int lane) {
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            x[wave][4 * db + g][lane] = make_float4(give[db][4 * g], give[db][4 * g + 1], give[db][4 * g + 2], give[db][4 * g + 3]);
+    lds_barrier();
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const float4 y = x[wave ^ 2][4 * db + g][lane];
+            keep[db][4 * g] = grp ? y.x + keep[db][4 * g] : keep[db][4 * g] + y.x;
+            keep[db][4 * g + 1] = grp ? y.y + keep[db][4 * g + 1] : keep[db][4 * g + 1] + y.y;
+            keep[db][4 * g + 2] = grp ? y.z + keep[db][4 * g + 2] : keep[db][4 * g + 2] + y.z;
+            keep[db][4 * g + 3] = grp ? y.w + keep[db][4 * g + 3] : keep[db][4 * g + 3] + y.w;
+        }
+}
 
 // ------------------------------------------------------------------------------------------------ dK, dV
-// LDS stage: Q tile, dO tile, and the tile rows' lse2 and delta
-struct DkdvStage {
-    uint8_t q[kTileBytes];
-    uint8_t g[kTileBytes];
-    float lse2[kTile];
-    float delta[kTile];
-};
-
-// dS workspace blocks (the dS path): 128 key rows of 256 bytes (the 64 queries of a query tile); 16-byte
-// chunk c of a row holds queries 4c .. 4c+3 (one dK/dV lane's four consecutive accumulator rows) and sits at
-// position c ^ (8 * ((row >> 2) & 1)), so the dQ pass's reads of rows r and r + 4 (its two lane halves)
-// fall in different banks.
+// dS workspace blocks (the dS path): per 128-key block and 64-query tile, 128 key rows of 256 bytes (the 64 queries of
+// the tile), chunk c of a row holding queries 4c .. 4c+3 (one dK/dV lane's four consecutive accumulator rows).
 constexpr int kDsRowBytes = 256;
-constexpr int kDsBlockBytes = kBlk * kDsRowBytes;  // 32 KB
-constexpr int kDsHalfBytes = kTile * kDsRowBytes;  // the rows of one 64-key tile: 16 KB
+constexpr int kDsBlockBytes = 128 * kDsRowBytes;  // 32 KB
 
-// dK and dV of key block kb_own of (batch, head) bh; kEmitDs: also dS -> the dS workspace
-template <bool kEmitDs>
-__device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, int bh, DkdvStage (&stg)[2]) {
+struct KvAcc {
+    floatx16 dv[4], dk[4];
+};
+// the wave's dK and dV with v_mfma_f32_32x32x2_f32 (k step s of lane half hh is dim 64*hh + s, or one row per half)
+__device__ __noinline__ void slow_dkdv(KvAcc& A, const FlashBwdArgs& a, int bh, int kw, int tile0, int step, int n_tiles, int q_begin, bool emit) {
+    const int lane = threadIdx.x & 63, ln = lane & 31, hh = lane >> 5;
+    const int T = a.T, key = kw + ln, b = bh / a.H, h = bh % a.H;
+    const float c = a.scale * kLog2e;
+    const int64_t qkv = (int64_t)b * T * a.ld_qkv + (int64_t)h * kD, od = (int64_t)b * T * a.ld_o + (int64_t)h * kD;
+    const float *Q = static_cast<const float*>(a.q) + qkv, *G = static_cast<const float*>(a.d_o) + od;
+    const float* kp = static_cast<const float*>(a.k) + qkv + (int64_t)min(key, T - 1) * a.ld_qkv + 64 * hh;
+    const float* vp = static_cast<const float*>(a.v) + qkv + (int64_t)min(key, T - 1) * a.ld_qkv + 64 * hh;
+    for (int db = 0; db < 4; ++db) A.dv[db] = A.dk[db] = zero16();
+    for (int t = tile0; t < n_tiles; t += step) {
+        const int q0 = q_begin + t * kTile;
+        if (a.causal && q0 + kTile - 1 < kw) continue;
+        floatx16 sc = zero16(), dp = zero16();
+        const bool in = q0 + ln < T;
+        const float* qp = Q + (int64_t)min(q0 + ln, T - 1) * a.ld_qkv + 64 * hh;
+        const float* gp = G + (int64_t)min(q0 + ln, T - 1) * a.ld_o + 64 * hh;
+        for (int s = 0; s < 64; ++s) {
+            const float qx = qp[s], gx = gp[s], kx = kp[s], vx = vp[s];
+            sc = mfma_f32(in ? qx : 0.0f, key < T ? kx : 0.0f, sc);
+            dp = mfma_f32(in ? gx : 0.0f, key < T ? vx : 0.0f, dp);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int qr = q0 + 8 * (i / 4) + 4 * hh + (i % 4);
+            const bool qin = qr < T;
+            const float lse = a.lse2[(int64_t)bh * T + min(qr, T - 1)], del = a.delta[(int64_t)bh * T + min(qr, T - 1)];
+            const bool masked = (a.causal && key > qr) || (emit && key >= T);
+            const float p = masked ? 0.0f : __builtin_amdgcn_exp2f(sc[i] * c - (qin ? lse : 0.0f));
+            const float ds = p * (dp[i] - (qin ? del : 0.0f));
+            sc[i] = p;
+            dp[i] = ds;
+            const float* gr = G + (int64_t)min(qr, T - 1) * a.ld_o + ln;
+            const float* qq = Q + (int64_t)min(qr, T - 1) * a.ld_qkv + ln;
+#pragma unroll
+            for (int db = 0; db < 4; ++db) {
+                const float gx = gr[32 * db], qx = qq[32 * db];
+                A.dv[db] = mfma_f32(qin ? gx : 0.0f, p, A.dv[db]);
+                A.dk[db] = mfma_f32(qin ? qx : 0.0f, ds, A.dk[db]);
+            }
+        }
+        if (emit) {
+            const BwdDsLayout lay(T, a.causal);
+            const int kb = kw / 128;
+            uint8_t* blk = static_cast<uint8_t*>(a.ds_ws) +
+                           (uint64_t)(bh * lay.per_head() + lay.block_offset(kb) + (q0 / 64 - lay.first_tile(kb))) * kDsBlockBytes;
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *reinterpret_cast<float4*>(blk + (kw % 128 + ln) * kDsRowBytes + (q0 & 32) * 4 + 16 * (2 * g + hh)) =
+                    make_float4(dp[4 * g], dp[4 * g + 1], dp[4 * g + 2], dp[4 * g + 3]);
+        }
+    }
+}
+
+// dK and dV of block kb_own (128/G keys) of (batch, head) bh; kEmitDs: also dS -> the dS workspace
+template <int G, bool kEmitDs>
+__device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, int bh, BwdLds<G>& lds) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = G == 1 ? 0 : wave >> 1;
+    const int w = G == 1 ? wave : wave & 1;
     const int ln = lane & 31;
     const int hh = lane >> 5;
     const int T = a.T;
     const float c = a.scale * kLog2e;
-
     const int b = bh / a.H, h = bh % a.H;
 
-    const float* Qg = static_cast<const float*>(a.q) + (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
-    const float* Kg = static_cast<const float*>(a.k) + (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
-    const float* Vg = static_cast<const float*>(a.v) + (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
-    const float* Gg = static_cast<const float*>(a.d_o) + (int64_t)b * T * a.ld_o + (int64_t)h * kD;
-    const float* lse2g = a.lse2 + (int64_t)bh * T;
-    const float* deltag = a.delta + (int64_t)bh * T;
+    const int64_t qkv = (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
+    const float* Kg = static_cast<const float*>(a.k) + qkv;
+    const float* Vg = static_cast<const float*>(a.v) + qkv;
     float* dKg = static_cast<float*>(a.d_k) + (int64_t)b * T * a.ld_grad + (int64_t)h * kD;
     float* dVg = static_cast<float*>(a.d_v) + (int64_t)b * T * a.ld_grad + (int64_t)h * kD;
+    const Stream<G> sq(static_cast<const float*>(a.q) + qkv, T, a.ld_qkv, lane, w);
+    const Stream<G> sg(static_cast<const float*>(a.d_o) + (int64_t)b * T * a.ld_o + (int64_t)h * kD, T, a.ld_o, lane, w);
+    // waves 0 and 1 of a group also bring the rows' lse2 and delta
+    const __amdgpu_buffer_rsrc_t rst = make_rsrc((w ? a.delta : a.lse2) + (int64_t)bh * T, (uint32_t)T * 4u);
+    const LaneAddr LA = lane_addr(lane);
+    GroupLds& my = lds.g[grp];
 
-    // Q, dO, lse2 and delta rows q0 .. q0+63 -> stage s
-    auto fetch = [&](DkdvStage& s, int q0) {
-        dma_tile(s.q, Qg, q0, T, a.ld_qkv, lane, wave);
-        dma_tile(s.g, Gg, q0, T, a.ld_o, lane, wave);
-        if (wave == 0) dma_stats(s.lse2, lse2g, q0, T, lane);
-        if (wave == 1) dma_stats(s.delta, deltag, q0, T, lane);
+    const int kw = kb_own * (kBlk / G) + 32 * w;  // the wave's first key
+    const int key = kw + ln;                      // this lane's key (the products' N index)
+    const int q_begin = a.causal ? kb_own * (kBlk / G) : 0;
+    const int n_tiles = (T - q_begin + kTile - 1) / kTile;
+    const int n_steps = (n_tiles + G - 1) / G;
+    auto tile_stat = [&](int t) { return load4(rst, (uint32_t)(q_begin + t * kTile + ln) * 4u); };
+
+    float4 x[Stream<G>::kUnits];  // units between memory and the planes: Q's and dO's in turn
+    float xs = tile_stat(grp);
+#pragma unroll
+    for (int n = 0; n < Stream<G>::kUnits; ++n) x[n] = sq.load(sq.at(grp, q_begin, n_tiles), n);
+    float4 y[Stream<G>::kUnits];
+#pragma unroll
+    for (int n = 0; n < Stream<G>::kUnits; ++n) y[n] = sg.load(sg.at(grp, q_begin, n_tiles), n);
+    Frag3 kf[8], vf[8];
+    float kmax, vmax, qmax = 0.0f, gmax = 0.0f;
+    load_frags(kf, Kg, key, T, a.ld_qkv, hh, 1.0f, kmax);
+    load_frags(vf, Vg, key, T, a.ld_qkv, hh, 1.0f, vmax);
+    KvAcc A;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) A.dv[db] = A.dk[db] = zero16();
+
+    auto put_q = [&](int t, int n) {  // unit n of Q's tile t -> its planes, then dO's unit of that tile is requested
+        qmax = max4(qmax, x[n]);
+        sq.put(my.a[t & 1], n, x[n]);
     };
+    auto put_g = [&](int n) {
+        gmax = max4(gmax, x[n]);
+        sg.put(my.b, n, x[n]);
+    };
+    auto put_stat = [&](int buf) {
+        if (w < 2 && lane < 32) my.stats[buf][w][lane] = xs;
+    };
+#pragma unroll
+    for (int n = 0; n < Stream<G>::kUnits; ++n) put_q(0, n);
+    put_stat(0);
+#pragma unroll
+    for (int n = 0; n < Stream<G>::kUnits; ++n) {
+        x[n] = y[n];
+        put_g(n);
+        x[n] = sq.load(sq.at(G + grp, q_begin, n_tiles), n);
+    }
+    xs = tile_stat(G + grp);
+    lds_barrier();
+
+    for (int it = 0; it < n_steps; ++it) {
+        const int t = it * G + grp;
+        const int q0 = q_begin + t * kTile;
+        const int cur = it & 1, nxt = cur ^ 1;
+        const uint8_t* qt = my.a[cur];
+        // some query of the tile is at or after some key of the wave
+        const bool visible = t < n_tiles && !(a.causal && q0 + kTile - 1 < kw) && kw < T;
+        const uint32_t g_at = sg.at(t + G, q_begin, n_tiles), q_at = sq.at(t + 2 * G, q_begin, n_tiles);
+        auto move_q = [&](int n) {  // the next tile's Q -> planes; its dO is requested
+            put_q(nxt, n);
+            x[n] = sg.load(g_at, n);
+        };
+        auto move_g = [&](int n) {  // the next tile's dO -> planes; the Q after it is requested
+            put_g(n);
+            x[n] = sq.load(q_at, n);
+        };
+        floatx16 sc, dp;
+        Words3 pw, dw;
+        if (visible) {
+            sc = dot_rows(qt, LA, kf, [&](auto I) {
+                constexpr int i = decltype(I)::value;
+                if constexpr (G == 2 && i < 8) move_q(i);
+                if constexpr (G == 1 && i < 8 && (i & 1)) move_q(i / 2);
+            });
+            put_stat(nxt);
+            xs = tile_stat(t + 2 * G);
+            float L[16], D[16];  // the rows' lse2 and delta: element i is query q0 + 8*(i/4) + 4*hh + i%4
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const float4 l4 = *reinterpret_cast<const float4*>(&my.stats[cur][0][8 * g + 4 * hh]);
+                const float4 d4 = *reinterpret_cast<const float4*>(&my.stats[cur][1][8 * g + 4 * hh]);
+                L[4 * g] = l4.x, L[4 * g + 1] = l4.y, L[4 * g + 2] = l4.z, L[4 * g + 3] = l4.w;
+                D[4 * g] = d4.x, D[4 * g + 1] = d4.y, D[4 * g + 2] = d4.z, D[4 * g + 3] = d4.w;
+            }
+            // element i is masked when dmask > 8*(i/4) + i%4, i.e. when key > query (causal); with dS stored, keys past
+            // T are masked too (their dS would otherwise be exp2(-lse2) (-delta))
+            const int dmask = (kEmitDs && key >= T) ? INT_MAX : a.causal ? key - (q0 + 4 * hh) : INT_MIN;
+            dp = dot_rows(my.b, LA, vf, [&](auto I) {  // P = exp2(S c - lse2), in place of S, and its split
+                constexpr int i = decltype(I)::value;
+                if constexpr (i < 4) {
+#pragma unroll
+                    for (int e = 4 * i; e < 4 * i + 4; ++e) {
+                        const float p = __builtin_amdgcn_exp2f(sc[e] * c - L[e]);
+                        sc[e] = dmask > 8 * (e / 4) + (e % 4) ? 0.0f : p;
+                    }
+                } else {
+                    pw.put(i - 4, sc[2 * (i - 4)], sc[2 * (i - 4) + 1]);
+                }
+            });
+            acc_cols(A.dv, my.b, LA, pw, [&](auto I) {  // dV^T += dO^T P; dS = P (dP - delta), in place of dP, and its split
+                constexpr int i = decltype(I)::value;
+                if constexpr (i < 4) {
+#pragma unroll
+                    for (int e = 4 * i; e < 4 * i + 4; ++e) dp[e] = sc[e] * (dp[e] - D[e]);
+                } else {
+                    dw.put(2 * (i - 4), dp[4 * (i - 4)], dp[4 * (i - 4) + 1]);
+                    dw.put(2 * (i - 4) + 1, dp[4 * (i - 4) + 2], dp[4 * (i - 4) + 3]);
+                }
+            });
+            if constexpr (kEmitDs) {  // chunk 2*g + hh of this query block's half of the lane's key row
+                const BwdDsLayout lay(T, a.causal);
+                const int kb = kw / 128;
+                uint8_t* blk = static_cast<uint8_t*>(a.ds_ws) +
+                               (uint64_t)(bh * lay.per_head() + lay.block_offset(kb) + (q0 / 64 - lay.first_tile(kb))) * kDsBlockBytes;
+                uint8_t* row = blk + (kw % 128 + ln) * kDsRowBytes + (q0 & 32) * 4 + 16 * hh;
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *reinterpret_cast<float4*>(row + 32 * g) = make_float4(dp[4 * g], dp[4 * g + 1], dp[4 * g + 2], dp[4 * g + 3]);
+            }
+        } else {
+#pragma unroll
+            for (int n = 0; n < Stream<G>::kUnits; ++n) move_q(n);
+            put_stat(nxt);
+            xs = tile_stat(t + 2 * G);
+        }
+        lds_barrier();  // dO's planes are free
+        if (visible) {
+            acc_cols(A.dk, qt, LA, dw, [&](auto I) {  // dK^T += Q^T dS
+                constexpr int i = decltype(I)::value;
+                if constexpr (G == 2) move_g(i);
+                else if constexpr (i & 1) move_g(i / 2);
+            });
+        } else {
+#pragma unroll
+            for (int n = 0; n < Stream<G>::kUnits; ++n) move_g(n);
+        }
+        lds_barrier();  // the next tile's planes are written
+    }
 
     {
-        const int kb = kb_own;
-        const int kw = kb * kBlk + 32 * wave;
-        const int key = kw + ln;
-
-        const int q_begin = a.causal ? kb * kBlk : 0;
-        const int n_steps = (T - q_begin + kTile - 1) / kTile;
-        fetch(stg[0], q_begin);  // both stages are free: the previous block ended with a barrier
-
-        // dS stores: this key block's blocks of the workspace; lane row 32*wave + ln
-        uint8_t* ds_base = nullptr;
-        if constexpr (kEmitDs) {
-            const BwdDsLayout lay(T, a.causal);
-            ds_base = static_cast<uint8_t*>(a.ds_ws) + (uint64_t)(bh * lay.per_head() + lay.block_offset(kb)) * kDsBlockBytes;
+        const bool ws = wide_streams(lds.end.amax, qmax, gmax, wave, lane);
+        const float z = finite_probe(A.dv) + finite_probe(A.dk);
+        const bool bad = key < T && (!(z == 0.0f) || ws || wide(kmax) || wide(vmax));
+        if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+            KvAcc S;  // (an object of its own: A stays in registers)
+            slow_dkdv(S, *kernel_args(), bh, kw, grp, G, n_tiles, q_begin, kEmitDs);
+            A = S;
         }
-        const int ds_row = (32 * wave + ln) * kDsRowBytes;
-        const int ds_xs = 8 * ((ln >> 2) & 1);
-
-        float kf[64], vf[64];
-        load_half_row(kf, Kg, key, T, a.ld_qkv, hh);
-        load_half_row(vf, Vg, key, T, a.ld_qkv, hh);
-        floatx16 dv[4], dk[4];
-#pragma unroll
-        for (int db = 0; db < 4; ++db) {
-            dv[db] = zero16();
-            dk[db] = zero16();
-        }
-        stage_barrier();
-        // kMask: the tile may hold masked elements; kSkip: the wave may have no query of the tile to take
-        auto tile = [&](auto MASK, auto SKIP, int it) __attribute__((always_inline)) {
-            constexpr bool kMask = decltype(MASK)::value;
-            const int q0 = q_begin + it * kTile;
-            const DkdvStage& s = stg[it & 1];
-            if (it + 1 < n_steps) fetch(stg[(it + 1) & 1], q0 + kTile);
-            if (!(decltype(SKIP)::value && a.causal && q0 + kTile - 1 < kw)) {
-                // (the dQ pass never reads the dS of a skipped tile and wave: all of it is masked); with dS
-                // stored, keys past T are masked too (their dS would otherwise be exp2(-lse2) (-delta))
-                const bool need_mask = (a.causal && q0 < kw + 31) || (kEmitDs && kw + 31 >= T);
-                // masking without branches: element i of query block qb (query q0 + 32*qb + 4*hh + off_i,
-                // off_i = 8*(i/4) + i%4) is masked when dmask[qb] > off_i, i.e. when key > query (causal) or,
-                // with dS stored, key >= T; INT_MIN when nothing in the tile is masked
-                int dmask[2];
-#pragma unroll
-                for (int qb = 0; qb < 2; ++qb)
-                    dmask[qb] = !need_mask              ? INT_MIN
-                                : (kEmitDs && key >= T) ? INT_MAX
-                                : a.causal              ? key - (q0 + 32 * qb + 4 * hh)
-                                                        : INT_MIN;
-                floatx16 sc[2], dp[2];
-                // S = Q K^T (raw), dP = dO V^T (two query blocks; explicit calls keep every index static)
-                dot_rows2(sc[0], dp[0], s.q, s.g, 0, ln, hh, kf, vf);
-                dot_rows2(sc[1], dp[1], s.q, s.g, 1, ln, hh, kf, vf);
-                // P and dS overwrite S and dP in place
-#pragma unroll
-                for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        const int qi = 32 * qb + 8 * (i / 4) + 4 * hh + (i % 4);
-                        float pv = __builtin_amdgcn_exp2f(sc[qb][i] * c - s.lse2[qi]);
-                        if constexpr (kMask) pv = dmask[qb] > 8 * (i / 4) + (i % 4) ? 0.0f : pv;
-                        sc[qb][i] = pv;
-                        dp[qb][i] = pv * (dp[qb][i] - s.delta[qi]);
-                    }
-                if constexpr (kEmitDs) {  // dS: chunk 8*qb + 2*g + hh of the lane's key row
-                    uint8_t* blk = ds_base + (size_t)(it * kDsBlockBytes);
-#pragma unroll
-                    for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-                        for (int g = 0; g < 4; ++g)
-                            *reinterpret_cast<float4*>(blk + ds_row + (((8 * qb + 2 * g + hh) ^ ds_xs) << 4)) =
-                                make_float4(dp[qb][4 * g], dp[qb][4 * g + 1], dp[qb][4 * g + 2], dp[qb][4 * g + 3]);
-                }
-                acc_cols(dv, s.g, ln, hh, sc);  // dV^T += dO^T P
-                acc_cols(dk, s.q, ln, hh, dp);  // dK^T += Q^T dS
-            }
-            stage_barrier();  // stage it&1 is free for the tile after next; tile it+1 has landed
-        };
-        // Tiles 0 and 1 hold the diagonal (causal masks; under causality waves 2-3 have no query of tile 0);
-        // from tile 2 on nothing is masked, so that loop is compiled without the selects and the skip (the
-        // same values: dmask is INT_MIN there). The kernel that stores dS keeps one loop: peeled, it spilled.
-        using True_ = std::true_type;
-        using False_ = std::false_type;
-        if constexpr (kEmitDs) {
-            for (int it = 0; it < n_steps; ++it) tile(True_{}, True_{}, it);
+    }
+    if constexpr (G == 2) {
+        if (grp == 0) {
+            add_groups(A.dv, A.dk, lds.end.x, 0, wave, lane);
+            if (key < T) store_rows(dVg, key, a.ld_grad, hh, A.dv, 1.0f);
         } else {
-            tile(True_{}, True_{}, 0);
-            if (n_steps > 1) tile(True_{}, False_{}, 1);
-            for (int it = 2; it < n_steps; ++it) tile(False_{}, False_{}, it);
+            add_groups(A.dk, A.dv, lds.end.x, 1, wave, lane);
+            if (key < T) store_rows(dKg, key, a.ld_grad, hh, A.dk, a.scale);  // dS carries the reference's scale (:293)
         }
-        if (key < T) {
-            store_rows(dKg, key, a.ld_grad, hh, dk, a.scale);  // dS carries the reference's scale (:293)
-            store_rows(dVg, key, a.ld_grad, hh, dv, 1.0f);
-        }
+    } else if (key < T) {
+        store_rows(dKg, key, a.ld_grad, hh, A.dk, a.scale);
+        store_rows(dVg, key, a.ld_grad, hh, A.dv, 1.0f);
     }
 }
 
 // ------------------------------------------------------------------------------------------------ dQ
-// LDS stage: K tile, V tile
-struct DqStage {
-    uint8_t k[kTileBytes];
-    uint8_t v[kTileBytes];
+struct QAcc {
+    floatx16 dq[4];
 };
+__device__ __noinline__ void slow_dq(QAcc& A, const FlashBwdArgs& a, int bh, int qw, int tile0, int step, int n_tiles) {
+    const int lane = threadIdx.x & 63, ln = lane & 31, hh = lane >> 5;
+    const int T = a.T, q = qw + ln, b = bh / a.H, h = bh % a.H;
+    const float c = a.scale * kLog2e;
+    const int64_t qkv = (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
+    const float *K = static_cast<const float*>(a.k) + qkv, *V = static_cast<const float*>(a.v) + qkv;
+    const bool in = q < T;
+    const int qc = min(q, T - 1);
+    const float* qp = static_cast<const float*>(a.q) + qkv + (int64_t)qc * a.ld_qkv + 64 * hh;
+    const float* gp = static_cast<const float*>(a.d_o) + (int64_t)b * T * a.ld_o + (int64_t)h * kD + (int64_t)qc * a.ld_o + 64 * hh;
+    const float lse2 = a.lse2[(int64_t)bh * T + qc], delta = a.delta[(int64_t)bh * T + qc];
+    const int lim = a.causal ? min(q, T - 1) : T - 1;
+    for (int db = 0; db < 4; ++db) A.dq[db] = zero16();
+    for (int t = tile0; t < n_tiles; t += step) {
+        const int k0 = t * kTile;
+        if (a.causal && k0 > qw + 31) break;
+        floatx16 sc = zero16(), dp = zero16();
+        const bool kin = k0 + ln < T;
+        const float* kp = K + (int64_t)min(k0 + ln, T - 1) * a.ld_qkv + 64 * hh;
+        const float* vp = V + (int64_t)min(k0 + ln, T - 1) * a.ld_qkv + 64 * hh;
+        for (int s = 0; s < 64; ++s) {
+            const float qx = qp[s], gx = gp[s], kx = kp[s], vx = vp[s];
+            sc = mfma_f32(kin ? kx : 0.0f, in ? qx : 0.0f, sc);
+            dp = mfma_f32(kin ? vx : 0.0f, in ? gx : 0.0f, dp);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int key = k0 + 8 * (i / 4) + 4 * hh + (i % 4);
+            const float p = key > lim ? 0.0f : __builtin_amdgcn_exp2f(sc[i] * c - (in ? lse2 : 0.0f));
+            const float ds = p * (dp[i] - (in ? delta : 0.0f));
+            const float* kr = K + (int64_t)min(key, T - 1) * a.ld_qkv + ln;
+#pragma unroll
+            for (int db = 0; db < 4; ++db) {
+                const float kx = kr[32 * db];
+                A.dq[db] = mfma_f32(key < T ? kx : 0.0f, ds, A.dq[db]);
+            }
+        }
+    }
+}
 
-// dQ of query block qb_own of (batch, head) bh
-__device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int bh, DqStage (&stg)[2]) {
+// dQ of block qb_own (128/G queries) of (batch, head) bh
+template <int G>
+__device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int bh, BwdLds<G>& lds) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = G == 1 ? 0 : wave >> 1;
+    const int w = G == 1 ? wave : wave & 1;
     const int ln = lane & 31;
     const int hh = lane >> 5;
     const int T = a.T;
     const float c = a.scale * kLog2e;
-
     const int b = bh / a.H, h = bh % a.H;
 
-    const float* Qg = static_cast<const float*>(a.q) + (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
-    const float* Kg = static_cast<const float*>(a.k) + (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
-    const float* Vg = static_cast<const float*>(a.v) + (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
+    const int64_t qkv = (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
     const float* Gg = static_cast<const float*>(a.d_o) + (int64_t)b * T * a.ld_o + (int64_t)h * kD;
     float* dQg = static_cast<float*>(a.d_q) + (int64_t)b * T * a.ld_grad + (int64_t)h * kD;
+    const Stream<G> sk(static_cast<const float*>(a.k) + qkv, T, a.ld_qkv, lane, w);
+    const Stream<G> sv(static_cast<const float*>(a.v) + qkv, T, a.ld_qkv, lane, w);
+    const LaneAddr LA = lane_addr(lane);
+    GroupLds& my = lds.g[grp];
 
-    // K and V rows k0 .. k0+63 -> stage s
-    auto fetch = [&](DqStage& s, int k0) {
-        dma_tile(s.k, Kg, k0, T, a.ld_qkv, lane, wave);
-        dma_tile(s.v, Vg, k0, T, a.ld_qkv, lane, wave);
+    const int qw = qb_own * (kBlk / G) + 32 * w;  // the wave's first query
+    const int q = qw + ln;
+    const int k_end = a.causal ? min((qb_own + 1) * (kBlk / G), T) : T;
+    const int n_tiles = (k_end + kTile - 1) / kTile;
+    const int n_steps = (n_tiles + G - 1) / G;
+
+    float4 x[Stream<G>::kUnits], y[Stream<G>::kUnits];
+#pragma unroll
+    for (int n = 0; n < Stream<G>::kUnits; ++n) x[n] = sk.load(sk.at(grp, 0, n_tiles), n);
+#pragma unroll
+    for (int n = 0; n < Stream<G>::kUnits; ++n) y[n] = sv.load(sv.at(grp, 0, n_tiles), n);
+    Frag3 qf[8], gf[8];
+    float qmax, gmax, kmax = 0.0f, vmax = 0.0f;
+    load_frags(qf, static_cast<const float*>(a.q) + qkv, q, T, a.ld_qkv, hh, 1.0f, qmax);
+    load_frags(gf, Gg, q, T, a.ld_o, hh, 1.0f, gmax);
+    const float lse2 = q < T ? a.lse2[(int64_t)bh * T + q] : 0.0f;
+    const float delta = q < T ? a.delta[(int64_t)bh * T + q] : 0.0f;
+    const int lim = a.causal ? min(q, T - 1) : T - 1;  // keys > lim are masked
+    QAcc A;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) A.dq[db] = zero16();
+    auto put_k = [&](int buf, int n) {
+        kmax = max4(kmax, x[n]);
+        sk.put(my.a[buf], n, x[n]);
     };
+    auto put_v = [&](int n) {
+        vmax = max4(vmax, x[n]);
+        sv.put(my.b, n, x[n]);
+    };
+#pragma unroll
+    for (int n = 0; n < Stream<G>::kUnits; ++n) put_k(0, n);
+#pragma unroll
+    for (int n = 0; n < Stream<G>::kUnits; ++n) {
+        x[n] = y[n];
+        put_v(n);
+        x[n] = sk.load(sk.at(G + grp, 0, n_tiles), n);
+    }
+    lds_barrier();
+
+    for (int it = 0; it < n_steps; ++it) {
+        const int t = it * G + grp;
+        const int k0 = t * kTile;
+        const int cur = it & 1, nxt = cur ^ 1;
+        const uint8_t* kt = my.a[cur];
+        const bool visible = t < n_tiles && !(a.causal && k0 > qw + 31) && qw < T;
+        const uint32_t v_at = sv.at(t + G, 0, n_tiles), k_at = sk.at(t + 2 * G, 0, n_tiles);
+        auto move_k = [&](int n) {  // the next tile's K -> planes; its V is requested
+            put_k(nxt, n);
+            x[n] = sv.load(v_at, n);
+        };
+        auto move_v = [&](int n) {  // the next tile's V -> planes; the K after it is requested
+            put_v(n);
+            x[n] = sk.load(k_at, n);
+        };
+        floatx16 sc, dp;
+        Words3 dw;
+        if (visible) {
+            sc = dot_rows(kt, LA, qf, [&](auto I) {  // S^T = K Q^T
+                constexpr int i = decltype(I)::value;
+                if constexpr (G == 2 && i < 8) move_k(i);
+                if constexpr (G == 1 && i < 8 && (i & 1)) move_k(i / 2);
+            });
+            const int emask = lim - (k0 + 4 * hh);  // element i (key k0 + 8*(i/4) + 4*hh + i%4) is masked past it
+            dp = dot_rows(my.b, LA, gf, [&](auto I) {  // dP^T = V dO^T; P^T in place of S^T
+                constexpr int i = decltype(I)::value;
+                if constexpr (i < 8) {
+#pragma unroll
+                    for (int e = 2 * i; e < 2 * i + 2; ++e) {
+                        const float p = __builtin_amdgcn_exp2f(sc[e] * c - lse2);
+                        sc[e] = 8 * (e / 4) + (e % 4) > emask ? 0.0f : p;
+                    }
+                }
+            });
+#pragma unroll
+            for (int e = 0; e < 16; ++e) dp[e] = sc[e] * (dp[e] - delta);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dw.put(e, dp[2 * e], dp[2 * e + 1]);
+        } else {
+#pragma unroll
+            for (int n = 0; n < Stream<G>::kUnits; ++n) move_k(n);
+        }
+        lds_barrier();  // V's planes are free
+        if (visible) {
+            acc_cols(A.dq, kt, LA, dw, [&](auto I) {  // dQ^T += K^T dS^T
+                constexpr int i = decltype(I)::value;
+                if constexpr (i < 2) {  // the second 16 keys' dS
+                    dw.put(4 + 2 * i, dp[8 + 4 * i], dp[9 + 4 * i]);
+                    dw.put(5 + 2 * i, dp[10 + 4 * i], dp[11 + 4 * i]);
+                }
+                if constexpr (G == 2) move_v(i);
+                else if constexpr (i & 1) move_v(i / 2);
+            });
+        } else {
+#pragma unroll
+            for (int n = 0; n < Stream<G>::kUnits; ++n) move_v(n);
+        }
+        lds_barrier();  // the next tile's planes are written
+    }
 
     {
-        const int qb = qb_own;
-        const int qw = qb * kBlk + 32 * wave;
-        const int q = qw + ln;
-
-        const int k_end = a.causal ? min(qb * kBlk + kBlk, T) : T;
-        const int n_steps = (k_end + kTile - 1) / kTile;
-        fetch(stg[0], 0);  // both stages are free: the previous block ended with a barrier
-
-        float qf[64], gf[64];
-        load_half_row(qf, Qg, q, T, a.ld_qkv, hh);
-        load_half_row(gf, Gg, q, T, a.ld_o, hh);
-        const float lse2 = q < T ? a.lse2[(int64_t)bh * T + q] : 0.0f;
-        const float delta = q < T ? a.delta[(int64_t)bh * T + q] : 0.0f;
-        const int lim = a.causal ? min(q, T - 1) : T - 1;
-        floatx16 dq[4];
+        const bool ws = wide_streams(lds.end.amax, kmax, vmax, wave, lane);
+        const bool bad = q < T && (!(finite_probe(A.dq) == 0.0f) || ws || wide(qmax) || wide(gmax));
+        if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+            QAcc S;
+            slow_dq(S, *kernel_args(), bh, qw, grp, G, n_tiles);
+            A = S;
+        }
+    }
+    if constexpr (G == 2) {  // group g stores dims 64g .. 64g+63
+        float4(&ex)[4][16][64] = lds.end.x;
+        auto at = [&](int db, int g) -> float4& { return ex[wave][4 * (db & 1) + g][lane]; };
 #pragma unroll
-        for (int db = 0; db < 4; ++db) dq[db] = zero16();
-
-        stage_barrier();
-        // kGen: the tile may hold masked keys, or none the wave's queries see
-        auto tile = [&](auto GEN, int it) __attribute__((always_inline)) {
-            constexpr bool kGen = decltype(GEN)::value;
-            const int k0 = it * kTile;
-            const DqStage& s = stg[it & 1];
-            if (it + 1 < n_steps) fetch(stg[(it + 1) & 1], k0 + kTile);
-            if (!(kGen && a.causal && k0 > qw + 31)) {
-                const bool need_mask = (a.causal && k0 + kTile - 1 > qw) || k0 + kTile > T;
-                // masking without branches: element i of key block kb (key k0 + 32*kb + 4*hh + off_i, off_i =
-                // 8*(i/4) + i%4) is masked when off_i > emask[kb], i.e. when key > lim
-                int emask[2];
+        for (int d = 0; d < 2; ++d)
 #pragma unroll
-                for (int kb = 0; kb < 2; ++kb) emask[kb] = need_mask ? lim - (k0 + 32 * kb + 4 * hh) : INT_MAX;
-                floatx16 sc[2], dp[2];
-                // S^T = K Q^T (raw), dP^T = V dO^T (two key blocks; explicit calls keep every index static)
-                dot_rows2(sc[0], dp[0], s.k, s.v, 0, ln, hh, qf, gf);
-                dot_rows2(sc[1], dp[1], s.k, s.v, 1, ln, hh, qf, gf);
-                floatx16 ds[2];
-#pragma unroll
-                for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        float pv = __builtin_amdgcn_exp2f(sc[kb][i] * c - lse2);
-                        if constexpr (kGen) pv = 8 * (i / 4) + (i % 4) > emask[kb] ? 0.0f : pv;
-                        ds[kb][i] = pv * (dp[kb][i] - delta);
-                    }
-                acc_cols(dq, s.k, ln, hh, ds);  // dQ^T += K^T dS^T
+            for (int g = 0; g < 4; ++g) {
+                const floatx16 v = grp ? A.dq[d] : A.dq[2 + d];
+                at(d, g) = make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
             }
-            stage_barrier();  // stage it&1 is free for the tile after next; tile it+1 has landed
-        };
-        // Tiles 0 .. n_plain-1 need no mask (every key at or before the wave's first query and before T); the
-        // rest (the diagonal under causality, the tile past T) take the selects and, past the wave's queries,
-        // nothing. Two loops, so the first is compiled without them (the same values: emask is INT_MAX).
-        const int k_plain = a.causal ? min(qw + 1, T) : T;
-        const int n_plain = min(max(k_plain, 0) / kTile, n_steps);
-        int it = 0;
-        for (; it < n_plain; ++it) tile(std::false_type{}, it);
-        for (; it < n_steps; ++it) tile(std::true_type{}, it);
-        if (q < T) store_rows(dQg, q, a.ld_grad, hh, dq, a.scale);
+        lds_barrier();
+        if (q < T) {
+            float* p = dQg + (int64_t)q * a.ld_grad + 64 * grp + 4 * hh;
+#pragma unroll
+            for (int d = 0; d < 2; ++d)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const floatx16 v = grp ? A.dq[2 + d] : A.dq[d];
+                    const float4 o = ex[wave ^ 2][4 * d + g][lane];
+                    *reinterpret_cast<float4*>(p + 32 * d + 8 * g) =
+                        make_float4((v[4 * g] + o.x) * a.scale, (v[4 * g + 1] + o.y) * a.scale, (v[4 * g + 2] + o.z) * a.scale,
+                                    (v[4 * g + 3] + o.w) * a.scale);
+                }
+        }
+    } else if (q < T) {
+        store_rows(dQg, q, a.ld_grad, hh, A.dq, a.scale);
     }
 }
 
 // ------------------------------------------------------------------------------------------------ dQ from dS
-// LDS stage: a 64-key tile of K and the dS rows of those keys for the block's two 64-query tiles
-struct DsqStage {
-    uint8_t k[kTileBytes];
-    uint8_t ds[2][kDsHalfBytes];
+struct DsLds {
+    uint8_t k[2][kPlanes];
+    float amax[4][2];
 };
 
-// dQ of query block qb_own of (batch, head) bh from the dS the dK/dV pass stored: per 64-key tile
-// dQ^T += K^T dS^T, the A operand from the K tile as in acc_cols and the B operand (one key and query per
-// lane and step) read from the dS tile.
-__device__ __forceinline__ void dq_ds_block(const FlashBwdArgs& a, int qb_own, int bh, DsqStage (&stg)[2]) {
+__device__ __noinline__ void slow_dq_ds(QAcc& A, const FlashBwdArgs& a, int bh, int qw, int n_use) {
+    const int lane = threadIdx.x & 63, ln = lane & 31, hh = lane >> 5;
+    const int T = a.T, b = bh / a.H, h = bh % a.H;
+    const float* K = static_cast<const float*>(a.k) + (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
+    const BwdDsLayout lay(T, a.causal);
+    const uint8_t* head = static_cast<const uint8_t*>(a.ds_ws) + (uint64_t)(bh * lay.per_head()) * kDsBlockBytes;
+    for (int db = 0; db < 4; ++db) A.dq[db] = zero16();
+    for (int t = 0; t < n_use; ++t) {
+        const int k0 = t * kTile, kb = k0 / 128;
+        const uint8_t* col = head + (uint64_t)(lay.block_offset(kb) + (qw / 64 - lay.first_tile(kb))) * kDsBlockBytes + 4 * (qw % 64 + ln);
+        for (int i = 0; i < 16; ++i) {
+            const int r = 8 * (i / 4) + 4 * hh + (i % 4);
+            const float ds = *reinterpret_cast<const float*>(col + (k0 % 128 + r) * kDsRowBytes);
+            const float* kr = K + (int64_t)min(k0 + r, T - 1) * a.ld_qkv + ln;
+#pragma unroll
+            for (int db = 0; db < 4; ++db) {
+                const float kx = kr[32 * db];
+                A.dq[db] = mfma_f32(k0 + r < T ? kx : 0.0f, ds, A.dq[db]);
+            }
+        }
+    }
+}
+
+// dQ of query block qb_own (128 queries) of (batch, head) bh from the dS the dK/dV pass stored: per 32-key tile
+// dQ^T += K^T dS^T, K's planes from LDS (two stages, one barrier per tile) and dS straight from memory, one tile ahead:
+// a lane's element is one key row at its own query, so a load instruction reads two rows of 128 bytes.
+__device__ __forceinline__ void dq_ds_block(const FlashBwdArgs& a, int qb_own, int bh, DsLds& lds) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -477,114 +872,131 @@ __device__ __forceinline__ void dq_ds_block(const FlashBwdArgs& a, int qb_own, i
     const int hh = lane >> 5;
     const int T = a.T;
     const int b = bh / a.H, h = bh % a.H;
-    const float* Kg = static_cast<const float*>(a.k) + (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
     float* dQg = static_cast<float*>(a.d_q) + (int64_t)b * T * a.ld_grad + (int64_t)h * kD;
+    const Stream<1> sk(static_cast<const float*>(a.k) + (int64_t)b * T * a.ld_qkv + (int64_t)h * kD, T, a.ld_qkv, lane, wave);
     const BwdDsLayout lay(T, a.causal);
     const uint8_t* ds_head = static_cast<const uint8_t*>(a.ds_ws) + (uint64_t)(bh * lay.per_head()) * kDsBlockBytes;
+    const LaneAddr LA = lane_addr(lane);
 
     const int qw = qb_own * kBlk + 32 * wave;  // the wave's first query
     const int q = qw + ln;
-    const int qt0 = 2 * qb_own;                // the block's first 64-query tile
-    const int n_qt = min(2, lay.nqt - qt0);
     const int k_end = a.causal ? min(qb_own * kBlk + kBlk, T) : T;
-    const int n_steps = (k_end + kTile - 1) / kTile;
+    const int n_tiles = (k_end + kTile - 1) / kTile;
+    // the tiles whose dS this wave's queries have (under causality the later ones were not stored)
+    const int n_use = qw >= T ? 0 : (a.causal ? min(n_tiles, qw / kTile + 1) : n_tiles);
 
-    // K rows k0 .. k0+63 and their dS rows of the block's query tiles -> stage s (the dS rows as stored:
-    // instruction n of wave w moves 1 KB of each 16 KB half)
-    auto fetch = [&](DsqStage& s, int k0) {
-        dma_tile(s.k, Kg, k0, T, a.ld_qkv, lane, wave);
-        const int kb = k0 / kBlk;
-        const uint8_t* blk = ds_head + (uint64_t)(lay.block_offset(kb) + (qt0 - lay.first_tile(kb))) * kDsBlockBytes;
-        const __amdgpu_buffer_rsrc_t r = make_rsrc(blk, (uint32_t)n_qt * kDsBlockBytes);
-        const uint32_t rows = (uint32_t)((k0 / kTile) & 1) * kDsHalfBytes;  // this tile's rows of the key block
+    floatx16 ds;  // element i: dS of key k0 + 8*(i/4) + 4*hh + i%4 and this lane's query
+    const uint32_t lane_off = (uint32_t)(4 * hh * kDsRowBytes + 4 * (qw % 64 + ln));
+    auto load_ds = [&](int t) {
+        const int k0 = t * kTile, kb = k0 / 128;
+        const uint8_t* blk = ds_head + (uint64_t)(lay.block_offset(kb) + (qw / 64 - lay.first_tile(kb))) * kDsBlockBytes;
+        const __amdgpu_buffer_rsrc_t r = make_rsrc(t < n_use ? blk : ds_head, t < n_use ? (uint32_t)kDsBlockBytes : 0u);
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int n = 0; n < 4; ++n) {
-                const uint32_t chunk = (uint32_t)((n * 4 + wave) * 64);  // 16-byte chunks of a 16 KB half
-                dma16(__builtin_amdgcn_readfirstlane(lds_addr(s.ds[t] + chunk * 16)),
-                      (uint32_t)t * kDsBlockBytes + rows + (chunk + (uint32_t)lane) * 16u, r);
-            }
+        for (int i = 0; i < 16; ++i)
+            ds[i] = load4(r, lane_off + (uint32_t)((k0 % 128 + 8 * (i / 4) + (i % 4)) * kDsRowBytes));
     };
-
-    // the B operand of step t (t = 16*blk + i): dS of key row 32*blk + 8*(i/4) + 4*hh + i%4 and this lane's
-    // query (column 32*(wave & 1) + ln of query tile wave / 2); that row's (row >> 2) & 1 is hh, so the
-    // chunk's position is a constant of the lane
-    const int qcol = 32 * (wave & 1) + ln;
-    const int ds_lane = (wave >> 1) * kDsHalfBytes + 4 * hh * kDsRowBytes + (((qcol >> 2) ^ (8 * hh)) << 4) + 4 * (qcol & 3);
-    floatx16 dq[4];
+    QAcc A;
 #pragma unroll
-    for (int db = 0; db < 4; ++db) dq[db] = zero16();
-
-    // the tiles this wave multiplies: 0 .. n_use-1 (no query of the wave, or every key of a later tile
-    // after its queries under causality, leaves the rest to the other waves); the rest only fetch and wait,
-    // in a loop of their own (a product skipped inside the loop made the compiler copy the accumulators)
-    const int n_use = q - ln >= T ? 0 : (a.causal ? min(n_steps, (qw + 31) / kTile + 1) : n_steps);
-    fetch(stg[0], 0);
-    stage_barrier();
-    int it = 0;
-    for (; it < n_use; ++it) {
-        const int k0 = it * kTile;
-        const DsqStage& s = stg[it & 1];
-        if (it + 1 < n_steps) fetch(stg[(it + 1) & 1], k0 + kTile);
-        {
-            // the second 32 keys are all after the wave's queries under causality: their dS was not stored
-            const bool second = !a.causal || k0 + 32 <= qw + 31;
-            floatx16 w[2];
+    for (int db = 0; db < 4; ++db) A.dq[db] = zero16();
+    float4 x[4];
+    float kmax = 0.0f, dmax = 0.0f;
 #pragma unroll
-            for (int blk = 0; blk < 2; ++blk)
+    for (int n = 0; n < 4; ++n) x[n] = sk.load(sk.at(0, 0, n_tiles), n);
+    load_ds(0);
+    auto move_k = [&](int t, uint32_t next_at, int n) {
+        kmax = max4(kmax, x[n]);
+        sk.put(lds.k[t & 1], n, x[n]);
+        x[n] = sk.load(next_at, n);
+    };
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int r = 32 * blk + 8 * (i / 4) + (i % 4);  // the key row without the lane half
-                    const float x = *reinterpret_cast<const float*>(s.ds[0] + ds_lane + r * kDsRowBytes);
-                    w[blk][i] = (blk == 0 || second) ? x : 0.0f;
-                }
-            acc_cols(dq, s.k, ln, hh, w);  // dQ^T += K^T dS^T
+    for (int n = 0; n < 4; ++n) move_k(0, sk.at(1, 0, n_tiles), n);
+    lds_barrier();
+    for (int t = 0; t < n_tiles; ++t) {
+        const uint32_t k_at = sk.at(t + 2, 0, n_tiles);
+        if (t < n_use) {
+            Words3 dw;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                dw.put(e, ds[2 * e], ds[2 * e + 1]);
+                dmax = fmaxf(dmax, fmaxf(fabsf(ds[2 * e]), fabsf(ds[2 * e + 1])));
+            }
+            load_ds(t + 1);
+            acc_cols(A.dq, lds.k[t & 1], LA, dw, [&](auto I) {
+                constexpr int i = decltype(I)::value;
+                if constexpr (i & 1) move_k(t + 1, k_at, i / 2);
+            });
+        } else {
+#pragma unroll
+            for (int n = 0; n < 4; ++n) move_k(t + 1, k_at, n);
         }
-        stage_barrier();  // stage it&1 is free for the tile after next; tile it+1 has landed
+        lds_barrier();
     }
-    for (; it < n_steps; ++it) {
-        if (it + 1 < n_steps) fetch(stg[(it + 1) & 1], (it + 1) * kTile);
-        stage_barrier();
+    {
+        const bool ws = wide_streams(lds.amax, kmax, dmax, wave, lane);
+        const bool bad = q < T && (!(finite_probe(A.dq) == 0.0f) || ws);
+        if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+            QAcc S;
+            slow_dq_ds(S, *kernel_args(), bh, qw, n_use);
+            A = S;
+        }
     }
-    if (q < T) store_rows(dQg, q, a.ld_grad, hh, dq, a.scale);
+    if (q < T) store_rows(dQg, q, a.ld_grad, hh, A.dq, a.scale);
 }
 
-// One 128-row block per workgroup, listed in decreasing causal cost, so that the hardware, which hands
-// the next workgroup to the first CU that frees up, runs a longest-first schedule.
+// One block per workgroup, listed in decreasing causal cost, so that the hardware, which hands the next workgroup to
+// the first CU that frees up, runs a longest-first schedule.
 // pass = 0 (dK/dV) or 1 (dQ): one pass per launch; workgroup BH*j + bh takes, for (batch, head) bh,
 //   key block j (dK/dV; key block 0 sees every query tile) or query block n-1-j (dQ).
 // pass = 2: both passes in one launch; workgroup 2*BH*j + BH*kind + bh takes the dK/dV of key block j
 //   (kind 0) or the dQ of query block n-1-j (kind 1), which see the same number of tiles under
 //   causality, so the list stays in decreasing cost and the two passes share the CUs.
-union BwdLds {
-    DkdvStage kv[2];
-    DqStage q[2];
-};
-
+template <int G>
 __global__ __launch_bounds__(kThreads, 1) void flash_bwd_f32_kernel(FlashBwdArgs a, int pass) {
-    __shared__ __attribute__((aligned(1024))) BwdLds lds;
+    __shared__ __attribute__((aligned(1024))) BwdLds<G> lds;
     const int BH = a.B * a.H;
-    const int n = (a.T + kBlk - 1) / kBlk;
+    const int n = (a.T + kBlk / G - 1) / (kBlk / G);
     const int j = (int)blockIdx.x / (pass == 2 ? 2 * BH : BH);
     const int kind = pass == 2 ? ((int)blockIdx.x / BH) & 1 : pass;
     const int bh = (int)blockIdx.x % BH;
-    if (kind == 0) dkdv_block<false>(a, j, bh, lds.kv);
-    else dq_block(a, n - 1 - j, bh, lds.q);
+    if (kind == 0) dkdv_block<G, false>(a, j, bh, lds);
+    else dq_block<G>(a, n - 1 - j, bh, lds);
 }
 
 // The dS path: the dK/dV pass (workgroup BH*j + bh: key block j) storing dS, then dQ = dS K (workgroup
 // BH*j + bh: query block n-1-j), both in decreasing causal cost.
+template <int G>
 __global__ __launch_bounds__(kThreads, 1) void flash_bwd_dkdv_ds_f32_kernel(FlashBwdArgs a) {
-    __shared__ __attribute__((aligned(1024))) DkdvStage st[2];
+    __shared__ __attribute__((aligned(1024))) BwdLds<G> lds;
     const int BH = a.B * a.H;
-    dkdv_block<true>(a, (int)blockIdx.x / BH, (int)blockIdx.x % BH, st);
+    dkdv_block<G, true>(a, (int)blockIdx.x / BH, (int)blockIdx.x % BH, lds);
 }
-__global__ __launch_bounds__(kThreads, 1) void flash_bwd_dq_ds_f32_kernel(FlashBwdArgs a) {
-    __shared__ __attribute__((aligned(1024))) DsqStage st[2];
+__global__ __launch_bounds__(kThreads, 2) void flash_bwd_dq_ds_f32_kernel(FlashBwdArgs a) {
+    __shared__ __attribute__((aligned(1024))) DsLds lds;
     const int BH = a.B * a.H;
     const int n = (a.T + kBlk - 1) / kBlk;
-    dq_ds_block(a, n - 1 - (int)blockIdx.x / BH, (int)blockIdx.x % BH, st);
+    dq_ds_block(a, n - 1 - (int)blockIdx.x / BH, (int)blockIdx.x % BH, lds);
+}
+
+template <int G>
+int launch(const FlashBwdArgs& a, int64_t blocks128, int cus, hipStream_t stream) {
+    const int64_t blocks = G == 1 ? blocks128 : (int64_t)((a.T + kBlk / G - 1) / (kBlk / G)) * a.B * a.H;
+    if (a.ds_ws) {  // dS stored by the dK/dV pass, dQ = dS K
+        hipLaunchKernelGGL(flash_bwd_dkdv_ds_f32_kernel<G>, dim3((unsigned)blocks), dim3(kThreads), 0, stream, a);
+        DT_HIP_TRY(hipGetLastError());
+        hipLaunchKernelGGL(flash_bwd_dq_ds_f32_kernel, dim3((unsigned)blocks128), dim3(kThreads), 0, stream, a);
+        DT_HIP_TRY(hipGetLastError());
+        return DT_OK;
+    }
+    if (blocks128 <= cus) {  // the passes share one launch (at most one 128-row block per CU and pass)
+        hipLaunchKernelGGL(flash_bwd_f32_kernel<G>, dim3((unsigned)(2 * blocks)), dim3(kThreads), 0, stream, a, 2);
+        DT_HIP_TRY(hipGetLastError());
+    } else {
+        for (int pass = 0; pass < 2; ++pass) {
+            hipLaunchKernelGGL(flash_bwd_f32_kernel<G>, dim3((unsigned)blocks), dim3(kThreads), 0, stream, a, pass);
+            DT_HIP_TRY(hipGetLastError());
+        }
+    }
+    return DT_OK;
 }
 
 }  // namespace
@@ -596,25 +1008,13 @@ int launch_flash_bwd_f32(const FlashBwdArgs& a, hipStream_t stream) {
     DT_TRY(launch_flash_bwd_prep(a, 0, stream));
     const int64_t blocks = (int64_t)((a.T + kBlk - 1) / kBlk) * a.B * a.H;  // per pass, one per workgroup
     if (2 * blocks > 0x7fffffff) return set_error(DT_ERR_UNSUPPORTED, "too many workgroups");
-    if (a.ds_ws) {  // dS stored by the dK/dV pass, dQ = dS K
-        hipLaunchKernelGGL(flash_bwd_dkdv_ds_f32_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, a);
-        DT_HIP_TRY(hipGetLastError());
-        hipLaunchKernelGGL(flash_bwd_dq_ds_f32_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, a);
-        DT_HIP_TRY(hipGetLastError());
-        return DT_OK;
-    }
     int cus = 0;
     DT_TRY(persistent_grid(0x7fffffff, &cus));
-    if (blocks <= cus) {  // the passes share one launch (at most one block per CU and pass)
-        hipLaunchKernelGGL(flash_bwd_f32_kernel, dim3((unsigned)(2 * blocks)), dim3(kThreads), 0, stream, a, 2);
-        DT_HIP_TRY(hipGetLastError());
-    } else {
-        for (int pass = 0; pass < 2; ++pass) {
-            hipLaunchKernelGGL(flash_bwd_f32_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, a, pass);
-            DT_HIP_TRY(hipGetLastError());
-        }
-    }
-    return DT_OK;
+    // Two groups per workgroup where both passes' 128-row blocks together are at most one per CU: there the longest
+    // block sets the time (B*H = 16, us per call, two groups / one: T = 1000, 128 blocks per pass, 112 / 143; T = 1280,
+    // 160 blocks, 176 / 179). With more blocks the CUs are busy, and the smaller blocks split every tile for fewer rows
+    // (B*H = 48, T = 400, 192 blocks: 88 / 79; T = 2048, 256 blocks: 383 / 335).
+    return 2 * blocks <= cus ? launch<2>(a, blocks, cus, stream) : launch<1>(a, blocks, cus, stream);
 }
 
 }  // namespace dt
