@@ -141,12 +141,12 @@ struct LaneAddr {
     uint32_t raddr[8];
     uint32_t taddr[2][4];
 };
-__device__ __forceinline__ LaneAddr lane_addr(int lane) {
+__device__ __forceinline__ LaneAddr lane_addr(int lane, uint32_t goff = 0) {  // goff: a group's offset in LDS
     LaneAddr A;
     const int ln = lane & 31, hh = lane >> 5;
     const int g = hh ^ swz(ln);
 #pragma unroll
-    for (int cc = 0; cc < 8; ++cc) A.raddr[cc] = (uint32_t)(ln * kRowBytes + (((2 * cc) ^ g) << 4));
+    for (int cc = 0; cc < 8; ++cc) A.raddr[cc] = goff + (uint32_t)(ln * kRowBytes + (((2 * cc) ^ g) << 4));
     // transposing reads: lane i of 16-lane group G reads row 4*hh + i/4 (+8 for the second read) of a
     // 16-row chunk, dims 32*db + 16*(G & 1) + 4*(i & 3) .. +3
     const int i16 = lane & 15;
@@ -157,7 +157,7 @@ __device__ __forceinline__ LaneAddr lane_addr(int lane) {
 #pragma unroll
         for (int db = 0; db < 4; ++db) {
             const int chunk = 4 * db + 2 * g2 + ((i16 & 3) >> 1);
-            A.taddr[s][db] = (uint32_t)((r - 8 * s) * kRowBytes + ((chunk ^ swz(r)) << 4) + 8 * (i16 & 1));
+            A.taddr[s][db] = goff + (uint32_t)((r - 8 * s) * kRowBytes + ((chunk ^ swz(r)) << 4) + 8 * (i16 & 1));
         }
     }
     return A;
@@ -166,8 +166,18 @@ __device__ __forceinline__ LaneAddr lane_addr(int lane) {
 // DMA offsets of a 64-row tile with row stride ld (elements): instruction i of wave w fills rows
 // 16*i + 4*w + lane/16, 16 bytes per lane at chunk position lane%16, fetching the global chunk the
 // swizzle puts there.
+// (G = 2: voff[v] is instruction 0's of wave + 2*v.)
+template <int G = 1>
 __device__ __forceinline__ void dma_offsets(uint32_t (&voff)[4], int lane, int wave, int ld) {
     const int rlo = lane >> 4;
+    if constexpr (G == 2) {
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            const int vw = wave + 2 * v;
+            voff[v] = (uint32_t)(((4 * vw + rlo) * ld + 8 * ((lane & 15) ^ (4 * rlo + vw))) * 2);
+        }
+        return;
+    }
     const int chunk = (lane & 15) ^ (4 * rlo + wave);
 #pragma unroll
     for (int i = 0; i < 4; ++i) voff[i] = (uint32_t)(((16 * i + 4 * wave + rlo) * ld + 8 * chunk) * 2);
@@ -197,10 +207,21 @@ __device__ __forceinline__ void dma_tile(uint8_t* tile, const uint16_t* base, in
 #pragma unroll
     for (int i = 0; i < 4; ++i) dma16(l0 + 4096 * i, voff[i], r);
 }
+// the same by the two waves of a group (G = 2): wave w takes the shares of waves w and w + 2, whose lane offsets start
+// at voff[0] and voff[1]
+__device__ __forceinline__ void dma_tile2(uint8_t* tile, const uint16_t* base, int r0, int T, int ld, const uint32_t (&voff)[4],
+                                          int w, uint32_t goff) {
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(base + (int64_t)r0 * ld, (uint32_t)(T - r0) * (uint32_t)ld * 2u);
+    const uint32_t l0 = __builtin_amdgcn_readfirstlane(lds_addr(tile + w * 1024) + goff);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int v = 0; v < 2; ++v) dma16(l0 + 4096 * i + 2048 * v, voff[v] + (uint32_t)(32 * i) * (uint32_t)ld, r);
+}
 // 64 floats t0 .. t0+63 of a [T] row -> LDS (one wave; entries past T arrive as zeros)
-__device__ __forceinline__ void dma_stats(float* dst, const float* base, int t0, int T, int lane) {
+__device__ __forceinline__ void dma_stats(float* dst, const float* base, int t0, int T, int lane, uint32_t goff) {
     const __amdgpu_buffer_rsrc_t r = make_rsrc(base + t0, (uint32_t)(T - t0) * 4u);
-    dma4(__builtin_amdgcn_readfirstlane(lds_addr(dst)), (uint32_t)lane * 4u, r);
+    dma4(__builtin_amdgcn_readfirstlane(lds_addr(dst) + goff), (uint32_t)lane * 4u, r);
 }
 
 // this wave's LDS DMA and LDS accesses are complete before any wave passes it
@@ -241,12 +262,41 @@ struct DkdvStage {
     float delta[kTile];
 };
 
-// dK and dV of key block kb_own of (batch, head) bh; kEmitDs: also dS -> the dS workspace
-template <bool kEmitDs>
-__device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, int bh, DkdvStage& st0, DkdvStage& st1) {
+// Two groups per workgroup (G = 2). The block is then 64 rows instead of 128; waves 0-1 and 2-3 hold the same block and
+// take alternate tiles, each pair with two stages of its own (group 1's lie goff bytes after group 0's), and the groups'
+// partial gradients are added through LDS at the end, group 0's term first. Twice as many workgroups of half the
+// length: where there are few blocks the longest one sets the time.
+
+// own + the other group's `give`, through 64 KB of LDS that no stage uses any more
+__device__ __forceinline__ void add_groups(floatx16 (&keep)[4], const floatx16 (&give)[4], float4* x, int grp, int wave, int lane) {
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            x[(wave * 16 + 4 * db + g) * 64 + lane] = make_float4(give[db][4 * g], give[db][4 * g + 1], give[db][4 * g + 2], give[db][4 * g + 3]);
+    stage_barrier();
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const float4 y = x[((wave ^ 2) * 16 + 4 * db + g) * 64 + lane];
+            const float yv[4] = {y.x, y.y, y.z, y.w};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) keep[db][4 * g + r] = grp ? yv[r] + keep[db][4 * g + r] : keep[db][4 * g + r] + yv[r];
+        }
+}
+
+// dK and dV of key block kb_own (128/G keys) of (batch, head) bh; kEmitDs: also dS -> the dS workspace. st0 and st1 are
+// group 0's stages; ex: 64 KB for the groups' exchange, over the stages (G = 2)
+template <int G, bool kEmitDs>
+__device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, int bh, DkdvStage& st0, DkdvStage& st1,
+                                           uint32_t group_bytes, float4* ex) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = G == 1 ? 0 : wave >> 1;
+    const int w = G == 1 ? wave : wave & 1;  // the wave within its group
+    const uint32_t goff = G == 1 ? 0u : (uint32_t)grp * group_bytes;
     const int ln = lane & 31;
     const int hh = lane >> 5;
     const int T = a.T;
@@ -254,10 +304,10 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
 
     const int b = bh / a.H, h = bh % a.H;
 
-    const LaneAddr LA = lane_addr(lane);
+    const LaneAddr LA = lane_addr(lane, goff);
     uint32_t voff_q[4], voff_g[4];
-    dma_offsets(voff_q, lane, wave, a.ld_qkv);
-    dma_offsets(voff_g, lane, wave, a.ld_o);
+    dma_offsets<G>(voff_q, lane, w, a.ld_qkv);
+    dma_offsets<G>(voff_g, lane, w, a.ld_o);
 
     const uint16_t* Qg = static_cast<const uint16_t*>(a.q) + (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
     const uint16_t* Kg = static_cast<const uint16_t*>(a.k) + (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
@@ -269,9 +319,8 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
     uint16_t* dVg = static_cast<uint16_t*>(a.d_v) + (int64_t)b * T * a.ld_grad + (int64_t)h * kD;
 
     {
-        const int kb = kb_own;
-        const int kw = kb * kBlk + 32 * wave;  // the wave's first key
-        const int key = kw + ln;               // this lane's key (the products' N index)
+        const int kw = kb_own * (kBlk / G) + 32 * w;  // the wave's first key
+        const int key = kw + ln;                      // this lane's key (the products' N index)
 
         bf16x8 kf[8], vf[8];
         load_frags(kf, Kg, key, T, a.ld_qkv, hh);
@@ -283,36 +332,45 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
             dk[db] = zero16();
         }
 
-        const int q_begin = a.causal ? kb * kBlk : 0;
-        const int n_steps = (T - q_begin + kTile - 1) / kTile;
+        const int q_begin = a.causal ? kb_own * (kBlk / G) : 0;
+        const int n_tiles = (T - q_begin + kTile - 1) / kTile;
+        const int n_steps = (n_tiles + G - 1) / G;
 
-        // dS stores: this key block's blocks of the workspace; lane row 32*wave + ln, chunk (4*qb + 2*u + hh) ^ xs
+        // dS stores: the workspace's blocks of the 128-key block that holds this wave's keys, row r of which (key kw + ln)
+        // is 32 * (the wave's place in it) + ln; ds_q0 is the query its first block starts at
+        const int kb = kw / kBlk;
+        const int ds_q0 = a.causal ? kb * kBlk : 0;
         const __amdgpu_buffer_rsrc_t ds_rsrc = [&] {
             if constexpr (kEmitDs) {
                 const BwdDsLayout lay(T, a.causal);
                 const uint8_t* base = static_cast<const uint8_t*>(a.ds_ws) +
                                       (uint64_t)(bh * lay.per_head() + lay.block_offset(kb)) * kDsBlockBytes;
-                return make_rsrc(base, (uint32_t)n_steps * kDsBlockBytes);
+                return make_rsrc(base, (uint32_t)((T - ds_q0 + kTile - 1) / kTile) * kDsBlockBytes);
             } else {
                 return make_rsrc(a.ds_ws, 0u);
             }
         }();
-        // unit (key row r = 32*wave + ln, store k = 2*qb + u, half hh) of a block at
+        // unit (key row r, store k = 2*qb + u, half hh) of a block at
         // ((((r/32)*8 + (r%32)/4)*4 + k)*4 + r%4)*2 + hh, times 16 bytes: every store instruction writes
         // eight whole 128-byte runs (four keys' two halves), and so does every read of the dQ pass's DMA
-        const uint32_t ds_lane = (uint32_t)(((wave * 8 + (ln >> 2)) * 32 + (ln & 3) * 2 + hh) * 16);
+        const uint32_t ds_lane = (uint32_t)((((kw / 32 & 3) * 8 + (ln >> 2)) * 32 + (ln & 3) * 2 + hh) * 16);
 
         auto dma = [&](DkdvStage& s, int q0) {
-            dma_tile(s.q, Qg, q0, T, a.ld_qkv, voff_q, wave);
-            dma_tile(s.g, Gg, q0, T, a.ld_o, voff_g, wave);
-            if (wave == 0) dma_stats(s.lse2, lse2g, q0, T, lane);
-            if (wave == 1) dma_stats(s.delta, deltag, q0, T, lane);
+            if constexpr (G == 1) {
+                dma_tile(s.q, Qg, q0, T, a.ld_qkv, voff_q, wave);
+                dma_tile(s.g, Gg, q0, T, a.ld_o, voff_g, wave);
+            } else {
+                dma_tile2(s.q, Qg, q0, T, a.ld_qkv, voff_q, w, goff);
+                dma_tile2(s.g, Gg, q0, T, a.ld_o, voff_g, w, goff);
+            }
+            if (w == 0) dma_stats(s.lse2, lse2g, q0, T, lane, goff);
+            if (w == 1) dma_stats(s.delta, deltag, q0, T, lane, goff);
         };
         // kMask: the tile may hold masked elements; kSkip: the wave may have no query of the tile to take
         auto step = [&](auto MASK, auto SKIP, const DkdvStage& s, DkdvStage& nxt, int q0, bool has_next)
                         __attribute__((always_inline)) {
             constexpr bool kMask = decltype(MASK)::value;
-            if (has_next) dma(nxt, q0 + kTile);
+            if (has_next) dma(nxt, q0 + G * kTile);
             if constexpr (decltype(SKIP)::value)
                 if (a.causal && q0 + kTile - 1 < kw) return;  // every query of the tile precedes the wave's keys
             // (the dQ pass never reads the dS of such a tile and wave: all of it is masked)
@@ -344,8 +402,8 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const int qi = 32 * qb + 8 * g + 4 * hh;
-                    const float4 L4 = *reinterpret_cast<const float4*>(&s.lse2[qi]);
-                    const float4 D4 = *reinterpret_cast<const float4*>(&s.delta[qi]);
+                    const float4 L4 = *reinterpret_cast<const float4*>(reinterpret_cast<const uint8_t*>(&s.lse2[qi]) + goff);
+                    const float4 D4 = *reinterpret_cast<const float4*>(reinterpret_cast<const uint8_t*>(&s.delta[qi]) + goff);
                     Lr[qb][4 * g] = L4.x, Lr[qb][4 * g + 1] = L4.y, Lr[qb][4 * g + 2] = L4.z, Lr[qb][4 * g + 3] = L4.w;
                     Dr[qb][4 * g] = D4.x, Dr[qb][4 * g + 1] = D4.y, Dr[qb][4 * g + 2] = D4.z, Dr[qb][4 * g + 3] = D4.w;
                 }
@@ -398,7 +456,7 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
                     constexpr int qb = (b - 24) >> 4, u = ((b - 24) >> 3) & 1;
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, dsb[qb][u]), ds_rsrc,
                                                           ds_lane + (uint32_t)((2 * qb + u) * 128),
-                                                          (int)((q0 - q_begin) / kTile) * kDsBlockBytes, 0);
+                                                          (int)((q0 - ds_q0) / kTile) * kDsBlockBytes, 0);
                 }
                 DT_BUNDLE_END;
             });
@@ -406,32 +464,59 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
 
         using True_ = std::true_type;
         using False_ = std::false_type;
-        dma(st0, q_begin);
+        if (grp < n_tiles) dma(st0, q_begin + grp * kTile);
         stage_barrier();
         // Tiles 0 and 1 hold the diagonal (causal masks; under causality waves 2-3 have no query of tile 0).
         // From tile 2 on nothing is masked but, with dS stored, the keys past T, a condition fixed per wave:
         // the loop is compiled without the selects when it is false (the same values: dmask is INT_MIN).
-        step(True_{}, True_{}, st0, st1, q_begin, 1 < n_steps);
-        stage_barrier();
-        if (n_steps > 1) {
-            step(True_{}, False_{}, st1, st0, q_begin + kTile, 2 < n_steps);
+        // With 64-key blocks only tile 0, group 0's first, holds the diagonal.
+        const bool tail = kEmitDs && kw + 31 >= T;
+        if constexpr (G == 1) {
+            step(True_{}, True_{}, st0, st1, q_begin, 1 < n_steps);
             stage_barrier();
-        }
-        auto rest = [&](auto MASK) __attribute__((always_inline)) {
-            for (int it = 2; it < n_steps; it += 2) {
-                const int q0 = q_begin + it * kTile;
-                step(MASK, False_{}, st0, st1, q0, it + 1 < n_steps);
-                stage_barrier();
-                if (it + 1 >= n_steps) break;
-                step(MASK, False_{}, st1, st0, q0 + kTile, it + 2 < n_steps);
+            if (n_steps > 1) {
+                step(True_{}, False_{}, st1, st0, q_begin + kTile, 2 < n_steps);
                 stage_barrier();
             }
-        };
-        if (kEmitDs && kw + 31 >= T) rest(True_{});
-        else rest(False_{});
-        if (key < T) {
-            store_rows(dKg, key, a.ld_grad, hh, dk, a.scale);  // dS carries the reference's scale (:293)
-            store_rows(dVg, key, a.ld_grad, hh, dv, 1.0f);
+            auto rest = [&](auto MASK) __attribute__((always_inline)) {
+                for (int it = 2; it < n_steps; it += 2) {
+                    const int q0 = q_begin + it * kTile;
+                    step(MASK, False_{}, st0, st1, q0, it + 1 < n_steps);
+                    stage_barrier();
+                    if (it + 1 >= n_steps) break;
+                    step(MASK, False_{}, st1, st0, q0 + kTile, it + 2 < n_steps);
+                    stage_barrier();
+                }
+            };
+            if (tail) rest(True_{});
+            else rest(False_{});
+            if (key < T) {
+                store_rows(dKg, key, a.ld_grad, hh, dk, a.scale);  // dS carries the reference's scale (:293)
+                store_rows(dVg, key, a.ld_grad, hh, dv, 1.0f);
+            }
+        } else {
+            // tile t = 2*it + grp in stage it & 1; a group without a tile in the last step only waits
+            if (grp < n_tiles) step(True_{}, False_{}, st0, st1, q_begin + grp * kTile, grp + 2 < n_tiles);
+            stage_barrier();
+            auto rest = [&](auto MASK) __attribute__((always_inline)) {
+                for (int it = 1; it < n_steps; it += 2) {
+                    const int t = 2 * it + grp, q0 = q_begin + t * kTile;
+                    if (t < n_tiles) step(MASK, False_{}, st1, st0, q0, t + 2 < n_tiles);
+                    stage_barrier();
+                    if (it + 1 >= n_steps) break;
+                    if (t + 2 < n_tiles) step(MASK, False_{}, st0, st1, q0 + 2 * kTile, t + 4 < n_tiles);
+                    stage_barrier();
+                }
+            };
+            if (tail) rest(True_{});
+            else rest(False_{});
+            if (grp == 0) {
+                add_groups(dv, dk, ex, 0, wave, lane);
+                if (key < T) store_rows(dVg, key, a.ld_grad, hh, dv, 1.0f);
+            } else {
+                add_groups(dk, dv, ex, 1, wave, lane);
+                if (key < T) store_rows(dKg, key, a.ld_grad, hh, dk, a.scale);
+            }
         }
     }
 }
@@ -442,11 +527,16 @@ struct DqStage {
     uint8_t v[kTileBytes];
 };
 
-// dQ of query block qb_own of (batch, head) bh
-__device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int bh, DqStage& st0, DqStage& st1) {
+// dQ of query block qb_own (128/G queries) of (batch, head) bh; st0, st1, ex as in dkdv_block
+template <int G>
+__device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int bh, DqStage& st0, DqStage& st1,
+                                         uint32_t group_bytes, float4* ex) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = G == 1 ? 0 : wave >> 1;
+    const int w = G == 1 ? wave : wave & 1;  // the wave within its group
+    const uint32_t goff = G == 1 ? 0u : (uint32_t)grp * group_bytes;
     const int ln = lane & 31;
     const int hh = lane >> 5;
     const int T = a.T;
@@ -454,9 +544,9 @@ __device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int 
 
     const int b = bh / a.H, h = bh % a.H;
 
-    const LaneAddr LA = lane_addr(lane);
+    const LaneAddr LA = lane_addr(lane, goff);
     uint32_t voff[4];
-    dma_offsets(voff, lane, wave, a.ld_qkv);
+    dma_offsets<G>(voff, lane, w, a.ld_qkv);
 
     const uint16_t* Qg = static_cast<const uint16_t*>(a.q) + (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
     const uint16_t* Kg = static_cast<const uint16_t*>(a.k) + (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
@@ -465,9 +555,8 @@ __device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int 
     uint16_t* dQg = static_cast<uint16_t*>(a.d_q) + (int64_t)b * T * a.ld_grad + (int64_t)h * kD;
 
     {
-        const int qb = qb_own;
-        const int qw = qb * kBlk + 32 * wave;  // the wave's first query
-        const int q = qw + ln;                 // this lane's query (the products' N index)
+        const int qw = qb_own * (kBlk / G) + 32 * w;  // the wave's first query
+        const int q = qw + ln;                        // this lane's query (the products' N index)
 
         bf16x8 qf[8], gf[8];
         load_frags(qf, Qg, q, T, a.ld_qkv, hh);
@@ -479,17 +568,23 @@ __device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int 
 #pragma unroll
         for (int db = 0; db < 4; ++db) dq[db] = zero16();
 
-        const int k_end = a.causal ? min(qb * kBlk + kBlk, T) : T;
-        const int n_steps = (k_end + kTile - 1) / kTile;
+        const int k_end = a.causal ? min((qb_own + 1) * (kBlk / G), T) : T;
+        const int n_tiles = (k_end + kTile - 1) / kTile;
+        const int n_steps = (n_tiles + G - 1) / G;
 
         auto dma = [&](DqStage& s, int k0) {
-            dma_tile(s.k, Kg, k0, T, a.ld_qkv, voff, wave);
-            dma_tile(s.v, Vg, k0, T, a.ld_qkv, voff, wave);
+            if constexpr (G == 1) {
+                dma_tile(s.k, Kg, k0, T, a.ld_qkv, voff, wave);
+                dma_tile(s.v, Vg, k0, T, a.ld_qkv, voff, wave);
+            } else {
+                dma_tile2(s.k, Kg, k0, T, a.ld_qkv, voff, w, goff);
+                dma_tile2(s.v, Vg, k0, T, a.ld_qkv, voff, w, goff);
+            }
         };
         // kGen: the tile may hold masked keys, or none the wave's queries see
         auto step = [&](auto GEN, const DqStage& s, DqStage& nxt, int k0, bool has_next) __attribute__((always_inline)) {
             constexpr bool kGen = decltype(GEN)::value;
-            if (has_next) dma(nxt, k0 + kTile);
+            if (has_next) dma(nxt, k0 + G * kTile);
             if constexpr (kGen)
                 if (a.causal && k0 > qw + 31) return;  // every key of the tile follows the wave's queries
             const bool need_mask = (a.causal && k0 + kTile - 1 > qw) || k0 + kTile > T;
@@ -552,30 +647,60 @@ __device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int 
         // rest (the diagonal under causality, the tile past T) take the selects and, past the wave's queries,
         // nothing. Two loops, so the first is compiled without them (the same values: emask is INT_MAX).
         const int k_plain = a.causal ? min(qw + 1, T) : T;
-        const int n_plain = min(max(k_plain, 0) / kTile, n_steps);
+        const int n_plain_tiles = min(max(k_plain, 0) / kTile, n_tiles);
+        const int n_plain = G == 1 ? n_plain_tiles : (max(n_plain_tiles - grp, 0) + 1) / 2;  // this group's
+        // step it takes the group's tile G*it + grp, in stage it & 1; a group without one in the last step only waits
+        auto has = [&](int it) { return G * it + grp < n_tiles; };
+        auto key0 = [&](int it) { return (G * it + grp) * kTile; };
         using True_ = std::true_type;
         using False_ = std::false_type;
-        dma(st0, 0);
+        if (G == 1 || has(0)) dma(st0, key0(0));
         stage_barrier();
         int it = 0;
         for (; it + 1 < n_plain; it += 2) {
-            const int k0 = it * kTile;
-            step(False_{}, st0, st1, k0, it + 1 < n_steps);
+            step(False_{}, st0, st1, key0(it), has(it + 1));
             stage_barrier();
-            step(False_{}, st1, st0, k0 + kTile, it + 2 < n_steps);
+            step(False_{}, st1, st0, key0(it + 1), has(it + 2));
             stage_barrier();
         }
         if (it < n_plain) {  // an odd count: the last plain tile is an even one
-            step(False_{}, st0, st1, it * kTile, it + 1 < n_steps);
+            step(False_{}, st0, st1, key0(it), has(it + 1));
             stage_barrier();
             ++it;
         }
         for (; it < n_steps; ++it) {
-            if (it & 1) step(True_{}, st1, st0, it * kTile, it + 1 < n_steps);
-            else step(True_{}, st0, st1, it * kTile, it + 1 < n_steps);
+            if (G == 1 || has(it)) {
+                if (it & 1) step(True_{}, st1, st0, key0(it), has(it + 1));
+                else step(True_{}, st0, st1, key0(it), has(it + 1));
+            }
             stage_barrier();
         }
-        if (q < T) store_rows(dQg, q, a.ld_grad, hh, dq, a.scale);
+        if constexpr (G == 1) {
+            if (q < T) store_rows(dQg, q, a.ld_grad, hh, dq, a.scale);
+        } else {  // group g stores dims 64g .. 64g+63: the other half of its sums goes to the other group
+#pragma unroll
+            for (int d = 0; d < 2; ++d)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const floatx16 v = grp ? dq[d] : dq[2 + d];
+                    ex[(wave * 8 + 4 * d + g) * 64 + lane] = make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
+                }
+            stage_barrier();
+            if (q < T) {
+                uint16_t* p = dQg + (int64_t)q * a.ld_grad + 64 * grp + 4 * hh;
+#pragma unroll
+                for (int d = 0; d < 2; ++d)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        const floatx16 v = grp ? dq[2 + d] : dq[d];
+                        const float4 o = ex[((wave ^ 2) * 8 + 4 * d + g) * 64 + lane];
+                        uint2 x;
+                        x.x = pack_bf16x2((v[4 * g] + o.x) * a.scale, (v[4 * g + 1] + o.y) * a.scale);
+                        x.y = pack_bf16x2((v[4 * g + 2] + o.z) * a.scale, (v[4 * g + 3] + o.w) * a.scale);
+                        *reinterpret_cast<uint2*>(p + 32 * d + 8 * g) = x;
+                    }
+            }
+        }
     }
 }
 
@@ -765,38 +890,73 @@ __device__ __forceinline__ void dq_ds_block(const FlashBwdArgs& a, int qb_own, i
 //   four products, before a dQ tile, three). With at most one block per pass for each CU (T = 2048,
 //   B*H = 16) the passes then share the CUs instead of running one after the other, each with its
 //   longest block setting its time.
+struct DkdvStages {
+    DkdvStage s0, s1;
+};
+struct DqStages {
+    DqStage s0, s1;
+};
+template <int G>
 union BwdLds {
-    struct {
-        DkdvStage s0, s1;
-    } kv;
-    struct {
-        DqStage s0, s1;
-    } q;
+    DkdvStages kv[G];
+    DqStages q[G];
+    float4 ex[G == 1 ? 1 : 4 * 16 * 64];  // the groups' exchange
 };
 
+template <int G>
 __global__ __launch_bounds__(kThreads, 1) void flash_bwd_bf16_kernel(FlashBwdArgs a, int pass) {
-    __shared__ __attribute__((aligned(1024))) BwdLds lds;
+    __shared__ __attribute__((aligned(1024))) BwdLds<G> lds;
     const int BH = a.B * a.H;
-    const int n = (a.T + kBlk - 1) / kBlk;
+    const int n = (a.T + kBlk / G - 1) / (kBlk / G);
     const int j = (int)blockIdx.x / (pass == 2 ? 2 * BH : BH);
     const int kind = pass == 2 ? ((int)blockIdx.x / BH) & 1 : pass;
     const int bh = (int)blockIdx.x % BH;
-    if (kind == 0) dkdv_block<false>(a, j, bh, lds.kv.s0, lds.kv.s1);
-    else dq_block(a, n - 1 - j, bh, lds.q.s0, lds.q.s1);
+    if (kind == 0) dkdv_block<G, false>(a, j, bh, lds.kv[0].s0, lds.kv[0].s1, (uint32_t)sizeof(DkdvStages), lds.ex);
+    else dq_block<G>(a, n - 1 - j, bh, lds.q[0].s0, lds.q[0].s1, (uint32_t)sizeof(DqStages), lds.ex);
 }
 
 // The dS path: the dK/dV pass (workgroup BH*j + bh: key block j) storing dS, then dQ = dS K (workgroup
 // BH*j + bh: query block n-1-j), both in decreasing causal cost.
+template <int G>
 __global__ __launch_bounds__(kThreads, 1) void flash_bwd_dkdv_ds_bf16_kernel(FlashBwdArgs a) {
-    __shared__ __attribute__((aligned(1024))) DkdvStage s0, s1;
     const int BH = a.B * a.H;
-    dkdv_block<true>(a, (int)blockIdx.x / BH, (int)blockIdx.x % BH, s0, s1);
+    const int j = (int)blockIdx.x / BH, bh = (int)blockIdx.x % BH;
+    if constexpr (G == 1) {
+        __shared__ __attribute__((aligned(1024))) DkdvStage s0, s1;
+        dkdv_block<1, true>(a, j, bh, s0, s1, 0u, nullptr);
+    } else {
+        __shared__ __attribute__((aligned(1024))) BwdLds<G> lds;
+        dkdv_block<G, true>(a, j, bh, lds.kv[0].s0, lds.kv[0].s1, (uint32_t)sizeof(DkdvStages), lds.ex);
+    }
 }
 __global__ __launch_bounds__(kDqThreads, 1) void flash_bwd_dq_ds_bf16_kernel(FlashBwdArgs a) {
     __shared__ __attribute__((aligned(1024))) DsqStage st[kDqStages];
     const int BH = a.B * a.H;
     const int n = (a.T + kBlk - 1) / kBlk;
     dq_ds_block(a, n - 1 - (int)blockIdx.x / BH, (int)blockIdx.x % BH, st);
+}
+
+template <int G>
+int launch(const FlashBwdArgs& a, int64_t blocks128, int cus, hipStream_t stream) {
+    const int64_t blocks = G == 1 ? blocks128 : (int64_t)((a.T + kBlk / G - 1) / (kBlk / G)) * a.B * a.H;
+    if (a.ds_ws) {  // dS stored by the dK/dV pass, dQ = dS K
+        hipLaunchKernelGGL(flash_bwd_dkdv_ds_bf16_kernel<G>, dim3((unsigned)blocks), dim3(kThreads), 0, stream, a);
+        DT_HIP_TRY(hipGetLastError());
+        hipLaunchKernelGGL(flash_bwd_dq_ds_bf16_kernel, dim3((unsigned)blocks128), dim3(kDqThreads), 0, stream, a);
+        DT_HIP_TRY(hipGetLastError());
+        return DT_OK;
+    }
+    if (blocks128 <= cus) {  // the passes share one launch (measured: T = 2048, B*H = 16: 148 -> 94 us; at
+                             // T = 4096, two blocks per CU and pass, one launch per pass is 4 % faster)
+        hipLaunchKernelGGL(flash_bwd_bf16_kernel<G>, dim3((unsigned)(2 * blocks)), dim3(kThreads), 0, stream, a, 2);
+        DT_HIP_TRY(hipGetLastError());
+    } else {
+        for (int pass = 0; pass < 2; ++pass) {
+            hipLaunchKernelGGL(flash_bwd_bf16_kernel<G>, dim3((unsigned)blocks), dim3(kThreads), 0, stream, a, pass);
+            DT_HIP_TRY(hipGetLastError());
+        }
+    }
+    return DT_OK;
 }
 
 }  // namespace
@@ -807,26 +967,12 @@ int launch_flash_bwd_bf16(const FlashBwdArgs& a, hipStream_t stream) {
     DT_TRY(launch_flash_bwd_prep(a, 1, stream));
     const int64_t blocks = (int64_t)((a.T + kBlk - 1) / kBlk) * a.B * a.H;  // per pass, one per workgroup
     if (2 * blocks > 0x7fffffff) return set_error(DT_ERR_UNSUPPORTED, "too many workgroups");
-    if (a.ds_ws) {  // dS stored by the dK/dV pass, dQ = dS K
-        hipLaunchKernelGGL(flash_bwd_dkdv_ds_bf16_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, a);
-        DT_HIP_TRY(hipGetLastError());
-        hipLaunchKernelGGL(flash_bwd_dq_ds_bf16_kernel, dim3((unsigned)blocks), dim3(kDqThreads), 0, stream, a);
-        DT_HIP_TRY(hipGetLastError());
-        return DT_OK;
-    }
     int cus = 0;
     DT_TRY(persistent_grid(0x7fffffff, &cus));
-    if (blocks <= cus) {  // the passes share one launch (measured: T = 2048, B*H = 16: 148 -> 94 us; at
-                          // T = 4096, two blocks per CU and pass, one launch per pass is 4 % faster)
-        hipLaunchKernelGGL(flash_bwd_bf16_kernel, dim3((unsigned)(2 * blocks)), dim3(kThreads), 0, stream, a, 2);
-        DT_HIP_TRY(hipGetLastError());
-    } else {
-        for (int pass = 0; pass < 2; ++pass) {
-            hipLaunchKernelGGL(flash_bwd_bf16_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, a, pass);
-            DT_HIP_TRY(hipGetLastError());
-        }
-    }
-    return DT_OK;
+    // Two groups per workgroup where both passes' 128-row blocks together are at most one per CU (B*H = 16, us per call,
+    // two groups / one: T = 512 18.7 / 24.7, T = 1000 34.4 / 39.1); past that the CUs are busy and the smaller blocks
+    // fetch every tile for fewer rows (T = 1280 51.9 / 46.6, T = 2048 97.5 / 80.6; B*H = 32, T = 777 50.1 / 40.9).
+    return 2 * blocks <= cus ? launch<2>(a, blocks, cus, stream) : launch<1>(a, blocks, cus, stream);
 }
 
 }  // namespace dt
