@@ -142,8 +142,14 @@ def _mode_of(x, mode: Optional[str]) -> int:
     raise TypeError(f"unsupported numpy dtype {x.dtype}: float32, or uint16 holding bf16 bits")
 
 
-def _stream_of(t) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+# the current stream of a device index as an address (0: the null stream), without building a Stream object
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) if torch is not None else None
+
+
+def _stream_of(t):
+    if _raw_stream is not None:
+        return _raw_stream(t.device.index)
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def _seq_lens_arg(seq_lens, B: int):
@@ -164,10 +170,11 @@ def flash_attention_forward(Q, K, V, scale: float, causal: bool = True, *, seq_l
     and returns rows t >= seq_lens[b] as the reference's empty row
     (output 0, m = -inf, l = 0). Raises DTError on invalid arguments.
     """
-    if Q.shape != K.shape or Q.shape != V.shape or len(Q.shape) != 4:
+    shape = Q.shape
+    if shape != K.shape or shape != V.shape or len(shape) != 4:
         raise ValueError(f"Q, K, V must share one [B,T,H,D] shape, got {tuple(Q.shape)}, {tuple(K.shape)}, "
                          f"{tuple(V.shape)}")
-    B, T, H, D = (int(s) for s in Q.shape)
+    B, T, H, D = shape
     dtype = _mode_of(Q, mode)
     lens_arr, lens_p = _seq_lens_arg(seq_lens, B)
     if _is_torch(Q):
@@ -180,8 +187,8 @@ def flash_attention_forward(Q, K, V, scale: float, causal: bool = True, *, seq_l
         ctx = ctx or default_context(Q.device.index or 0)
         Q, K, V = Q.contiguous(), K.contiguous(), V.contiguous()
         O = torch.empty_like(Q)
-        m = torch.empty((B, T, H), dtype=torch.float32, device=Q.device)
-        l = torch.empty((B, T, H), dtype=torch.float32, device=Q.device)
+        m = Q.new_empty((B, T, H), dtype=torch.float32)
+        l = Q.new_empty((B, T, H), dtype=torch.float32)
         C.call("dt_flash_attn_fwd", ctx.handle, Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(),
                m.data_ptr(), l.data_ptr(), B, T, H, D, float(scale), int(bool(causal)), lens_p, dtype,
                C.DT_MEM_DEVICE, _stream_of(Q))
@@ -227,7 +234,7 @@ def flash_attention_backward(d_output, output, softmax_m, softmax_l, Q, K, V, sc
     dtype = _mode_of(Q, mode)
     if _is_torch(Q):
         ins = [t.contiguous() for t in (d_output, output, Q, K, V)]
-        if any(not _is_torch(t) or not t.is_cuda or t.dtype != Q.dtype for t in ins):
+        if not all([_is_torch(t) and t.is_cuda and t.dtype == Q.dtype for t in ins]):
             raise TypeError("d_output, output, Q, K, V must be torch device tensors of one dtype")
         m, l = softmax_m.contiguous().float(), softmax_l.contiguous().float()
         ctx = ctx or default_context(Q.device.index or 0)
