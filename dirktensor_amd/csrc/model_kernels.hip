@@ -262,73 +262,103 @@ __global__ __launch_bounds__(256) void ce_rows_kernel(const float* logits, const
     }
 }
 
-// The same row with the whole row held in registers (kChunks float4 per thread, 1024 threads, so V / 4 <= 1024 *
-// kChunks; V % 4 == 0, 16-byte aligned rows): the row is read from memory once instead of twice. The row's
-// maximum is formed first and the sum of exponentials then taken relative to it.
-template <int kChunks>
-__global__ __launch_bounds__(1024) void ce_rows_reg_kernel(const float* logits, const int32_t* target, float* term,
-                                                           float* grad, int V, float inv_count) {
-    __shared__ float red[16];
+// The same row held on the CU, so that it is read from memory once instead of twice: kChunks float4 per thread in
+// registers, and with kLds that many more in LDS (the 1024-thread form only; each thread reads back what it wrote).
+// V < 4 * kThreads * (kChunks + kLds) + 4. The row's maximum is formed first and the sum of exponentials then taken
+// relative to it. Any V and any 4-byte alignment: rows of an odd length start unaligned, which global 16-byte accesses
+// take, and the last V % 4 logits are one extra value of the first threads. Per call, read twice by 256 threads (in
+// single floats where V % 4 != 0) and now: 2048 x 100277 693 -> 385 us, 1024 x 50001 294 -> 127, 2048 x 30001 234 -> 128,
+// 500 x 110001 503 -> 152; 64 x 8000, which 1024 threads held before, 44 -> 34. HBM bound: the row kernel moves 1.64 GB in
+// about 310 us at 2048 x 100352. A persistent form that requested the next row's chunk as each was stored spilled (621).
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+template <int kThreads, int kChunks, int kLds>
+__global__ __launch_bounds__(kThreads) void ce_rows_reg_kernel(const float* logits, const int32_t* target, float* term,
+                                                               float* grad, int V, float inv_count) {
+    constexpr int kWaves = kThreads / 64;
+    __shared__ float red[kWaves];
+    __shared__ f4u xl[kLds > 0 ? kLds * kThreads : 1];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int64_t row = blockIdx.x;
     const int tgt = target[row];
     const float* l = logits + row * V;
     float* g = grad ? grad + row * V : nullptr;
-    const int V4 = V / 4;
+    const int V4 = V / 4, it = 4 * V4 + tid;  // it: this thread's logit of the last V % 4, if below V
     if (tgt < 0) {
         if (tid == 0) term[row] = 0.0f;
-        if (g)
-            for (int i = tid; i < V4; i += 1024)
-                reinterpret_cast<float4*>(g)[i] = make_float4(0.0f * inv_count, 0.0f * inv_count, 0.0f * inv_count,
-                                                              0.0f * inv_count);
+        if (g) {
+            const float z = 0.0f * inv_count;
+            for (int i = tid; i < V4; i += kThreads) *reinterpret_cast<f4u*>(g + 4 * i) = (f4u){z, z, z, z};
+            if (it < V) g[it] = z;
+        }
         return;
     }
     const float l_tgt = tid == 0 ? l[tgt] : 0.0f;  // before the barriers: the gradient may overwrite it
     constexpr float kNegInf = -__builtin_huge_valf();
-    float4 x[kChunks];
-    float m = kNegInf;
+    const f4u none = {kNegInf, kNegInf, kNegInf, kNegInf};
+    f4u x[kChunks];
+    auto max4 = [](f4u v) { return fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)); };
+    const float xt = it < V ? l[it] : kNegInf;
+    float m = xt;
 #pragma unroll
     for (int c = 0; c < kChunks; ++c) {
-        const int i = c * 1024 + tid;
-        x[c] = i < V4 ? reinterpret_cast<const float4*>(l)[i] : make_float4(kNegInf, kNegInf, kNegInf, kNegInf);
-        m = fmaxf(m, fmaxf(fmaxf(x[c].x, x[c].y), fmaxf(x[c].z, x[c].w)));
+        const int i = c * kThreads + tid;
+        x[c] = i < V4 ? *reinterpret_cast<const f4u*>(l + 4 * i) : none;
     }
+#pragma unroll
+    for (int c = 0; c < kLds; ++c) {
+        const int i = (kChunks + c) * kThreads + tid;
+        const f4u v = i < V4 ? *reinterpret_cast<const f4u*>(l + 4 * i) : none;
+        xl[c * kThreads + tid] = v;
+        m = fmaxf(m, max4(v));
+    }
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) m = fmaxf(m, max4(x[c]));
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
     if (lane == 0) red[wv] = m;
     __syncthreads();
     float mx = red[0];
-    for (int k = 1; k < 16; ++k) mx = fmaxf(mx, red[k]);
+    for (int k = 1; k < kWaves; ++k) mx = fmaxf(mx, red[k]);
     __syncthreads();  // red is reused below
+    auto sum4 = [&](f4u v) { return (expf(v.x - mx) + expf(v.y - mx)) + (expf(v.z - mx) + expf(v.w - mx)); };
     float s = 0.0f;
 #pragma unroll
-    for (int c = 0; c < kChunks; ++c)
-        s += (expf(x[c].x - mx) + expf(x[c].y - mx)) + (expf(x[c].z - mx) + expf(x[c].w - mx));
+    for (int c = 0; c < kChunks; ++c) s += sum4(x[c]);
+#pragma unroll
+    for (int c = 0; c < kLds; ++c) s += sum4(xl[c * kThreads + tid]);
+    if (it < V) s += expf(xt - mx);
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
     if (lane == 0) red[wv] = s;
     __syncthreads();
     float se = 0.0f;
-    for (int k = 0; k < 16; ++k) se += red[k];
+    for (int k = 0; k < kWaves; ++k) se += red[k];
     if (tid == 0) term[row] = logf(se) - (l_tgt - mx);
     if (g) {
         const float inv = 1.0f / se;
+        auto put = [&](int i, f4u v) {
+            float p[4] = {expf(v.x - mx) * inv, expf(v.y - mx) * inv, expf(v.z - mx) * inv, expf(v.w - mx) * inv};
 #pragma unroll
-        for (int c = 0; c < kChunks; ++c) {
-            const int i = c * 1024 + tid;
-            if (i < V4) {
-                float p[4] = {expf(x[c].x - mx) * inv, expf(x[c].y - mx) * inv, expf(x[c].z - mx) * inv,
-                              expf(x[c].w - mx) * inv};
+            for (int e = 0; e < 4; ++e)
+                if (4 * i + e == tgt) p[e] -= 1.0f;
+            const f4u v4 = {p[0] * inv_count, p[1] * inv_count, p[2] * inv_count, p[3] * inv_count};
+            // long rows: streaming stores (375 -> 359 us per call at 2048 x 100352)
+            if constexpr (kThreads == 1024) __builtin_nontemporal_store(v4, reinterpret_cast<f4u*>(g + 4 * i));
+            else *reinterpret_cast<f4u*>(g + 4 * i) = v4;
+        };
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (4 * i + e == tgt) p[e] -= 1.0f;
-                reinterpret_cast<float4*>(g)[i] =
-                    make_float4(p[0] * inv_count, p[1] * inv_count, p[2] * inv_count, p[3] * inv_count);
-            }
+        for (int c = 0; c < kChunks; ++c)
+            if (c * kThreads + tid < V4) put(c * kThreads + tid, x[c]);
+#pragma unroll
+        for (int c = 0; c < kLds; ++c)
+            if ((kChunks + c) * kThreads + tid < V4) put((kChunks + c) * kThreads + tid, xl[c * kThreads + tid]);
+        if (it < V) {
+            float p = expf(xt - mx) * inv;
+            if (it == tgt) p -= 1.0f;
+            g[it] = p * inv_count;
         }
     }
 }
-constexpr int kCeChunks = 25;  // rows of up to 102400 logits in registers
 
 // loss = sum of the terms (fixed order, fp64) / count, one workgroup
 __global__ __launch_bounds__(256) void ce_reduce_kernel(const float* term, int64_t rows, float inv_count, float* loss) {
@@ -549,10 +579,21 @@ int launch_swiglu(const void* gu, void* act, int rows, int hid, int bf16, hipStr
 int launch_ce_loss(const float* logits, const int32_t* target, float* term, float* grad, float* loss, int rows, int V,
                    int count, hipStream_t s) {
     const float inv = count > 0 ? 1.0f / (float)count : __builtin_nanf("");  // 0 / 0 as in the reference
+    // the smallest form that holds the row; longer rows are read twice
     const bool vec = V % 4 == 0 && ((uintptr_t)logits | (uintptr_t)grad) % 16 == 0;
-    if (vec && V / 4 <= 1024 * kCeChunks)
-        hipLaunchKernelGGL(ce_rows_reg_kernel<kCeChunks>, dim3(rows), dim3(1024), 0, s, logits, target, term, grad, V,
-                           inv);
+    auto reg = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, dim3(rows), dim3(threads), 0, s, logits, target, term, grad, V, inv);
+    };
+    const int n = (V / 4 + 255) / 256;  // in chunks of 256 float4
+    if (n <= 2) reg(ce_rows_reg_kernel<256, 2, 0>, 256);
+    else if (n <= 4) reg(ce_rows_reg_kernel<256, 4, 0>, 256);
+    else if (n <= 8) reg(ce_rows_reg_kernel<256, 8, 0>, 256);
+    else if (n <= 16) reg(ce_rows_reg_kernel<256, 16, 0>, 256);
+    else if (n <= 32) reg(ce_rows_reg_kernel<512, 16, 0>, 512);
+    else if (n <= 4 * 13) reg(ce_rows_reg_kernel<1024, 13, 0>, 1024);
+    else if (n <= 4 * 19) reg(ce_rows_reg_kernel<1024, 19, 0>, 1024);
+    else if (n <= 4 * 25) reg(ce_rows_reg_kernel<1024, 25, 0>, 1024);
+    else if (n <= 4 * 32) reg(ce_rows_reg_kernel<1024, 23, 9>, 1024);
     else if (vec) hipLaunchKernelGGL(ce_rows_kernel<true>, dim3(rows), dim3(256), 0, s, logits, target, term, grad, V, inv);
     else hipLaunchKernelGGL(ce_rows_kernel<false>, dim3(rows), dim3(256), 0, s, logits, target, term, grad, V, inv);
     DT_HIP_TRY(hipGetLastError());
