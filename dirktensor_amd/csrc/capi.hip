@@ -1326,12 +1326,18 @@ int dt_attn_layer_step(dt_attn_layer* L, float lr, void* stream) {
     if (!std::isfinite(lr)) return set_error(DT_ERR_INVALID_ARG, "lr must be finite");
     DT_TRY(check_device_binding(L->ctx));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    DT_TRY(attn_layer_step_mats(L, lr, s));
-    // :319-320, RMSNorm.cpp:38-40: both norm weights in one launch
-    float* w[2] = {L->q_norm, L->k_norm};
-    const float* g[2] = {L->g_qn, L->g_kn};
-    const int n[2] = {L->d_model, L->d_model};
-    return launch_sgd_vecs(w, g, n, 2, lr, s);
+    DT_TRY(attn_layer_ensure_grads(L, s));
+    DT_TRY(attn_layer_settle_grads(L, s));
+    // OlmoAttention.cpp:315-320, RMSNorm.cpp:38-40: the matrices, with their bf16 copies, and both norm weights at once
+    const int64_t dm = L->d_model;
+    const bool copies = L->w_qkv16 && L->w_o16;
+    const SgdSeg segs[4] = {{L->w_qkv, L->g_qkv, copies ? L->w_qkv16 : nullptr, 3 * dm * dm},
+                            {L->w_o, L->g_o, copies ? L->w_o16 : nullptr, dm * dm},
+                            {L->q_norm, L->g_qn, nullptr, dm},
+                            {L->k_norm, L->g_kn, nullptr, dm}};
+    DT_TRY(launch_sgd_segs(segs, 4, lr, s));
+    L->w16_stale = !copies;
+    return DT_OK;
 }
 
 int dt_attn_layer_zero_grad(dt_attn_layer* L, void* stream) {

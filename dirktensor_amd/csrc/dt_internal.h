@@ -192,6 +192,14 @@ int launch_colsum(const float* partial, int nblk, int ncols, float* out, hipStre
                   float* out1 = nullptr);
 // w -= lr * g; w16 (nullable): the bf16 copy of w, refreshed in the same pass
 int launch_sgd(float* w, const float* g, float lr, int64_t n, hipStream_t stream, uint16_t* w16 = nullptr);
+// the same update of up to four tensors (n % 4 == 0, 16-byte aligned) in one launch
+struct SgdSeg {
+    float* w;
+    const float* g;
+    uint16_t* w16;  // nullable
+    int64_t n;
+};
+int launch_sgd_segs(const SgdSeg* segs, int count, float lr, hipStream_t stream);
 // the same update of count short vectors (the norm weights) in one launch, one workgroup per vector
 int launch_sgd_vecs(float* const* w, const float* const* g, const int* n, int count, float lr, hipStream_t stream);
 int launch_fill_zero(float* p, int64_t n, hipStream_t stream);

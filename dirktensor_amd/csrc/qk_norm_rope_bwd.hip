@@ -31,6 +31,8 @@
 
 #include "dt_internal.h"
 
+#include <climits>
+
 namespace dt {
 namespace {
 
@@ -189,6 +191,45 @@ __global__ __launch_bounds__(256) void sgd4_kernel(float4* w, const float4* g, f
     }
 }
 
+// The update of a few tensors of different sizes in one launch, four groups of four elements per thread: block b takes 1024
+// groups of the segment whose blocks it falls in. A layer's step took three launches (42 us of kernels at d_model 2048,
+// HBM bound, and the gaps between them); the norm vectors' few blocks run beside the matrices'.
+constexpr int kSgdSegs = 4;
+struct SgdSegs {
+    float4* w[kSgdSegs];
+    const float4* g[kSgdSegs];
+    uint2* w16[kSgdSegs];  // nullable: the bf16 copy
+    int64_t n4[kSgdSegs];
+    int block0[kSgdSegs];  // a segment's first block, ascending (INT_MAX: no segment)
+};
+__global__ __launch_bounds__(256) void sgd_segs_kernel(SgdSegs v, float lr) {
+#pragma clang fp contract(off)
+    int k = 0;
+#pragma unroll
+    for (int i = 1; i < kSgdSegs; ++i) k = (int)blockIdx.x >= v.block0[i] ? i : k;
+    float4* w = v.w[k];
+    const float4* g = v.g[k];
+    uint2* w16 = v.w16[k];
+    const int64_t n4 = v.n4[k], i0 = (int64_t)((int)blockIdx.x - v.block0[k]) * 1024 + threadIdx.x;
+    float4 gv[4], wv[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (i0 + 256 * j < n4) {
+            gv[j] = g[i0 + 256 * j];
+            wv[j] = w[i0 + 256 * j];
+        }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (i0 + 256 * j < n4) {
+            wv[j].x = wv[j].x - lr * gv[j].x;
+            wv[j].y = wv[j].y - lr * gv[j].y;
+            wv[j].z = wv[j].z - lr * gv[j].z;
+            wv[j].w = wv[j].w - lr * gv[j].w;
+            w[i0 + 256 * j] = wv[j];
+            if (w16) w16[i0 + 256 * j] = make_uint2(pack_bf16x2(wv[j].x, wv[j].y), pack_bf16x2(wv[j].z, wv[j].w));
+        }
+}
+
 // sgd_kernel's update over several short vectors, workgroup b taking vector b
 constexpr int kMaxSgdVecs = 96;
 struct SgdVecs {
@@ -253,6 +294,28 @@ int launch_sgd(float* w, const float* g, float lr, int64_t n, hipStream_t stream
         DT_HIP_TRY(hipGetLastError());
         if (w16) return launch_f32_to_bf16(w, w16, n, stream);
     }
+    DT_HIP_TRY(hipGetLastError());
+    return DT_OK;
+}
+
+int launch_sgd_segs(const SgdSeg* segs, int count, float lr, hipStream_t stream) {
+    SgdSegs v{};
+    int64_t blocks = 0;
+    for (int i = 0; i < kSgdSegs; ++i) {
+        v.block0[i] = INT_MAX;
+        if (i >= count) continue;
+        const SgdSeg& x = segs[i];
+        if (x.n % 4 != 0 || ((uintptr_t)x.w | (uintptr_t)x.g | (uintptr_t)x.w16) % 16 != 0)
+            return set_error(DT_ERR_INVALID_ARG, "SGD segments: a multiple of 4 elements and 16-byte alignment required");
+        v.w[i] = reinterpret_cast<float4*>(x.w);
+        v.g[i] = reinterpret_cast<const float4*>(x.g);
+        v.w16[i] = reinterpret_cast<uint2*>(x.w16);
+        v.n4[i] = x.n / 4;
+        v.block0[i] = (int)blocks;
+        blocks += (x.n / 4 + 1023) / 1024;
+    }
+    if (count < 1 || count > kSgdSegs || blocks > 0x7ffffff) return set_error(DT_ERR_INVALID_ARG, "SGD segments out of range");
+    hipLaunchKernelGGL(sgd_segs_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, v, lr);
     DT_HIP_TRY(hipGetLastError());
     return DT_OK;
 }
