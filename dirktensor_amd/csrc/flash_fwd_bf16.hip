@@ -700,7 +700,7 @@ int persistent_grid(int64_t n_items, int* grid) {
 // Launches with at most one 64-query tile per CU run the kernel of flash_fwd_bf16_few.hip instead: up to T = 1536 (us per
 // call, this kernel / that one: H = 16, T = 1000 18.2 / 15.8; H = 8, T = 1500 22.8 / 19.6; beyond, long items are split
 // here: H = 8, T = 2000 23.5 / 24.0, H = 2, T = 4090 28.5 / 48.5). With up to two tiles per CU it is no faster (H = 16,
-// T = 1530 24.0 / 26.0). Launches that this kernel folds (causal, full sequences of a multiple of 128) stay here too:
+// T = 1530 24.0 / 26.0). Causal launches of full sequences of a multiple of 128, which this kernel folds, stay here too:
 // their results are bit-identical to those of the same rows in any larger launch.
 static bool few_queries(const FlashArgs& a, int cus) {
     const bool folds = a.causal && !a.ragged && a.T % kItemRows == 0 && a.T > kItemRows;
