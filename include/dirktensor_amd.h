@@ -12,7 +12,8 @@
  * d_model = H*D row (OlmoAttention.cpp:71; FlashAttention.cpp:87-88).
  *
  * Modes:
- *   DT_FP32_EXACT  fp32 inputs/outputs, fp32 MFMA (v_mfma_f32_32x32x2_f32),
+ *   DT_FP32_EXACT  fp32 inputs/outputs, fp32 products (the attention's from exact
+ *                  three-way bf16 splits, with less error than fp32 MFMA),
  *                  fp32 accumulation; parity target 1e-4 of max|O|.
  *   DT_BF16        bf16 Q/K/V/O, bf16 MFMA (v_mfma_f32_32x32x16_bf16) with
  *                  fp32 accumulation and fp32 softmax; parity target 2e-2.
