@@ -67,7 +67,6 @@ struct FlashArgs {
 int persistent_grid(int64_t n_items, int* grid);
 int launch_flash_fwd_f32(const FlashArgs& a, const SeqLens* lens, hipStream_t stream);
 int launch_flash_fwd_bf16(const FlashArgs& a, const SeqLens* lens, hipStream_t stream);
-int launch_flash_fwd_bf16_few(const FlashArgs& a, const SeqLens* lens, hipStream_t stream);  // 64-query workgroups
 // split items a launch of the bf16 forward would use (the workspace capacity it needs, in items)
 int flash_fwd_split_items(const FlashArgs& a, const SeqLens* lens, int* n_items);
 

@@ -697,16 +697,6 @@ int persistent_grid(int64_t n_items, int* grid) {
     return DT_OK;
 }
 
-// Launches with at most one 64-query tile per CU run the kernel of flash_fwd_bf16_few.hip instead: up to T = 1536 (us per
-// call, this kernel / that one: H = 16, T = 1000 18.2 / 15.8; H = 8, T = 1500 22.8 / 19.6; beyond, long items are split
-// here: H = 8, T = 2000 23.5 / 24.0, H = 2, T = 4090 28.5 / 48.5). With up to two tiles per CU it is no faster (H = 16,
-// T = 1530 24.0 / 26.0). Causal launches of full sequences of a multiple of 128, which this kernel folds, stay here too:
-// their results are bit-identical to those of the same rows in any larger launch.
-static bool few_queries(const FlashArgs& a, int cus) {
-    const bool folds = a.causal && !a.ragged && a.T % kItemRows == 0 && a.T > kItemRows;
-    return !folds && a.T <= 1536 && (int64_t)((a.T + 63) / 64) * a.B * a.H <= cus;
-}
-
 static int plan(const FlashArgs& a, const SeqLens* lens, int* grid, Schedule* sc) {
     SeqLens sl;
     if (a.ragged) sl = *lens;
@@ -721,9 +711,6 @@ static int plan(const FlashArgs& a, const SeqLens* lens, int* grid, Schedule* sc
 
 int flash_fwd_split_items(const FlashArgs& a, const SeqLens* lens, int* n_items) {
     int grid = 0;
-    *n_items = 0;
-    DT_TRY(persistent_grid(0x7fffffff, &grid));
-    if (few_queries(a, grid)) return DT_OK;
     Schedule sc;
     DT_TRY(plan(a, lens, &grid, &sc));
     *n_items = sc.n_slots;
@@ -735,8 +722,6 @@ int launch_flash_fwd_bf16(const FlashArgs& a, const SeqLens* lens, hipStream_t s
     if ((int64_t)a.T * a.ldk * 2 >= ((int64_t)1 << 31) || (int64_t)a.T * a.ldq * 2 >= ((int64_t)1 << 31))
         return set_error(DT_ERR_UNSUPPORTED, "Q/K/V extent of one sequence exceeds 2 GiB");
     int grid = 0;
-    DT_TRY(persistent_grid(0x7fffffff, &grid));
-    if (few_queries(a, grid)) return launch_flash_fwd_bf16_few(a, lens, stream);
     Schedule sc;
     DT_TRY(plan(a, lens, &grid, &sc));
     if (sc.n_slots > 0 && (sc.n_slots > a.split_slots || !a.split_ws || !a.split_cnt)) {  // no room: whole items

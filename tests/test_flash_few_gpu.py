@@ -1,5 +1,5 @@
-"""bf16 forward of launches with few queries (64-query workgroups, keys in four groups): edges of its query and key tiles,
-ragged batches and both sides of the rule that selects it, against attention in 64 bits."""
+"""bf16 forward of launches with few queries (fewer items than CUs, folded or not): edges of query and key tiles and
+ragged batches, against attention in 64 bits."""
 
 import math
 
@@ -32,7 +32,7 @@ def _reference(q, k, v, causal, lens):
     return o.permute(0, 2, 1, 3), m.permute(0, 2, 1), l.permute(0, 2, 1)
 
 
-# bf16 Q (scaled), K, V and P: 2^-9 each, in sums of many terms; O lies at about 2.4e-3 from 64 bits in either kernel, m and l
+# bf16 Q (scaled), K, V and P: 2^-9 each, in sums of many terms; O lies at about 2.4e-3 from 64 bits, m and l
 # (scores of a few units from bf16 operands) below that
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("B,T,H", [(1, 1, 1), (1, 31, 2), (2, 32, 1), (1, 33, 3), (1, 64, 16), (3, 65, 2), (1, 96, 1), (1, 127, 2),

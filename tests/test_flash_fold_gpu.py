@@ -33,8 +33,6 @@ def test_folded_odd_lengths(B, T, H, dtype):
         assert float((got.double() - want).norm() / want.norm()) < tol
     rep = 300 // (B * H * (T // 128 + 1)) + 1  # more than one round: unfolded
     big = flash_attention_forward(*[t.repeat(1, 1, rep, 1) for t in (q, k, v)], SCALE, True)
-    if dtype == torch.bfloat16 and T <= 1536 and ((T + 63) // 64) * B * H <= 256:
-        return  # (few queries: another kernel, which splits the keys otherwise)
     for i in range(rep):
         assert torch.equal(big.output[:, :, i * H:(i + 1) * H], r.output)
         assert torch.equal(big.softmax_m[:, :, i * H:(i + 1) * H], r.softmax_m)
