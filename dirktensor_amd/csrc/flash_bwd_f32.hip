@@ -2,12 +2,13 @@
 //
 // Replaces flash_attention_backward (FlashAttention.cpp:185-359) with fp32 tensors. As in the forward
 // (flash_fwd_f32.hip), every fp32 product runs on v_mfma_f32_32x32x16_bf16: an operand x is the exact sum of three
-// bf16 values h + m + l, and x y is formed from the six partial products of weight 2^-16 and above, small ones
-// first, accumulated in fp32. That is 192 matrix-pipe cycles per 16 steps of k against 512 on
-// v_mfma_f32_32x32x2_f32, with less rounding (it rounds every second k). Operands that a split does not hold in full
-// (infinities, the last binade, values around 2^-109 and below) are found at the end of a block, from a result that
-// is not finite or from the largest value of each operand, and the wave then repeats its block with the fp32
-// instruction, straight from memory (slow_dkdv, slow_dq).
+// bf16 values h + m + l, and x y is formed from six of their partial products (the other three come to 2^-24 of x y at most),
+// small ones first, accumulated in fp32. That is 192 matrix-pipe cycles per 16 steps of k against 512 on
+// v_mfma_f32_32x32x2_f32, with less rounding (it rounds every second k). Every operand, P and dS too, is split times 2^24,
+// so that no part of any fp32 number is lost under bf16's denormals; that is taken out again where a score enters exp2, in
+// dP, and at a block's end. What a split does not hold (2^103 and above, infinities, NaN) shows in a result that is not
+// finite or in a score of -inf, and the wave then repeats its block with the fp32 instruction, straight from memory
+// (slow_dkdv, slow_dq).
 //
 // Decomposition, as in the bf16 mode: flash_bwd_dkdv owns a block of keys of one (batch, head), 32 per wave with the
 // planes of their K and V rows in registers, and streams 32-query tiles of Q and dO; flash_bwd_dq owns queries (Q and
@@ -58,6 +59,7 @@ typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef short shortx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef short shortx8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
 
@@ -69,7 +71,9 @@ constexpr int kPlanes = 3 * kPlane;              // h, m, l
 constexpr int kBlk = 128;                        // rows owned by a workgroup of one group
 constexpr int kThreads = 256;
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kWide = 0x1p100f;
+constexpr float kNegInf = -__builtin_huge_valf();
+constexpr float kUp = 0x1p24f;      // the operands' factor
+constexpr float kDown2 = 0x1p-48f;  // takes it out of a product
 constexpr int kBufferDword3 = 0x00020000;  // raw buffer, 32-bit data format (gfx9 family)
 
 __device__ __forceinline__ floatx16 mfma(bf16x8 a, bf16x8 b, floatx16 c) {
@@ -114,7 +118,7 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     bf16x2 r = __builtin_convertvector((floatx2){lo, hi}, bf16x2);
     return __builtin_bit_cast(uint32_t, r);
 }
-// the bf16 planes of a pair of floats: x = h + m + l exactly for finite x in 2^-109 .. 2^127
+// the bf16 planes of a pair of floats: x = h + m + l exactly for 0 and |x| in 2^-102 .. 2^127 (fp32 numbers times 2^24)
 struct Split2 {
     uint32_t h, m, l;
 };
@@ -130,11 +134,11 @@ __device__ __forceinline__ Split2 split2(float x0, float x1) {
 struct Frag3 {
     bf16x8 h, m, l;
 };
-// eight accumulator elements as a B operand, packed pair by pair
+// sixteen accumulator elements (two B operands) times 2^24, packed pair by pair
 struct Words3 {
     uint32_t w[3][8];  // [h, m, l][pair of elements]
     __device__ __forceinline__ void put(int pair, float x0, float x1) {
-        const Split2 s = split2(x0, x1);
+        const Split2 s = split2(x0 * kUp, x1 * kUp);
         w[0][pair] = s.h;
         w[1][pair] = s.m;
         w[2][pair] = s.l;
@@ -143,12 +147,6 @@ struct Words3 {
         return __builtin_bit_cast(bf16x8, make_uint4(w[p][4 * u], w[p][4 * u + 1], w[p][4 * u + 2], w[p][4 * u + 3]));
     }
 };
-// max |x| over both lane halves is within what splits hold (or all zero)
-__device__ __forceinline__ bool wide(float amax) { return amax > kWide || (amax < 1.0f / kWide && amax > 0.0f); }
-__device__ __forceinline__ float max4(float a, float4 x) {
-    return fmaxf(a, fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))));
-}
-
 __device__ __forceinline__ int swz(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
 
 // Lane addresses inside a plane.
@@ -265,7 +263,7 @@ struct Stream {
         return load16(r, off + (tile_at + (uint32_t)((8 / G) * n) * ld4));
     }
     __device__ __forceinline__ void put(uint8_t* planes, int n, float4 x) const {
-        const Split2 s0 = split2(x.x, x.y), s1 = split2(x.z, x.w);
+        const Split2 s0 = split2(x.x * kUp, x.y * kUp), s1 = split2(x.z * kUp, x.w * kUp);
         // swz's upper bits count rows of 8/G: G = 1 flips bit 1 on odd units, G = 2 takes n mod 4
         const uint32_t flip = G == 1 ? (uint32_t)(n & 1) << 5 : (uint32_t)(n & 3) << 4;
         uint8_t* p = planes + ((waddr ^ flip) + (uint32_t)(n * (8 / G) * kRow));
@@ -275,24 +273,19 @@ struct Stream {
     }
 };
 
-// the lane's own row, split: f[cc] = X[row][16*cc + 8*hh .. +8] * mul (zeros when row >= T); its largest |x| -> amax
-__device__ __forceinline__ void load_frags(Frag3 (&f)[8], const float* base, int row, int T, int ld, int hh, float mul, float& amax) {
+// the lane's own row, split: f[cc] = X[row][16*cc + 8*hh .. +8] * 2^24 (zeros when row >= T)
+__device__ __forceinline__ void load_frags(Frag3 (&f)[8], const float* base, int row, int T, int ld, int hh) {
     const bool in = row < T;
     const float* p = base + (int64_t)(in ? row : 0) * ld + 8 * hh;
     float4 x[16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) x[j] = *reinterpret_cast<const float4*>(p + 16 * (j >> 1) + 4 * (j & 1));
-    if (!in) mul = 0.0f;
-    float m = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) m = max4(m, x[j]);
-    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
-    amax = in ? fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) : 0.0f;
+    auto up = [&](float v) { return in ? v * kUp : 0.0f; };
 #pragma unroll
     for (int cc = 0; cc < 8; ++cc) {
         const float4 a = x[2 * cc], b = x[2 * cc + 1];
-        const Split2 s0 = split2(in ? a.x * mul : 0.0f, in ? a.y * mul : 0.0f), s1 = split2(in ? a.z * mul : 0.0f, in ? a.w * mul : 0.0f);
-        const Split2 s2 = split2(in ? b.x * mul : 0.0f, in ? b.y * mul : 0.0f), s3 = split2(in ? b.z * mul : 0.0f, in ? b.w * mul : 0.0f);
+        const Split2 s0 = split2(up(a.x), up(a.y)), s1 = split2(up(a.z), up(a.w));
+        const Split2 s2 = split2(up(b.x), up(b.y)), s3 = split2(up(b.z), up(b.w));
         f[cc].h = __builtin_bit_cast(bf16x8, make_uint4(s0.h, s1.h, s2.h, s3.h));
         f[cc].m = __builtin_bit_cast(bf16x8, make_uint4(s0.m, s1.m, s2.m, s3.m));
         f[cc].l = __builtin_bit_cast(bf16x8, make_uint4(s0.l, s1.l, s2.l, s3.l));
@@ -318,6 +311,19 @@ __device__ __forceinline__ float finite_probe(const floatx16 (&x)[4]) {
     return z;
 }
 
+// Keeps a block's finished sums apart from the registers its loop accumulates in (without it the compiler gives the loop's
+// accumulators a place that suits the tail, and spills some eighty registers around the loop).
+__device__ __forceinline__ void settle(floatx16 (&x)[4]) { asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3])); }
+// A score's factor scale log2 e 2^-48 is denormal for the smallest scales: such calls take the fp32 instruction. (scale > 0;
+// compared as an integer, in scalar registers.)
+__device__ __forceinline__ bool scale_fits(float scale) { return __float_as_int(scale) > (127 - 70) << 23; }
+
+// The lane, formed anew: what is computed from it belongs to the place of the call and is not kept in registers before it.
+__device__ __forceinline__ int lane_here() {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+}
 // LDS of one group: the first operand's planes twice, the second's once, and for dK/dV the tile rows' lse2 and delta
 struct GroupLds {
     uint8_t a[2][kPlanes];
@@ -327,10 +333,7 @@ struct GroupLds {
 template <int G>
 union BwdLds {
     GroupLds g[G];
-    struct {
-        float4 x[4][16][64];  // the groups' exchange (G = 2): 64 KB
-        float amax[4][2];
-    } end;
+    float4 x[4][16][64];  // the groups' exchange (G = 2): 64 KB
 };
 static_assert(sizeof(BwdLds<2>) <= 160 * 1024, "LDS of one CU");
 
@@ -340,45 +343,23 @@ __device__ __forceinline__ const FlashBwdArgs* kernel_args() {
     return (const FlashBwdArgs*)__builtin_amdgcn_kernarg_segment_ptr();
 }
 
-// The largest |x| of each streamed operand over the workgroup's waves (each wave saw its share of its group's tiles;
-// the whole workgroup's is as good), through LDS that nothing else uses now. Ends with a barrier.
-__device__ __forceinline__ bool wide_streams(float (&lds)[4][2], float a0, float a1, int wave, int lane) {
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) {
-        a0 = fmaxf(a0, __shfl_xor(a0, s, 64));
-        a1 = fmaxf(a1, __shfl_xor(a1, s, 64));
-    }
-    if (lane == 0) {
-        lds[wave][0] = a0;
-        lds[wave][1] = a1;
-    }
-    lds_barrier();
-    float m0 = 0.0f, m1 = 0.0f;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        m0 = fmaxf(m0, lds[w][0]);
-        m1 = fmaxf(m1, lds[w][1]);
-    }
-    return wide(m0) || wide(m1);
-}
-
 // The two groups' partial sums: group g keeps own + other of `keep` and hands `give` over (group 0's terms first).
-__device__ __forceinline__ void add_groups(floatx16 (&keep)[4], const floatx16 (&give)[4], float4 (&x)[4][16][64], int grp, int wave, int lane) {
+__device__ __forceinline__ void add_groups(floatx16 (&keep)[4], const floatx16 (&give)[4], float f, float4 (&x)[4][16][64], int grp, int wave, int lane) {
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
         for (int g = 0; g < 4; ++g)
-            x[wave][4 * db + g][lane] = make_float4(give[db][4 * g], give[db][4 * g + 1], give[db][4 * g + 2], give[db][4 * g + 3]);
+            x[wave][4 * db + g][lane] = make_float4(give[db][4 * g] * f, give[db][4 * g + 1] * f, give[db][4 * g + 2] * f, give[db][4 * g + 3] * f);
     lds_barrier();
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const float4 y = x[wave ^ 2][4 * db + g][lane];
-            keep[db][4 * g] = grp ? y.x + keep[db][4 * g] : keep[db][4 * g] + y.x;
-            keep[db][4 * g + 1] = grp ? y.y + keep[db][4 * g + 1] : keep[db][4 * g + 1] + y.y;
-            keep[db][4 * g + 2] = grp ? y.z + keep[db][4 * g + 2] : keep[db][4 * g + 2] + y.z;
-            keep[db][4 * g + 3] = grp ? y.w + keep[db][4 * g + 3] : keep[db][4 * g + 3] + y.w;
+            keep[db][4 * g] = keep[db][4 * g] * f + y.x;
+            keep[db][4 * g + 1] = keep[db][4 * g + 1] * f + y.y;
+            keep[db][4 * g + 2] = keep[db][4 * g + 2] * f + y.z;
+            keep[db][4 * g + 3] = keep[db][4 * g + 3] * f + y.w;
         }
 }
 
@@ -486,21 +467,17 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
 #pragma unroll
     for (int n = 0; n < Stream<G>::kUnits; ++n) y[n] = sg.load(sg.at(grp, q_begin, n_tiles), n);
     Frag3 kf[8], vf[8];
-    float kmax, vmax, qmax = 0.0f, gmax = 0.0f;
-    load_frags(kf, Kg, key, T, a.ld_qkv, hh, 1.0f, kmax);
-    load_frags(vf, Vg, key, T, a.ld_qkv, hh, 1.0f, vmax);
+    load_frags(kf, Kg, key, T, a.ld_qkv, hh);
+    load_frags(vf, Vg, key, T, a.ld_qkv, hh);
+    float s_min = 0.0f;  // the lowest score
     KvAcc A;
 #pragma unroll
     for (int db = 0; db < 4; ++db) A.dv[db] = A.dk[db] = zero16();
 
     auto put_q = [&](int t, int n) {  // unit n of Q's tile t -> its planes, then dO's unit of that tile is requested
-        qmax = max4(qmax, x[n]);
         sq.put(my.a[t & 1], n, x[n]);
     };
-    auto put_g = [&](int n) {
-        gmax = max4(gmax, x[n]);
-        sg.put(my.b, n, x[n]);
-    };
+    auto put_g = [&](int n) { sg.put(my.b, n, x[n]); };
     auto put_stat = [&](int buf) {
         if (w < 2 && lane < 32) my.stats[buf][w][lane] = xs;
     };
@@ -521,6 +498,7 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
         const int q0 = q_begin + t * kTile;
         const int cur = it & 1, nxt = cur ^ 1;
         const uint8_t* qt = my.a[cur];
+        const int lane = lane_here(), ln = lane & 31, hh = lane >> 5, key = kw + ln;
         // some query of the tile is at or after some key of the wave
         const bool visible = t < n_tiles && !(a.causal && q0 + kTile - 1 < kw) && kw < T;
         const uint32_t g_at = sg.at(t + G, q_begin, n_tiles), q_at = sq.at(t + 2 * G, q_begin, n_tiles);
@@ -553,12 +531,25 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
             // element i is masked when dmask > 8*(i/4) + i%4, i.e. when key > query (causal); with dS stored, keys past
             // T are masked too (their dS would otherwise be exp2(-lse2) (-delta))
             const int dmask = (kEmitDs && key >= T) ? INT_MAX : a.causal ? key - (q0 + 4 * hh) : INT_MIN;
+            const __amdgpu_buffer_rsrc_t ds_block = [&] {
+                if constexpr (kEmitDs) {
+                    const BwdDsLayout lay(T, a.causal);
+                    const int kb = kw / 128;
+                    return make_rsrc(static_cast<const uint8_t*>(a.ds_ws) +
+                                         (uint64_t)(bh * lay.per_head() + lay.block_offset(kb) + (q0 / 64 - lay.first_tile(kb))) * kDsBlockBytes,
+                                     (uint32_t)kDsBlockBytes);
+                } else {
+                    return make_rsrc(a.ds_ws, 0u);
+                }
+            }();
+            const uint32_t ds_row = (uint32_t)((kw % 128 + ln) * kDsRowBytes + (q0 & 32) * 4 + 16 * hh);
             dp = dot_rows(my.b, LA, vf, [&](auto I) {  // P = exp2(S c - lse2), in place of S, and its split
                 constexpr int i = decltype(I)::value;
                 if constexpr (i < 4) {
 #pragma unroll
                     for (int e = 4 * i; e < 4 * i + 4; ++e) {
-                        const float p = __builtin_amdgcn_exp2f(sc[e] * c - L[e]);
+                        s_min = fminf(s_min, sc[e]);
+                        const float p = __builtin_amdgcn_exp2f(fmaf(sc[e], c * kDown2, -L[e]));
                         sc[e] = dmask > 8 * (e / 4) + (e % 4) ? 0.0f : p;
                     }
                 } else {
@@ -569,22 +560,17 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
                 constexpr int i = decltype(I)::value;
                 if constexpr (i < 4) {
 #pragma unroll
-                    for (int e = 4 * i; e < 4 * i + 4; ++e) dp[e] = sc[e] * (dp[e] - D[e]);
+                    for (int e = 4 * i; e < 4 * i + 4; ++e) dp[e] = sc[e] * fmaf(dp[e], kDown2, -D[e]);
                 } else {
-                    dw.put(2 * (i - 4), dp[4 * (i - 4)], dp[4 * (i - 4) + 1]);
-                    dw.put(2 * (i - 4) + 1, dp[4 * (i - 4) + 2], dp[4 * (i - 4) + 3]);
+                    constexpr int g = i - 4;
+                    dw.put(2 * g, dp[4 * g], dp[4 * g + 1]);
+                    dw.put(2 * g + 1, dp[4 * g + 2], dp[4 * g + 3]);
+                    if constexpr (kEmitDs)  // chunk 2*g + hh of this query block's half of the lane's key row
+                        __builtin_amdgcn_raw_buffer_store_b128(
+                            __builtin_bit_cast(u32x4, make_float4(dp[4 * g], dp[4 * g + 1], dp[4 * g + 2], dp[4 * g + 3])), ds_block,
+                            ds_row + 32 * g, 0, 0);
                 }
             });
-            if constexpr (kEmitDs) {  // chunk 2*g + hh of this query block's half of the lane's key row
-                const BwdDsLayout lay(T, a.causal);
-                const int kb = kw / 128;
-                uint8_t* blk = static_cast<uint8_t*>(a.ds_ws) +
-                               (uint64_t)(bh * lay.per_head() + lay.block_offset(kb) + (q0 / 64 - lay.first_tile(kb))) * kDsBlockBytes;
-                uint8_t* row = blk + (kw % 128 + ln) * kDsRowBytes + (q0 & 32) * 4 + 16 * hh;
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    *reinterpret_cast<float4*>(row + 32 * g) = make_float4(dp[4 * g], dp[4 * g + 1], dp[4 * g + 2], dp[4 * g + 3]);
-            }
         } else {
 #pragma unroll
             for (int n = 0; n < Stream<G>::kUnits; ++n) move_q(n);
@@ -606,26 +592,30 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
     }
 
     {
-        const bool ws = wide_streams(lds.end.amax, qmax, gmax, wave, lane);
+        const int lane = lane_here(), hh = lane >> 5, key = kw + (lane & 31);
         const float z = finite_probe(A.dv) + finite_probe(A.dk);
-        const bool bad = key < T && (!(z == 0.0f) || ws || wide(kmax) || wide(vmax));
+        const bool bad = key < T && (!(z == 0.0f) || s_min == kNegInf || !scale_fits(a.scale));
+        float f = kDown2;  // takes the operands' factors out
         if (__builtin_amdgcn_ballot_w64(bad) != 0) {
-            KvAcc S;  // (an object of its own: A stays in registers)
+            KvAcc S;
             slow_dkdv(S, *kernel_args(), bh, kw, grp, G, n_tiles, q_begin, kEmitDs);
+            settle(S.dv);
+            settle(S.dk);
             A = S;
+            f = 1.0f;
         }
-    }
-    if constexpr (G == 2) {
-        if (grp == 0) {
-            add_groups(A.dv, A.dk, lds.end.x, 0, wave, lane);
-            if (key < T) store_rows(dVg, key, a.ld_grad, hh, A.dv, 1.0f);
-        } else {
-            add_groups(A.dk, A.dv, lds.end.x, 1, wave, lane);
-            if (key < T) store_rows(dKg, key, a.ld_grad, hh, A.dk, a.scale);  // dS carries the reference's scale (:293)
+        if constexpr (G == 2) {
+            if (grp == 0) {
+                add_groups(A.dv, A.dk, f, lds.x, 0, wave, lane);
+                if (key < T) store_rows(dVg, key, a.ld_grad, hh, A.dv, 1.0f);
+            } else {
+                add_groups(A.dk, A.dv, f, lds.x, 1, wave, lane);
+                if (key < T) store_rows(dKg, key, a.ld_grad, hh, A.dk, a.scale);  // dS carries the reference's scale (:293)
+            }
+        } else if (key < T) {
+            store_rows(dKg, key, a.ld_grad, hh, A.dk, a.scale * f);
+            store_rows(dVg, key, a.ld_grad, hh, A.dv, f);
         }
-    } else if (key < T) {
-        store_rows(dKg, key, a.ld_grad, hh, A.dk, a.scale);
-        store_rows(dVg, key, a.ld_grad, hh, A.dv, 1.0f);
     }
 }
 
@@ -707,23 +697,17 @@ __device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int 
 #pragma unroll
     for (int n = 0; n < Stream<G>::kUnits; ++n) y[n] = sv.load(sv.at(grp, 0, n_tiles), n);
     Frag3 qf[8], gf[8];
-    float qmax, gmax, kmax = 0.0f, vmax = 0.0f;
-    load_frags(qf, static_cast<const float*>(a.q) + qkv, q, T, a.ld_qkv, hh, 1.0f, qmax);
-    load_frags(gf, Gg, q, T, a.ld_o, hh, 1.0f, gmax);
+    load_frags(qf, static_cast<const float*>(a.q) + qkv, q, T, a.ld_qkv, hh);
+    load_frags(gf, Gg, q, T, a.ld_o, hh);
+    float s_min = 0.0f;  // the lowest score
     const float lse2 = q < T ? a.lse2[(int64_t)bh * T + q] : 0.0f;
     const float delta = q < T ? a.delta[(int64_t)bh * T + q] : 0.0f;
     const int lim = a.causal ? min(q, T - 1) : T - 1;  // keys > lim are masked
     QAcc A;
 #pragma unroll
     for (int db = 0; db < 4; ++db) A.dq[db] = zero16();
-    auto put_k = [&](int buf, int n) {
-        kmax = max4(kmax, x[n]);
-        sk.put(my.a[buf], n, x[n]);
-    };
-    auto put_v = [&](int n) {
-        vmax = max4(vmax, x[n]);
-        sv.put(my.b, n, x[n]);
-    };
+    auto put_k = [&](int buf, int n) { sk.put(my.a[buf], n, x[n]); };
+    auto put_v = [&](int n) { sv.put(my.b, n, x[n]); };
 #pragma unroll
     for (int n = 0; n < Stream<G>::kUnits; ++n) put_k(0, n);
 #pragma unroll
@@ -763,13 +747,14 @@ __device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int 
                 if constexpr (i < 8) {
 #pragma unroll
                     for (int e = 2 * i; e < 2 * i + 2; ++e) {
-                        const float p = __builtin_amdgcn_exp2f(sc[e] * c - lse2);
+                        s_min = fminf(s_min, sc[e]);
+                        const float p = __builtin_amdgcn_exp2f(fmaf(sc[e], c * kDown2, -lse2));
                         sc[e] = 8 * (e / 4) + (e % 4) > emask ? 0.0f : p;
                     }
                 }
             });
 #pragma unroll
-            for (int e = 0; e < 16; ++e) dp[e] = sc[e] * (dp[e] - delta);
+            for (int e = 0; e < 16; ++e) dp[e] = sc[e] * fmaf(dp[e], kDown2, -delta);
 #pragma unroll
             for (int e = 0; e < 4; ++e) dw.put(e, dp[2 * e], dp[2 * e + 1]);
         } else {
@@ -794,24 +779,24 @@ __device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int 
         lds_barrier();  // the next tile's planes are written
     }
 
-    {
-        const bool ws = wide_streams(lds.end.amax, kmax, vmax, wave, lane);
-        const bool bad = q < T && (!(finite_probe(A.dq) == 0.0f) || ws || wide(qmax) || wide(gmax));
-        if (__builtin_amdgcn_ballot_w64(bad) != 0) {
-            QAcc S;
-            slow_dq(S, *kernel_args(), bh, qw, grp, G, n_tiles);
-            A = S;
-        }
+    const bool bad = q < T && (!(finite_probe(A.dq) == 0.0f) || s_min == kNegInf || !scale_fits(a.scale));
+    float f = kDown2;  // takes the operands' factors out
+    if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+        QAcc S;
+        slow_dq(S, *kernel_args(), bh, qw, grp, G, n_tiles);
+        settle(S.dq);
+        A = S;
+        f = 1.0f;
     }
     if constexpr (G == 2) {  // group g stores dims 64g .. 64g+63
-        float4(&ex)[4][16][64] = lds.end.x;
+        float4(&ex)[4][16][64] = lds.x;
         auto at = [&](int db, int g) -> float4& { return ex[wave][4 * (db & 1) + g][lane]; };
 #pragma unroll
         for (int d = 0; d < 2; ++d)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const floatx16 v = grp ? A.dq[d] : A.dq[2 + d];
-                at(d, g) = make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
+                at(d, g) = make_float4(v[4 * g] * f, v[4 * g + 1] * f, v[4 * g + 2] * f, v[4 * g + 3] * f);
             }
         lds_barrier();
         if (q < T) {
@@ -823,19 +808,18 @@ __device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int 
                     const floatx16 v = grp ? A.dq[2 + d] : A.dq[d];
                     const float4 o = ex[wave ^ 2][4 * d + g][lane];
                     *reinterpret_cast<float4*>(p + 32 * d + 8 * g) =
-                        make_float4((v[4 * g] + o.x) * a.scale, (v[4 * g + 1] + o.y) * a.scale, (v[4 * g + 2] + o.z) * a.scale,
-                                    (v[4 * g + 3] + o.w) * a.scale);
+                        make_float4((v[4 * g] * f + o.x) * a.scale, (v[4 * g + 1] * f + o.y) * a.scale, (v[4 * g + 2] * f + o.z) * a.scale,
+                                    (v[4 * g + 3] * f + o.w) * a.scale);
                 }
         }
     } else if (q < T) {
-        store_rows(dQg, q, a.ld_grad, hh, A.dq, a.scale);
+        store_rows(dQg, q, a.ld_grad, hh, A.dq, a.scale * f);
     }
 }
 
 // ------------------------------------------------------------------------------------------------ dQ from dS
 struct DsLds {
     uint8_t k[2][kPlanes];
-    float amax[4][2];
 };
 
 __device__ __noinline__ void slow_dq_ds(QAcc& A, const FlashBwdArgs& a, int bh, int qw, int n_use) {
@@ -899,12 +883,10 @@ __device__ __forceinline__ void dq_ds_block(const FlashBwdArgs& a, int qb_own, i
 #pragma unroll
     for (int db = 0; db < 4; ++db) A.dq[db] = zero16();
     float4 x[4];
-    float kmax = 0.0f, dmax = 0.0f;
 #pragma unroll
     for (int n = 0; n < 4; ++n) x[n] = sk.load(sk.at(0, 0, n_tiles), n);
     load_ds(0);
     auto move_k = [&](int t, uint32_t next_at, int n) {
-        kmax = max4(kmax, x[n]);
         sk.put(lds.k[t & 1], n, x[n]);
         x[n] = sk.load(next_at, n);
     };
@@ -916,10 +898,7 @@ __device__ __forceinline__ void dq_ds_block(const FlashBwdArgs& a, int qb_own, i
         if (t < n_use) {
             Words3 dw;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                dw.put(e, ds[2 * e], ds[2 * e + 1]);
-                dmax = fmaxf(dmax, fmaxf(fabsf(ds[2 * e]), fabsf(ds[2 * e + 1])));
-            }
+            for (int e = 0; e < 8; ++e) dw.put(e, ds[2 * e], ds[2 * e + 1]);
             load_ds(t + 1);
             acc_cols(A.dq, lds.k[t & 1], LA, dw, [&](auto I) {
                 constexpr int i = decltype(I)::value;
@@ -931,16 +910,15 @@ __device__ __forceinline__ void dq_ds_block(const FlashBwdArgs& a, int qb_own, i
         }
         lds_barrier();
     }
-    {
-        const bool ws = wide_streams(lds.amax, kmax, dmax, wave, lane);
-        const bool bad = q < T && (!(finite_probe(A.dq) == 0.0f) || ws);
-        if (__builtin_amdgcn_ballot_w64(bad) != 0) {
-            QAcc S;
-            slow_dq_ds(S, *kernel_args(), bh, qw, n_use);
-            A = S;
-        }
+    const bool bad = q < T && !(finite_probe(A.dq) == 0.0f);
+    float f = a.scale * kDown2;
+    if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+        QAcc S;
+        slow_dq_ds(S, *kernel_args(), bh, qw, n_use);
+        A = S;
+        f = a.scale;
     }
-    if (q < T) store_rows(dQg, q, a.ld_grad, hh, A.dq, a.scale);
+    if (q < T) store_rows(dQg, q, a.ld_grad, hh, A.dq, f);
 }
 
 // One block per workgroup, listed in decreasing causal cost, so that the hardware, which hands the next workgroup to

@@ -8,21 +8,20 @@
 // round folds its units instead (flash_items.h): an item is then the 64-query
 // tiles p and n-1-p of one (batch, head), rows 0-63 and 64-127.
 //
-// Products. Every fp32 operand x is split into three bf16 values x = h + m + l
-// (each the rounding of what the ones before it leave: 24 significand bits in
-// three times 8, so the sum is x itself), and a product x y is formed on
-// v_mfma_f32_32x32x16_bf16 from the six partial products of weight 2^-16 and
-// above (lh, hl, mm, mh, hm, hh; the three left out are below 2^-26 of x y),
-// accumulated in fp32. Six bf16 MFMAs take 192 cycles for 16 steps of k where
-// v_mfma_f32_32x32x2_f32 takes 512, and the result is nearer to the exact one:
-// over random 128-long dot products the relative error (2-norm) is 6.1e-8 with
-// the small partial products summed first, against 2.0e-7 for the fp32
-// instruction, which rounds after every second k instead of after every sixteenth.
-// Infinities and the last binade do not split (inf * 0 in a partial product is
-// NaN, and rounding to bf16 overflows), and below 2^-109 the last part falls under
-// bf16's smallest denormal. A wave whose result is not finite, whose softmax is empty
-// where it has keys, or whose queries or output lie outside [2^-100, 2^100],
-// therefore repeats its keys with the fp32 instruction, straight from memory
+// Products. Every fp32 operand x is taken times 2^24 and split into three bf16 values x = h + m + l (each the rounding
+// of what the ones before it leave: 24 significand bits in three times 8, so the sum is x itself), and a product x y is
+// formed on v_mfma_f32_32x32x16_bf16 from the six partial products lh, hl, mm, mh, hm, hh, accumulated in fp32. The
+// three left out (ml, lm, ll) come to at most 2^-24 of x y, the size of one fp32 rounding, and to 2^-28 on average. Six
+// bf16 MFMAs take 192 cycles for 16 steps of k where v_mfma_f32_32x32x2_f32 takes 512, and the result is nearer to the
+// exact one: over random 128-long dot products the relative error (2-norm) is 6.1e-8 with the small partial products
+// summed first, against 2.0e-7 for the fp32 instruction, which rounds after every second k instead of after every
+// sixteenth.
+//
+// The factor 2^24 (for Q: scale log2 e times a power of two) keeps every part of every fp32 number, the smallest too, above
+// bf16's denormals, whatever lies beside it in its row. It is exact, and taken out again where a score enters exp2 and
+// at an item's end. What is left out of the split's range is 2^103 and above, infinities and NaN: they give a result that
+// is not finite (a scaled operand or sum that overflows to infinity, inf * 0 = NaN), an empty softmax where there are keys,
+// or a score of -inf. A wave that finds one of these repeats its keys with the fp32 instruction, straight from memory
 // (slow_keys), and keeps that result.
 //
 // Work split: 8 waves in two groups of 4. Both groups hold the same 128 queries
@@ -71,7 +70,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef short shortx4 __attribute__((ext_vector_type(4)));
 typedef short shortx8 __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
 
 constexpr int kD = 128;                      // head_dim (model_config.h:3)
@@ -87,8 +85,8 @@ constexpr int kObufRow = kD * 4 + 16;        // a row of the output staging tile
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kNegInf = -__builtin_huge_valf();
 constexpr float kInf = __builtin_huge_valf();
-constexpr float kRescaleLog2 = 8.0f;
-constexpr float kWide = 0x1p100f;
+constexpr uint32_t kRescaleExp = 3;  // the reference point moves when a score exceeds it by 2^3 in the log2 domain
+constexpr float kUp = 0x1p24f;  // the operands' factor
 constexpr int kBufferDword3 = 0x00020000;  // raw buffer, 32-bit data format (gfx9 family)
 
 // LDS: the groups' planes [group](K h, m, l, V h, m, l) in the loop; at an item's end the exchange between the groups
@@ -114,7 +112,7 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     bf16x2 r = __builtin_convertvector((floatx2){lo, hi}, bf16x2);
     return __builtin_bit_cast(uint32_t, r);
 }
-// the bf16 planes of a pair of floats: x = h + m + l exactly for finite x below 2^127
+// the bf16 planes of a pair of floats: x = h + m + l exactly for 0 and |x| in 2^-102 .. 2^127 (fp32 numbers times 2^24)
 struct Split2 {
     uint32_t h, m, l;
 };
@@ -157,7 +155,22 @@ __device__ __forceinline__ float4 load16(__amdgpu_buffer_rsrc_t r, uint32_t off)
 // LDS accesses only: vector memory requests in flight (the next tiles, output stores) are not waited for
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// Per-wave state of one item: O^T: o[db][i] = O[qrow][32*db + 8*(i/4) + 4*hh + i%4] (unnormalised, relative to m_s)
+// The lane, formed anew: what is computed from it belongs to the place of the call and is not kept in registers across the
+// item loop, which needs all of them (kept, some forty of them were spilled to scratch memory).
+__device__ __forceinline__ int lane_here() {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+}
+
+// likewise the scale
+__device__ __forceinline__ float scale_here(float s) {
+    asm volatile("" : "+s"(s));
+    return s;
+}
+
+// Per-wave state of one item: O^T: o[db][i] = O[qrow][32*db + 8*(i/4) + 4*hh + i%4] (unnormalised, relative to m_s). In the
+// split products' loop o is 2^48 times that and m_t and m_s are 1 / down times what they say.
 struct Acc {
     floatx16 o[4];
     float m_t, m_s, l;  // this lane half's maximum, the reference point (the same in both halves), this half's sum
@@ -253,12 +266,19 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
 
     const int T = a.T;
     const int G = gridDim.x;
-    const float c = a.scale * kLog2e;
+    // Q's factor: c = scale log2 e times the power of two 2^24 / 2^e, 2^e <= scale < 2^(e+1); and what takes it and K's out of
+    // a score again, 2^(e-48), which would be denormal for the smallest scales: such calls take the fp32 instruction
+    const uint32_t sb = __float_as_uint(a.scale), se = sb >> 23;  // se = e + 127
+    const bool scale_fits = se > 56;
+    const float cu = __uint_as_float((sb & 0x7fffffu) | (127u + 24u) << 23) * kLog2e;
+    const float down = __uint_as_float((scale_fits ? se - 48 : 127u) << 23);
+    const float grow_by = __uint_as_float((scale_fits ? 127u + kRescaleExp + (48 + 127) - se : 127u) << 23);  // 2^kRescaleExp / down
 
     for (int round = 0;; ++round) {
         const int k_unit = snake_item(round, G, (int)blockIdx.x);
         if (k_unit >= sc.n_units) break;
         const Unit u = decode_unit(k_unit, sc, a.H, sc.cum);  // a whole item: this kernel's schedules split nothing
+        const int lane = lane_here(), ln = lane & 31, hh = lane >> 5;
         const int b = u.b, h = u.h;
         const int L = u.L;  // valid keys / rows of this sequence
         const int q0 = u.qa;
@@ -299,7 +319,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
         };
         // that unit -> the planes
         auto put = [&](int kv, int n, float4 x) {
-            const Split2 s0 = split2(x.x, x.y), s1 = split2(x.z, x.w);
+            const Split2 s0 = split2(x.x * kUp, x.y * kUp), s1 = split2(x.z * kUp, x.w * kUp);
             uint8_t* p = kv ? vput + n * 8 * kRowV : kput + n * 8 * kRowK;
             const int plane = kv ? kPlaneV : kPlaneK;
             *reinterpret_cast<uint2*>(p) = make_uint2(s0.h, s1.h);
@@ -311,9 +331,8 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
 #pragma unroll
         for (int n = 0; n < 4; ++n) xk[n] = load(0, grp, n);
 
-        // Q fragment, times scale * log2 e, split: qf[cc] = Q[qrow][16*cc + 8*hh .. +8] * c
+        // Q fragment, times cu, split: qf[cc] = Q[qrow][16*cc + 8*hh .. +8] * cu
         Frag3 qf[8];
-        bool q_wide;  // values whose products a split may not hold in full
         {
             const float* qp = Qg + (int64_t)min(qrow, T - 1) * a.ldq + 8 * hh;  // (rows past T: any values)
             float4 xq[16];
@@ -323,17 +342,11 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
             for (int n = 0; n < 4; ++n) x[n] = load(1, grp, n);
 #pragma unroll
             for (int n = 0; n < 4; ++n) put(0, n, xk[n]);  // the group's first K tile
-            float qmax = 0.0f;
-#pragma unroll
-            for (int j = 0; j < 16; ++j)
-                qmax = fmaxf(qmax, fmaxf(fmaxf(fabsf(xq[j].x), fabsf(xq[j].y)), fmaxf(fabsf(xq[j].z), fabsf(xq[j].w))));
-            qmax = max_halves(qmax);
-            q_wide = qmax > kWide || (qmax < 1.0f / kWide && qmax > 0.0f);
 #pragma unroll
             for (int cc = 0; cc < 8; ++cc) {
                 const float4 x0 = xq[2 * cc], x1 = xq[2 * cc + 1];
-                const Split2 s0 = split2(x0.x * c, x0.y * c), s1 = split2(x0.z * c, x0.w * c);
-                const Split2 s2 = split2(x1.x * c, x1.y * c), s3 = split2(x1.z * c, x1.w * c);
+                const Split2 s0 = split2(x0.x * cu, x0.y * cu), s1 = split2(x0.z * cu, x0.w * cu);
+                const Split2 s2 = split2(x1.x * cu, x1.y * cu), s3 = split2(x1.z * cu, x1.w * cu);
                 qf[cc].h = __builtin_bit_cast(bf16x8, make_uint4(s0.h, s1.h, s2.h, s3.h));
                 qf[cc].m = __builtin_bit_cast(bf16x8, make_uint4(s0.m, s1.m, s2.m, s3.m));
                 qf[cc].l = __builtin_bit_cast(bf16x8, make_uint4(s0.l, s1.l, s2.l, s3.l));
@@ -347,6 +360,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
         A.m_t = kNegInf;
         A.m_s = kNegInf;
         A.l = 0.0f;
+        float s_min = 0.0f;  // the lowest score
 
         lds_barrier();
 
@@ -360,13 +374,13 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
             floatx16 st;
             uint32_t pw[3][8];  // P's planes, packed pairs
             auto split_p = [&](int j) {
-                const Split2 s = split2(st[2 * j], st[2 * j + 1]);
+                const Split2 s = split2(st[2 * j] * kUp, st[2 * j + 1] * kUp);
                 pw[0][j] = s.h;
                 pw[1][j] = s.m;
                 pw[2][j] = s.l;
             };
             if (visible) {
-                // S^T, with V's planes written under it: st[i] = t[qrow][key], key = k0 + 8*(i/4) + 4*hh + i%4; the five
+                // S^T, with V's planes written under it: st[i] = t[qrow][key] / down, key = k0 + 8*(i/4) + 4*hh + i%4; the five
                 // small partial products of every chunk first, then the large one (K's h plane is read again for it).
                 // Fragments are read one chunk ahead of their MFMAs.
                 auto read_k = [&](int cc, int p) {
@@ -403,6 +417,8 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
                     DT_BUNDLE_END;
                 });
 
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s_min = fminf(s_min, st[i]);
                 if (k0 + kBN > L || (a.causal && k0 + kBN - 1 > qw0)) {  // diagonal / ragged tail only
                     asm volatile("");  // keeps this block a branch
 #pragma unroll
@@ -417,11 +433,11 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
                 }
                 const float tmax = fmaxf(t0, t1);
                 A.m_t = fmaxf(A.m_t, tmax);
-                const bool grow = (A.m_s == kNegInf) ? (tmax > kNegInf) : (tmax > A.m_s + kRescaleLog2);
+                const bool grow = (A.m_s == kNegInf) ? (tmax > kNegInf) : (tmax > A.m_s + grow_by);
                 if (__builtin_amdgcn_ballot_w64(grow) != 0) {  // wave-uniform, rare after the first tile
                     asm volatile("");  // keeps this block a branch
                     const float m_new = max_halves(A.m_t);
-                    const float alpha = (A.m_s == kNegInf) ? 0.0f : exp2f(A.m_s - m_new);
+                    const float alpha = (A.m_s == kNegInf) ? 0.0f : exp2f((A.m_s - m_new) * down);
                     A.m_s = m_new;
                     A.l *= alpha;
 #pragma unroll
@@ -429,12 +445,12 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
 #pragma unroll
                         for (int i = 0; i < 16; ++i) A.o[db][i] *= alpha;
                 }
-                const float ref = (A.m_s == kNegInf) ? 0.0f : A.m_s;
+                const float ref = (A.m_s == kNegInf) ? 0.0f : A.m_s * down;
                 float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll
                 for (int i = 0; i < 16; i += 2) {
-                    st[i] = __builtin_amdgcn_exp2f(st[i] - ref);
-                    st[i + 1] = __builtin_amdgcn_exp2f(st[i + 1] - ref);
+                    st[i] = __builtin_amdgcn_exp2f(fmaf(st[i], down, -ref));
+                    st[i + 1] = __builtin_amdgcn_exp2f(fmaf(st[i + 1], down, -ref));
                     s0 += st[i];
                     s1 += st[i + 1];
                 }
@@ -479,7 +495,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
                         put(0, f / 6, x[f / 6]);
                         x[f / 6] = load(1, kt + 2, f / 6);
                     }
-                    if constexpr (f % 1 == 1-1) DT_BUNDLE_END;
+                    DT_BUNDLE_END;
                 });
             } else {
 #pragma unroll
@@ -492,113 +508,115 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
         }
         if (!grp && skew) lds_barrier();
 
+        float f = 1.0f / (kUp * kUp), fm = down;  // take the operands' factors out
         {
-            // a result that is not finite or below what V's split holds in full, an empty softmax over visible keys, or
-            // wide queries: the wave's keys again, in fp32
-            float z = A.l * 0.0f, omax = 0.0f;
+            // a result that is not finite, an empty softmax over visible keys, or a score of -inf: the wave's keys again,
+            // in fp32
+            float z = A.l * 0.0f;
 #pragma unroll
             for (int db = 0; db < 4; ++db)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    z = fmaf(A.o[db][i], 0.0f, z);
-                    omax = fmaxf(omax, fabsf(A.o[db][i]));
-                }
+                for (int i = 0; i < 16; ++i) z = fmaf(A.o[db][i], 0.0f, z);
             const bool keys = grp * kBN <= lim;
-            const bool bad = qrow < L && keys && (!(z == 0.0f) || !(sum_halves(A.l) > 0.0f) || q_wide ||
-                                                  (omax < 1.0f / kWide && omax > 0.0f));
+            const bool bad = qrow < L && keys && (!(z == 0.0f) || !(sum_halves(A.l) > 0.0f) || s_min == kNegInf || !scale_fits);
             if (__builtin_amdgcn_ballot_w64(bad) != 0) {
                 Acc S;  // (an object of its own: A stays in registers)
                 slow_keys(S, Qg + (int64_t)min(qrow, T - 1) * a.ldq, Kg, Vg, a.ldk, a.ldv, grp, n_tiles, qw0, lim, L, T,
-                          a.causal, c);
+                          a.causal, scale_here(a.scale) * kLog2e);
                 A = S;
+                f = fm = 1.0f;
             }
         }
 
-        // Merge: group g finalises dims 64g .. 64g+63 of its block's rows and hands the other half of its partial O to the
-        // other group (float4 k of lane `lane` at xo(g)[k*64 + lane]), with its (m_s, m_t, l) at xs(g). The loop's last
-        // barrier has freed the planes.
-        A.m_t = max_halves(A.m_t);
-        A.l = sum_halves(A.l);
-        auto xo = [&](int g) { return reinterpret_cast<float4*>(lds) + (g * 4 + wq) * (8 * 64); };
-        auto xs = [&](int g) { return reinterpret_cast<float*>(lds + kXoBytes) + (g * 4 + wq) * (3 * 64); };
-        uint8_t* obuf = lds + kXoBytes + kXsBytes;  // the output tile on its way to HBM
         {
-            float4* out = xo(grp);
-            auto hand = [&](auto DB) {
-                constexpr int db = decltype(DB)::value;
+            // Merge: group g finalises dims 64g .. 64g+63 of its block's rows and hands the other half of its partial O to the
+            // other group (float4 k of lane `lane` at xo(g)[k*64 + lane]), with its (m_s, m_t, l) at xs(g). The loop's last
+            // barrier has freed the planes.
+            A.m_t = max_halves(A.m_t) * fm;
+            A.m_s *= fm;
+            A.l = sum_halves(A.l);
+            const int lane = lane_here(), ln = lane & 31, hh = lane >> 5, qrow = qw0 + ln;
+            auto xo = [&](int g) { return reinterpret_cast<float4*>(lds) + (g * 4 + wq) * (8 * 64); };
+            auto xs = [&](int g) { return reinterpret_cast<float*>(lds + kXoBytes) + (g * 4 + wq) * (3 * 64); };
+            uint8_t* obuf = lds + kXoBytes + kXsBytes;  // the output tile on its way to HBM
+            {
+                float4* out = xo(grp);
+                auto hand = [&](auto DB) {
+                    constexpr int db = decltype(DB)::value;
 #pragma unroll
-                for (int I = 0; I < 4; ++I)
-                    out[(4 * (db & 1) + I) * 64 + lane] =
-                        make_float4(A.o[db][4 * I], A.o[db][4 * I + 1], A.o[db][4 * I + 2], A.o[db][4 * I + 3]);
-            };
-            if (grp == 0) {
-                hand(std::integral_constant<int, 2>{});
-                hand(std::integral_constant<int, 3>{});
-            } else {
-                hand(std::integral_constant<int, 0>{});
-                hand(std::integral_constant<int, 1>{});
+                    for (int I = 0; I < 4; ++I)
+                        out[(4 * (db & 1) + I) * 64 + lane] =
+                            make_float4(A.o[db][4 * I] * f, A.o[db][4 * I + 1] * f, A.o[db][4 * I + 2] * f, A.o[db][4 * I + 3] * f);
+                };
+                if (grp == 0) {
+                    hand(std::integral_constant<int, 2>{});
+                    hand(std::integral_constant<int, 3>{});
+                } else {
+                    hand(std::integral_constant<int, 0>{});
+                    hand(std::integral_constant<int, 1>{});
+                }
+                float* s = xs(grp);
+                s[lane] = A.m_s;
+                s[64 + lane] = A.m_t;
+                s[128 + lane] = A.l;
             }
-            float* s = xs(grp);
-            s[lane] = A.m_s;
-            s[64 + lane] = A.m_t;
-            s[128 + lane] = A.l;
-        }
-        lds_barrier();
-        {
-            // both groups form the same statistics, group 0's terms first (FlashAttention.cpp:159-175)
-            const float* so = xs(1 - grp);
-            const float os = so[lane], ot = so[64 + lane], ol = so[128 + lane];
-            const float m0s = grp ? os : A.m_s, m1s = grp ? A.m_s : os;
-            const float m0t = grp ? ot : A.m_t, m1t = grp ? A.m_t : ot;
-            const float l0 = grp ? ol : A.l, l1 = grp ? A.l : ol;
-            const float ms = fmaxf(m0s, m1s);
-            const float a0 = (m0s == kNegInf) ? 0.0f : exp2f(m0s - ms);
-            const float a1 = (m1s == kNegInf) ? 0.0f : exp2f(m1s - ms);
-            const float l = l0 * a0 + l1 * a1;
-            const float mt = fmaxf(m0t, m1t);
-            const bool valid = qrow < L && l > 0.0f;
-            const float inv = valid ? 1.0f / l : 0.0f;
-            const float4* in = xo(1 - grp);
-            uint8_t* orow = obuf + (32 * wq + ln) * kObufRow + 16 * hh;
-            auto fin = [&](auto DB) {
-                constexpr int db = decltype(DB)::value;
+            lds_barrier();
+            {
+                // both groups form the same statistics, group 0's terms first (FlashAttention.cpp:159-175)
+                const float* so = xs(1 - grp);
+                const float os = so[lane], ot = so[64 + lane], ol = so[128 + lane];
+                const float m0s = grp ? os : A.m_s, m1s = grp ? A.m_s : os;
+                const float m0t = grp ? ot : A.m_t, m1t = grp ? A.m_t : ot;
+                const float l0 = grp ? ol : A.l, l1 = grp ? A.l : ol;
+                const float ms = fmaxf(m0s, m1s);
+                const float a0 = (m0s == kNegInf) ? 0.0f : exp2f(m0s - ms);
+                const float a1 = (m1s == kNegInf) ? 0.0f : exp2f(m1s - ms);
+                const float l = l0 * a0 + l1 * a1;
+                const float mt = fmaxf(m0t, m1t);
+                const bool valid = qrow < L && l > 0.0f;
+                const float inv = valid ? 1.0f / l : 0.0f;
+                const float4* in = xo(1 - grp);
+                uint8_t* orow = obuf + (32 * wq + ln) * kObufRow + 16 * hh;
+                auto fin = [&](auto DB) {
+                    constexpr int db = decltype(DB)::value;
 #pragma unroll
-                for (int I = 0; I < 4; ++I) {
-                    const float4 y = in[(4 * (db & 1) + I) * 64 + lane];
-                    const float yv[4] = {y.x, y.y, y.z, y.w};
-                    float v[4];
+                    for (int I = 0; I < 4; ++I) {
+                        const float4 y = in[(4 * (db & 1) + I) * 64 + lane];
+                        const float yv[4] = {y.x, y.y, y.z, y.w};
+                        float v[4];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float own = A.o[db][4 * I + r];
-                        const float x = (db < 2) ? own * a0 + yv[r] * a1 : yv[r] * a0 + own * a1;
-                        const float q = x * inv;  // x / l (l >= 1), with one correction step
-                        const float e = fmaf(fmaf(-q, l, x), inv, q);
-                        v[r] = valid ? (fabsf(q) < kInf ? e : q) : 0.0f;
+                        for (int r = 0; r < 4; ++r) {
+                            const float own = A.o[db][4 * I + r] * f;
+                            const float x = (db < 2) ? own * a0 + yv[r] * a1 : yv[r] * a0 + own * a1;
+                            const float q = x * inv;  // x / l (l >= 1), with one correction step
+                            const float e = fmaf(fmaf(-q, l, x), inv, q);
+                            v[r] = valid ? (fabsf(q) < kInf ? e : q) : 0.0f;
+                        }
+                        *reinterpret_cast<float4*>(orow + 32 * (4 * db + I)) = make_float4(v[0], v[1], v[2], v[3]);
                     }
-                    *reinterpret_cast<float4*>(orow + 32 * (4 * db + I)) = make_float4(v[0], v[1], v[2], v[3]);
+                };
+                if (grp == 0) {
+                    fin(std::integral_constant<int, 0>{});
+                    fin(std::integral_constant<int, 1>{});
+                    if (qrow < T && hh == 0) {
+                        if (a.m) a.m[stat_base + (int64_t)qrow * a.H] = valid ? mt * (a.scale / (scale_here(a.scale) * kLog2e)) : kNegInf;
+                        if (a.l) a.l[stat_base + (int64_t)qrow * a.H] = valid ? l * exp2f(ms - mt) : 0.0f;
+                    }
+                } else {
+                    fin(std::integral_constant<int, 2>{});
+                    fin(std::integral_constant<int, 3>{});
                 }
-            };
-            if (grp == 0) {
-                fin(std::integral_constant<int, 0>{});
-                fin(std::integral_constant<int, 1>{});
-                if (qrow < T && hh == 0) {
-                    if (a.m) a.m[stat_base + (int64_t)qrow * a.H] = valid ? mt * (a.scale / c) : kNegInf;
-                    if (a.l) a.l[stat_base + (int64_t)qrow * a.H] = valid ? l * exp2f(ms - mt) : 0.0f;
-                }
-            } else {
-                fin(std::integral_constant<int, 2>{});
-                fin(std::integral_constant<int, 3>{});
             }
-        }
-        lds_barrier();
-        // the item's 128 output rows: 32 lanes per 512-byte row, 2 rows per store instruction
+            lds_barrier();
+            // the item's 128 output rows: 32 lanes per 512-byte row, 2 rows per store instruction
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int ch = j * kThreads + tid;  // 16-byte chunk ch % 32 of row ch / 32
-            const int r = ch >> 5, cq = ch & 31;
-            const int qr = (j < 4 ? u.qa : u.qb - 64) + r;  // rows 0-63 in j < 4
-            const float4 w = *reinterpret_cast<const float4*>(obuf + r * kObufRow + 16 * cq);
-            if (qr < T) *reinterpret_cast<float4*>(&Og[(int64_t)qr * a.ldo + 4 * cq]) = w;
+            for (int j = 0; j < 8; ++j) {
+                const int ch = j * kThreads + 64 * wave + lane;  // 16-byte chunk ch % 32 of row ch / 32
+                const int r = ch >> 5, cq = ch & 31;
+                const int qr = (j < 4 ? u.qa : u.qb - 64) + r;  // rows 0-63 in j < 4
+                const float4 w = *reinterpret_cast<const float4*>(obuf + r * kObufRow + 16 * cq);
+                if (qr < T) *reinterpret_cast<float4*>(&Og[(int64_t)qr * a.ldo + 4 * cq]) = w;
+            }
         }
         // every wave has read the output tile before the next item's DMA and planes may overwrite it; the output
         // stores need not have completed

@@ -13,7 +13,9 @@
  *
  * Modes:
  *   DT_FP32_EXACT  fp32 inputs/outputs, fp32 products (the attention's from exact
- *                  three-way bf16 splits, with less error than fp32 MFMA),
+ *                  three-way bf16 splits over fp32's whole range: at most 2^-24
+ *                  of a product is left out, and sums come out nearer to 64 bits
+ *                  than fp32 MFMA's; past 2^103 the fp32 MFMA itself),
  *                  fp32 accumulation; parity target 1e-4 of max|O|.
  *   DT_BF16        bf16 Q/K/V/O, bf16 MFMA (v_mfma_f32_32x32x16_bf16) with
  *                  fp32 accumulation and fp32 softmax; parity target 2e-2.

@@ -67,7 +67,7 @@ def test_against_64_bits(B, T, H, causal, path):
 @pytest.mark.parametrize("path", ["recompute", "from_ds"])
 @pytest.mark.parametrize("gs,vs", [(1e-35, 1.0), (1e30, 1e-30), (1.0, 1e-33)])
 def test_scaled_values(gs, vs, path):
-    """Gradients and values far from 1, down to where a split's last part is denormal."""
+    """Gradients and values far from 1, down to where a split's last part would be denormal without a factor."""
     from dirktensor_amd import flash_attention_backward
 
     args, ref = _inputs(1, 200, 2, True, 7, vs=vs, gs=gs)

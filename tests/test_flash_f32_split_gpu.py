@@ -35,9 +35,10 @@ def _rel(a, b):
     return float((a.double() - b).norm() / b.norm())
 
 
-# A split operand is exact and every product's error is below 2^-26, so what is left is fp32 accumulation: at most
-# 2^-24 per addition of a chain of 48 for S and of 12 per 32 keys for O, and exp2's argument rounded at 2^-24 of a
-# score's size (a few tens): 1e-6 in the 2-norm is several times what these sums give.
+# A split operand is exact and the partial products left out come to at most 2^-24 of a product (2^-28 on average), no more
+# than one fp32 rounding. The rest is fp32 accumulation, at most 2^-24 per addition of a chain of 48 for S and of 12 per 32
+# keys for O, and exp2's argument rounded at 2^-24 of a score's size (a few tens): 1e-6 in the 2-norm is several times what
+# these give on random data, where the roundings are independent.
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("B,T,H", [(1, 1, 1), (1, 31, 2), (2, 32, 1), (1, 33, 3), (1, 64, 16), (1, 65, 2), (1, 127, 1),
                                    (2, 129, 2), (1, 191, 1), (1, 256, 8), (1, 385, 2), (1, 1000, 2)])
@@ -54,7 +55,7 @@ def test_against_64_bits(B, T, H, causal):
 
 @pytest.mark.parametrize("vs", [1e-35, 1e-30, 1e30, 1e36])
 def test_scaled_values(vs):
-    """V far from 1, down to where its split's last part is denormal and up to where the unnormalised sum of 150 rows
+    """V far from 1, down to where the last part of its split would be denormal without a factor and up to where the unnormalised sum of 150 rows
     (l is at most a few tens) nears fp32's range; Q and K scaled against each other."""
     from dirktensor_amd import flash_attention_forward
 
