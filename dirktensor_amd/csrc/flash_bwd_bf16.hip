@@ -470,7 +470,6 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
         // From tile 2 on nothing is masked but, with dS stored, the keys past T, a condition fixed per wave:
         // the loop is compiled without the selects when it is false (the same values: dmask is INT_MIN).
         // With 64-key blocks only tile 0, group 0's first, holds the diagonal.
-        const bool tail = kEmitDs && kw + 31 >= T;
         if constexpr (G == 1) {
             step(True_{}, True_{}, st0, st1, q_begin, 1 < n_steps);
             stage_barrier();
@@ -488,7 +487,7 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
                     stage_barrier();
                 }
             };
-            if (tail) rest(True_{});
+            if (kEmitDs && kw + 31 >= T) rest(True_{});
             else rest(False_{});
             if (key < T) {
                 store_rows(dKg, key, a.ld_grad, hh, dk, a.scale);  // dS carries the reference's scale (:293)
@@ -508,8 +507,7 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
                     stage_barrier();
                 }
             };
-            if (tail) rest(True_{});
-            else rest(False_{});
+            rest(std::bool_constant<kEmitDs>{});  // (with dS stored, one loop for both: a second copy spilled 16 registers)
             if (grp == 0) {
                 add_groups(dv, dk, ex, 0, wave, lane);
                 if (key < T) store_rows(dVg, key, a.ld_grad, hh, dv, 1.0f);

@@ -33,7 +33,7 @@
 //
 // What bounds it: the matrix pipe, 192 MFMAs per tile and wave for dK/dV at one wave per SIMD (K, V, dK and dV of 32 keys
 // take 320 of a lane's 512 registers), and with few blocks the longest of them. B = 1, H = 16, us per call against the
-// same decomposition on v_mfma_f32_32x32x2_f32: T = 1000 268 -> 110, T = 2048 568 -> 335, T = 4096 1540 -> 1028.
+// same decomposition on v_mfma_f32_32x32x2_f32: T = 1000 268 -> 109, T = 2048 568 -> 325, T = 4096 1540 -> 998.
 //
 // LDS planes: 32 rows of 256 bytes, 16-byte chunk c of row r at c ^ swz(r), swz(r) = 4*(r & 3) + ((r >> 2) & 3):
 // row-wise fragment reads, transposing reads (ds_read_b64_tr_b16, in the accumulator's row order) and the split's
@@ -324,6 +324,39 @@ __device__ __forceinline__ int lane_here() {
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
     return l;
 }
+// likewise the scale
+__device__ __forceinline__ float scale_here(float s) {
+    asm volatile("" : "+s"(s));
+    return s;
+}
+// The fp32 rows of one (batch, head) for the fp32 instruction, straight from memory (rows at or past T: zeros)
+struct Rows {
+    __amdgpu_buffer_rsrc_t r;
+    uint32_t ld4;
+    __device__ __forceinline__ Rows(const void* base, int b, int h, int T, int ld)
+        : r(make_rsrc(static_cast<const float*>(base) + (int64_t)b * T * ld + (int64_t)h * kD, (uint32_t)T * (uint32_t)ld * 4u)),
+          ld4((uint32_t)ld * 4u) {}
+    __device__ __forceinline__ float at(int row, int dim) const { return load4(r, (uint32_t)row * ld4 + 4u * dim); }
+    // dims 64*hh .. +63 of a row
+    __device__ __forceinline__ void half_row(float4 (&x)[16], int row, int hh) const {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) x[j] = load16(r, (uint32_t)row * ld4 + 256u * hh + 16u * j);
+    }
+    // this lane's row (M) times the lane's half row f (N)
+    __device__ __forceinline__ floatx16 dot(int row, int hh, const float4 (&f)[16]) const {
+        floatx16 c = zero16();
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const float4 x = load16(r, (uint32_t)row * ld4 + 256u * hh + 16u * j);
+            c = mfma_f32(x.x, f[j].x, c);
+            c = mfma_f32(x.y, f[j].y, c);
+            c = mfma_f32(x.z, f[j].z, c);
+            c = mfma_f32(x.w, f[j].w, c);
+        }
+        return c;
+    }
+};
+
 // LDS of one group: the first operand's planes twice, the second's once, and for dK/dV the tile rows' lse2 and delta
 struct GroupLds {
     uint8_t a[2][kPlanes];
@@ -336,12 +369,6 @@ union BwdLds {
     float4 x[4][16][64];  // the groups' exchange (G = 2): 64 KB
 };
 static_assert(sizeof(BwdLds<2>) <= 160 * 1024, "LDS of one CU");
-
-// The kernel's FlashBwdArgs (its first argument) where the launch put it: a reference to the parameter itself, handed
-// to a function that is not inlined, would move the parameter, and every descriptor made from it, out of scalar registers.
-__device__ __forceinline__ const FlashBwdArgs* kernel_args() {
-    return (const FlashBwdArgs*)__builtin_amdgcn_kernarg_segment_ptr();
-}
 
 // The two groups' partial sums: group g keeps own + other of `keep` and hands `give` over (group 0's terms first).
 __device__ __forceinline__ void add_groups(floatx16 (&keep)[4], const floatx16 (&give)[4], float f, float4 (&x)[4][16][64], int grp, int wave, int lane) {
@@ -372,45 +399,38 @@ constexpr int kDsBlockBytes = 128 * kDsRowBytes;  // 32 KB
 struct KvAcc {
     floatx16 dv[4], dk[4];
 };
-// the wave's dK and dV with v_mfma_f32_32x32x2_f32 (k step s of lane half hh is dim 64*hh + s, or one row per half)
-__device__ __noinline__ void slow_dkdv(KvAcc& A, const FlashBwdArgs& a, int bh, int kw, int tile0, int step, int n_tiles, int q_begin, bool emit) {
-    const int lane = threadIdx.x & 63, ln = lane & 31, hh = lane >> 5;
+// The wave's dK and dV with v_mfma_f32_32x32x2_f32, operands straight from memory (k step s of lane half hh is dim 64*hh + s,
+// or one row per half). This and the two below are inlined, with every index a constant: a call, or an element picked at run
+// time, would put registers in scratch memory, which the runtime has to allocate.
+__device__ __forceinline__ void slow_dkdv(KvAcc& A, const FlashBwdArgs& a, int bh, int kw, int tile0, int step, int n_tiles, int q_begin,
+                                          bool emit) {
+    const int lane = lane_here(), ln = lane & 31, hh = lane >> 5;
     const int T = a.T, key = kw + ln, b = bh / a.H, h = bh % a.H;
-    const float c = a.scale * kLog2e;
-    const int64_t qkv = (int64_t)b * T * a.ld_qkv + (int64_t)h * kD, od = (int64_t)b * T * a.ld_o + (int64_t)h * kD;
-    const float *Q = static_cast<const float*>(a.q) + qkv, *G = static_cast<const float*>(a.d_o) + od;
-    const float* kp = static_cast<const float*>(a.k) + qkv + (int64_t)min(key, T - 1) * a.ld_qkv + 64 * hh;
-    const float* vp = static_cast<const float*>(a.v) + qkv + (int64_t)min(key, T - 1) * a.ld_qkv + 64 * hh;
+    const float c = scale_here(a.scale) * kLog2e;
+    const Rows Q(a.q, b, h, T, a.ld_qkv), K(a.k, b, h, T, a.ld_qkv), V(a.v, b, h, T, a.ld_qkv), G(a.d_o, b, h, T, a.ld_o);
+    const __amdgpu_buffer_rsrc_t rl = make_rsrc(a.lse2 + (int64_t)bh * T, (uint32_t)T * 4u);
+    const __amdgpu_buffer_rsrc_t rd = make_rsrc(a.delta + (int64_t)bh * T, (uint32_t)T * 4u);
+#pragma unroll
     for (int db = 0; db < 4; ++db) A.dv[db] = A.dk[db] = zero16();
+    float4 kx[16], vx[16];
+    K.half_row(kx, key, hh);
+    V.half_row(vx, key, hh);
+#pragma unroll 1
     for (int t = tile0; t < n_tiles; t += step) {
         const int q0 = q_begin + t * kTile;
         if (a.causal && q0 + kTile - 1 < kw) continue;
-        floatx16 sc = zero16(), dp = zero16();
-        const bool in = q0 + ln < T;
-        const float* qp = Q + (int64_t)min(q0 + ln, T - 1) * a.ld_qkv + 64 * hh;
-        const float* gp = G + (int64_t)min(q0 + ln, T - 1) * a.ld_o + 64 * hh;
-        for (int s = 0; s < 64; ++s) {
-            const float qx = qp[s], gx = gp[s], kx = kp[s], vx = vp[s];
-            sc = mfma_f32(in ? qx : 0.0f, key < T ? kx : 0.0f, sc);
-            dp = mfma_f32(in ? gx : 0.0f, key < T ? vx : 0.0f, dp);
-        }
+        floatx16 sc = Q.dot(q0 + ln, hh, kx), dp = G.dot(q0 + ln, hh, vx);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            const int qr = q0 + 8 * (i / 4) + 4 * hh + (i % 4);
-            const bool qin = qr < T;
-            const float lse = a.lse2[(int64_t)bh * T + min(qr, T - 1)], del = a.delta[(int64_t)bh * T + min(qr, T - 1)];
+            const int qr = q0 + 8 * (i / 4) + 4 * hh + (i % 4);  // past T: lse2, delta and the rows read as zeros
             const bool masked = (a.causal && key > qr) || (emit && key >= T);
-            const float p = masked ? 0.0f : __builtin_amdgcn_exp2f(sc[i] * c - (qin ? lse : 0.0f));
-            const float ds = p * (dp[i] - (qin ? del : 0.0f));
-            sc[i] = p;
+            const float p = masked ? 0.0f : __builtin_amdgcn_exp2f(sc[i] * c - load4(rl, 4u * qr));
+            const float ds = p * (dp[i] - load4(rd, 4u * qr));
             dp[i] = ds;
-            const float* gr = G + (int64_t)min(qr, T - 1) * a.ld_o + ln;
-            const float* qq = Q + (int64_t)min(qr, T - 1) * a.ld_qkv + ln;
 #pragma unroll
             for (int db = 0; db < 4; ++db) {
-                const float gx = gr[32 * db], qx = qq[32 * db];
-                A.dv[db] = mfma_f32(qin ? gx : 0.0f, p, A.dv[db]);
-                A.dk[db] = mfma_f32(qin ? qx : 0.0f, ds, A.dk[db]);
+                A.dv[db] = mfma_f32(G.at(qr, 32 * db + ln), p, A.dv[db]);
+                A.dk[db] = mfma_f32(Q.at(qr, 32 * db + ln), ds, A.dk[db]);
             }
         }
         if (emit) {
@@ -598,7 +618,7 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
         float f = kDown2;  // takes the operands' factors out
         if (__builtin_amdgcn_ballot_w64(bad) != 0) {
             KvAcc S;
-            slow_dkdv(S, *kernel_args(), bh, kw, grp, G, n_tiles, q_begin, kEmitDs);
+            slow_dkdv(S, a, bh, kw, grp, G, n_tiles, q_begin, kEmitDs);
             settle(S.dv);
             settle(S.dk);
             A = S;
@@ -623,42 +643,30 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
 struct QAcc {
     floatx16 dq[4];
 };
-__device__ __noinline__ void slow_dq(QAcc& A, const FlashBwdArgs& a, int bh, int qw, int tile0, int step, int n_tiles) {
-    const int lane = threadIdx.x & 63, ln = lane & 31, hh = lane >> 5;
+__device__ __forceinline__ void slow_dq(QAcc& A, const FlashBwdArgs& a, int bh, int qw, int tile0, int step, int n_tiles) {
+    const int lane = lane_here(), ln = lane & 31, hh = lane >> 5;
     const int T = a.T, q = qw + ln, b = bh / a.H, h = bh % a.H;
-    const float c = a.scale * kLog2e;
-    const int64_t qkv = (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
-    const float *K = static_cast<const float*>(a.k) + qkv, *V = static_cast<const float*>(a.v) + qkv;
-    const bool in = q < T;
-    const int qc = min(q, T - 1);
-    const float* qp = static_cast<const float*>(a.q) + qkv + (int64_t)qc * a.ld_qkv + 64 * hh;
-    const float* gp = static_cast<const float*>(a.d_o) + (int64_t)b * T * a.ld_o + (int64_t)h * kD + (int64_t)qc * a.ld_o + 64 * hh;
-    const float lse2 = a.lse2[(int64_t)bh * T + qc], delta = a.delta[(int64_t)bh * T + qc];
+    const float c = scale_here(a.scale) * kLog2e;
+    const Rows Q(a.q, b, h, T, a.ld_qkv), K(a.k, b, h, T, a.ld_qkv), V(a.v, b, h, T, a.ld_qkv), G(a.d_o, b, h, T, a.ld_o);
+    const float lse2 = q < T ? a.lse2[(int64_t)bh * T + q] : 0.0f, delta = q < T ? a.delta[(int64_t)bh * T + q] : 0.0f;
     const int lim = a.causal ? min(q, T - 1) : T - 1;
+#pragma unroll
     for (int db = 0; db < 4; ++db) A.dq[db] = zero16();
+    float4 qx[16], gx[16];
+    Q.half_row(qx, q, hh);
+    G.half_row(gx, q, hh);
+#pragma unroll 1
     for (int t = tile0; t < n_tiles; t += step) {
         const int k0 = t * kTile;
         if (a.causal && k0 > qw + 31) break;
-        floatx16 sc = zero16(), dp = zero16();
-        const bool kin = k0 + ln < T;
-        const float* kp = K + (int64_t)min(k0 + ln, T - 1) * a.ld_qkv + 64 * hh;
-        const float* vp = V + (int64_t)min(k0 + ln, T - 1) * a.ld_qkv + 64 * hh;
-        for (int s = 0; s < 64; ++s) {
-            const float qx = qp[s], gx = gp[s], kx = kp[s], vx = vp[s];
-            sc = mfma_f32(kin ? kx : 0.0f, in ? qx : 0.0f, sc);
-            dp = mfma_f32(kin ? vx : 0.0f, in ? gx : 0.0f, dp);
-        }
+        const floatx16 sc = K.dot(k0 + ln, hh, qx), dp = V.dot(k0 + ln, hh, gx);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int key = k0 + 8 * (i / 4) + 4 * hh + (i % 4);
-            const float p = key > lim ? 0.0f : __builtin_amdgcn_exp2f(sc[i] * c - (in ? lse2 : 0.0f));
-            const float ds = p * (dp[i] - (in ? delta : 0.0f));
-            const float* kr = K + (int64_t)min(key, T - 1) * a.ld_qkv + ln;
+            const float p = key > lim ? 0.0f : __builtin_amdgcn_exp2f(sc[i] * c - lse2);
+            const float ds = p * (dp[i] - delta);
 #pragma unroll
-            for (int db = 0; db < 4; ++db) {
-                const float kx = kr[32 * db];
-                A.dq[db] = mfma_f32(key < T ? kx : 0.0f, ds, A.dq[db]);
-            }
+            for (int db = 0; db < 4; ++db) A.dq[db] = mfma_f32(K.at(key, 32 * db + ln), ds, A.dq[db]);
         }
     }
 }
@@ -783,7 +791,7 @@ __device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int 
     float f = kDown2;  // takes the operands' factors out
     if (__builtin_amdgcn_ballot_w64(bad) != 0) {
         QAcc S;
-        slow_dq(S, *kernel_args(), bh, qw, grp, G, n_tiles);
+        slow_dq(S, a, bh, qw, grp, G, n_tiles);
         settle(S.dq);
         A = S;
         f = 1.0f;
@@ -822,25 +830,24 @@ struct DsLds {
     uint8_t k[2][kPlanes];
 };
 
-__device__ __noinline__ void slow_dq_ds(QAcc& A, const FlashBwdArgs& a, int bh, int qw, int n_use) {
-    const int lane = threadIdx.x & 63, ln = lane & 31, hh = lane >> 5;
+__device__ __forceinline__ void slow_dq_ds(QAcc& A, const FlashBwdArgs& a, int bh, int qw, int n_use) {
+    const int lane = lane_here(), ln = lane & 31, hh = lane >> 5;
     const int T = a.T, b = bh / a.H, h = bh % a.H;
-    const float* K = static_cast<const float*>(a.k) + (int64_t)b * T * a.ld_qkv + (int64_t)h * kD;
+    const Rows K(a.k, b, h, T, a.ld_qkv);
     const BwdDsLayout lay(T, a.causal);
     const uint8_t* head = static_cast<const uint8_t*>(a.ds_ws) + (uint64_t)(bh * lay.per_head()) * kDsBlockBytes;
+#pragma unroll
     for (int db = 0; db < 4; ++db) A.dq[db] = zero16();
+#pragma unroll 1
     for (int t = 0; t < n_use; ++t) {
         const int k0 = t * kTile, kb = k0 / 128;
         const uint8_t* col = head + (uint64_t)(lay.block_offset(kb) + (qw / 64 - lay.first_tile(kb))) * kDsBlockBytes + 4 * (qw % 64 + ln);
+#pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int r = 8 * (i / 4) + 4 * hh + (i % 4);
             const float ds = *reinterpret_cast<const float*>(col + (k0 % 128 + r) * kDsRowBytes);
-            const float* kr = K + (int64_t)min(k0 + r, T - 1) * a.ld_qkv + ln;
 #pragma unroll
-            for (int db = 0; db < 4; ++db) {
-                const float kx = kr[32 * db];
-                A.dq[db] = mfma_f32(k0 + r < T ? kx : 0.0f, ds, A.dq[db]);
-            }
+            for (int db = 0; db < 4; ++db) A.dq[db] = mfma_f32(K.at(k0 + r, 32 * db + ln), ds, A.dq[db]);
         }
     }
 }
@@ -913,9 +920,7 @@ __device__ __forceinline__ void dq_ds_block(const FlashBwdArgs& a, int qb_own, i
     const bool bad = q < T && !(finite_probe(A.dq) == 0.0f);
     float f = a.scale * kDown2;
     if (__builtin_amdgcn_ballot_w64(bad) != 0) {
-        QAcc S;
-        slow_dq_ds(S, *kernel_args(), bh, qw, n_use);
-        A = S;
+        slow_dq_ds(A, a, bh, qw, n_use);
         f = a.scale;
     }
     if (q < T) store_rows(dQg, q, a.ld_grad, hh, A.dq, f);

@@ -46,7 +46,7 @@
 //
 // What bounds it: the matrix pipe is busy 6144 of the ~9600 cycles of a step (two waves per SIMD, 96 MFMAs each); the
 // rest is the split (without it 95 us where the kernel takes 118, B = 2, T = 1500, H = 16) and the softmax's first
-// half. Before, on v_mfma_f32_32x32x2_f32: 201 us there, and at B = 1, T = 64, 16.5 us against 13.0. Fragments
+// half. Before, on v_mfma_f32_32x32x2_f32: 201 us there, and at B = 1, T = 64, 16.5 us against 12.1. Fragments
 // prefetched in finer steps, and the tiles staged as fp32 in LDS by DMA instead of through registers, took 128 and 120.
 //
 // Numerics follow the reference: S = scale * Q K^T (FlashAttention.cpp:83-91),
@@ -132,6 +132,10 @@ __device__ __forceinline__ floatx16 mfma(bf16x8 a, bf16x8 b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+__device__ __forceinline__ floatx16 mfma_f32(float a, float b, floatx16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+
 // Row reductions over the two lane halves (lane l and lane l ^ 32 hold the same query): v_permlane32_swap with x as
 // both operands leaves the lower half's value and the upper half's in every lane (the same order in both halves).
 __device__ __forceinline__ float max_halves(float x) {
@@ -150,6 +154,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, ui
 
 __device__ __forceinline__ float4 load16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+
+__device__ __forceinline__ float load4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
 }
 
 // LDS accesses only: vector memory requests in flight (the next tiles, output stores) are not waited for
@@ -176,26 +184,36 @@ struct Acc {
     float m_t, m_s, l;  // this lane half's maximum, the reference point (the same in both halves), this half's sum
 };
 
-// The wave's keys with v_mfma_f32_32x32x2_f32, operands straight from memory: tiles kt0, kt0 + 2, ... of the queries'
-// visible ones. Taken when the split products gave a result that is not finite; scores that are -inf, +inf or NaN
-// in fp32 arithmetic come out as such here.
-__device__ __noinline__ void slow_keys(Acc& A, const float* q, const float* K, const float* V, int ldk, int ldv, int kt0,
-                                       int n_tiles, int qw0, int lim, int L, int T, int causal, float c) {
-    const int lane = threadIdx.x & 63, ln = lane & 31, hh = lane >> 5;
+// The wave's keys with v_mfma_f32_32x32x2_f32, operands straight from memory (rk, rv: the sequence's rows, zeros past it):
+// tiles kt0, kt0 + 2, ... of the queries' visible ones. Taken when the split products gave a result that is not finite;
+// scores that are -inf, +inf or NaN in fp32 arithmetic come out as such here. Inlined, with every index a constant: a call,
+// or an element of A picked at run time, would put registers in scratch memory, which the runtime has to allocate.
+__device__ __forceinline__ void slow_keys(Acc& A, const float* q, __amdgpu_buffer_rsrc_t rk, __amdgpu_buffer_rsrc_t rv, int ldk,
+                                          int ldv, int kt0, int n_tiles, int qw0, int lim, int causal, float c) {
+    const int lane = lane_here(), ln = lane & 31, hh = lane >> 5;
     float m_run = kNegInf, l_run = 0.0f;
+#pragma unroll
     for (int db = 0; db < 4; ++db)
+#pragma unroll
         for (int i = 0; i < 16; ++i) A.o[db][i] = 0.0f;
+    float4 qx[16];  // k step s of lane half hh is dim 64*hh + s
+#pragma unroll
+    for (int j = 0; j < 16; ++j) qx[j] = *reinterpret_cast<const float4*>(q + 64 * hh + 4 * j);
+#pragma unroll 1
     for (int kt = kt0; kt < n_tiles; kt += 2) {
         const int k0 = kt * kBN;
         if (causal && k0 > qw0 + 31) break;
         floatx16 st;
+#pragma unroll
         for (int i = 0; i < 16; ++i) st[i] = 0.0f;
-        // k step s of lane half hh is dim 64*hh + s; keys past L read as zeros (and are masked)
-        const float* kp = K + (int64_t)min(k0 + ln, T - 1) * ldk + 64 * hh;
-        const bool kv = k0 + ln < L;
-        for (int s = 0; s < 64; ++s) {
-            const float kx = kp[s], qx = q[64 * hh + s];
-            st = __builtin_amdgcn_mfma_f32_32x32x2f32(kv ? kx : 0.0f, qx, st, 0, 0, 0);
+        const uint32_t krow = (uint32_t)((k0 + ln) * ldk + 64 * hh) * 4u;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const float4 kx = load16(rk, krow + 16 * j);
+            st = mfma_f32(kx.x, qx[j].x, st);
+            st = mfma_f32(kx.y, qx[j].y, st);
+            st = mfma_f32(kx.z, qx[j].z, st);
+            st = mfma_f32(kx.w, qx[j].w, st);
         }
         float tmax = kNegInf;
 #pragma unroll
@@ -221,16 +239,12 @@ __device__ __noinline__ void slow_keys(Acc& A, const float* q, const float* K, c
         for (int db = 0; db < 4; ++db)
 #pragma unroll
             for (int i = 0; i < 16; ++i) A.o[db][i] *= alpha;
+        const uint32_t vrow = (uint32_t)((k0 + 4 * hh) * ldv + ln) * 4u;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int key = k0 + 8 * (i / 4) + 4 * hh + (i % 4);
-            const float* vp = V + (int64_t)min(key, T - 1) * ldv + ln;
+        for (int i = 0; i < 16; ++i)
 #pragma unroll
-            for (int db = 0; db < 4; ++db) {
-                const float vx = vp[32 * db];
-                A.o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(key < L ? vx : 0.0f, st[i], A.o[db], 0, 0, 0);
-            }
-        }
+            for (int db = 0; db < 4; ++db)
+                A.o[db] = mfma_f32(load4(rv, vrow + (uint32_t)((8 * (i / 4) + (i % 4)) * ldv + 32 * db) * 4u), st[i], A.o[db]);
     }
     A.m_t = A.m_s = m_run;
     A.l = l_run;
@@ -520,10 +534,8 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
             const bool keys = grp * kBN <= lim;
             const bool bad = qrow < L && keys && (!(z == 0.0f) || !(sum_halves(A.l) > 0.0f) || s_min == kNegInf || !scale_fits);
             if (__builtin_amdgcn_ballot_w64(bad) != 0) {
-                Acc S;  // (an object of its own: A stays in registers)
-                slow_keys(S, Qg + (int64_t)min(qrow, T - 1) * a.ldq, Kg, Vg, a.ldk, a.ldv, grp, n_tiles, qw0, lim, L, T,
-                          a.causal, scale_here(a.scale) * kLog2e);
-                A = S;
+                slow_keys(A, Qg + (int64_t)min(qrow, T - 1) * a.ldq, rk, rv, a.ldk, a.ldv, grp, n_tiles, qw0, lim, a.causal,
+                          scale_here(a.scale) * kLog2e);
                 f = fm = 1.0f;
             }
         }
@@ -618,8 +630,8 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
                 if (qr < T) *reinterpret_cast<float4*>(&Og[(int64_t)qr * a.ldo + 4 * cq]) = w;
             }
         }
-        // every wave has read the output tile before the next item's DMA and planes may overwrite it; the output
-        // stores need not have completed
+        // every wave has read the output tile before the next item's planes may overwrite it; the output stores need not
+        // have completed
         lds_barrier();
     }
 }

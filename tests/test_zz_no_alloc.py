@@ -120,7 +120,8 @@ def test_noalloc_above_the_ds_path_threshold(gpu, mode):
 
 
 @pytest.mark.gpu
-def test_noalloc_call_allocates_nothing(gpu):
+@pytest.mark.parametrize("mode", ["bf16", "fp32"])
+def test_noalloc_call_allocates_nothing(gpu, mode):
     """On a fresh context, a no-alloc backward whose row statistics take the whole 8 MiB array (B*T*H = 2^20 rows:
     B=4, T=8192, H=32) leaves the device's free memory unchanged (a warm-up call on a tiny shape loads the kernels
     first), and its gradients are bit-identical to a recompute-path dt_flash_attn_bwd's."""
@@ -128,33 +129,35 @@ def test_noalloc_call_allocates_nothing(gpu):
 
     from dirktensor_amd import Context
 
+    tdt = torch.float32 if mode == "fp32" else torch.bfloat16
+    dtype = C.DT_FP32_EXACT if mode == "fp32" else C.DT_BF16
     B, T, H, causal = 4, 8192, 32, 1
-    print(f"no-alloc backward, free-memory check: B={B} T={T} H={H} bf16", flush=True)
+    print(f"no-alloc backward, free-memory check: B={B} T={T} H={H} {mode}", flush=True)
     ctx = Context(0)
     stream = torch.cuda.current_stream().cuda_stream
     q, k, v, g = (torch.randn(B, T, H, 128, device=gpu, generator=torch.Generator(device=gpu).manual_seed(s))
-                  .to(torch.bfloat16) for s in (11, 12, 13, 14))
+                  .to(tdt) for s in (11, 12, 13, 14))
     o = torch.empty_like(q)
     m = torch.empty((B, T, H), dtype=torch.float32, device=gpu)
     l = torch.empty_like(m)
     C.call("dt_flash_attn_fwd", ctx.handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), m.data_ptr(),
-           l.data_ptr(), B, T, H, 128, SCALE, causal, None, C.DT_BF16, C.DT_MEM_DEVICE, stream)
+           l.data_ptr(), B, T, H, 128, SCALE, causal, None, dtype, C.DT_MEM_DEVICE, stream)
     got = [torch.empty_like(q) for _ in range(3)]
     small = [x[:1, :64, :2].contiguous() for x in (g, o, q, k, v)]
     sm = m[:1, :64, :2].contiguous()
     sl = l[:1, :64, :2].contiguous()
     souts = [torch.empty_like(small[2]) for _ in range(3)]
     _bwd_call("dt_flash_attn_bwd_noalloc", ctx, small[0], small[1], sm, sl, small[2], small[3], small[4], souts, 1, 64,
-              2, causal, C.DT_BF16, stream, True)
+              2, causal, dtype, stream, True)
     torch.cuda.synchronize()
     free0, _ = torch.cuda.mem_get_info()
-    _bwd_call("dt_flash_attn_bwd_noalloc", ctx, g, o, m, l, q, k, v, got, B, T, H, causal, C.DT_BF16, stream, True)
+    _bwd_call("dt_flash_attn_bwd_noalloc", ctx, g, o, m, l, q, k, v, got, B, T, H, causal, dtype, stream, True)
     torch.cuda.synchronize()
     free1, _ = torch.cuda.mem_get_info()
     assert free1 == free0, f"free device memory changed by {free0 - free1} bytes across the no-alloc call"
     ref = [torch.empty_like(q) for _ in range(3)]
     ctx.set_bwd_dq_path("recompute")
-    _bwd_call("dt_flash_attn_bwd", ctx, g, o, m, l, q, k, v, ref, B, T, H, causal, C.DT_BF16, stream, False)
+    _bwd_call("dt_flash_attn_bwd", ctx, g, o, m, l, q, k, v, ref, B, T, H, causal, dtype, stream, False)
     torch.cuda.synchronize()
     for name, a, b in zip(("dQ", "dK", "dV"), got, ref):
         assert torch.isfinite(a.float()).all()
