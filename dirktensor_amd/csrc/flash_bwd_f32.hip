@@ -177,8 +177,9 @@ __device__ __forceinline__ LaneAddr lane_addr(int lane) {
 
 // The product over the head dimension: rows of a tile (M) times the lane's row f (N), the five small partial products
 // of every chunk first, then the large one (whose plane is read again). Fragments are read one chunk ahead; ride(I)
-// is issued beside bundle I of 12.
-template <typename Ride>
+// is issued beside bundle I of 12. kSwap: partial products in the order that the product with the roles exchanged has, so
+// that S and dP, and with them dS, have the same bits in the dK/dV pass (tiles of Q and dO) and the dQ pass (of K and V).
+template <bool kSwap = false, typename Ride>
 __device__ __forceinline__ floatx16 dot_rows(const uint8_t* tile, const LaneAddr& LA, const Frag3 (&f)[8], Ride&& ride) {
     auto rd = [&](int cc, int p) {
         return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(tile + LA.raddr[cc] + p * kPlane));
@@ -193,11 +194,19 @@ __device__ __forceinline__ floatx16 dot_rows(const uint8_t* tile, const LaneAddr
         if constexpr (cc + 1 < 8) x[(cc + 1) & 1] = rd3(cc + 1);
         else xh[0] = rd(0, 0), xh[1] = rd(1, 0);
         const Frag3 k = x[cc & 1];
-        c = mfma(k.l, f[cc].h, c);
-        c = mfma(k.h, f[cc].l, c);
-        c = mfma(k.m, f[cc].m, c);
-        c = mfma(k.m, f[cc].h, c);
-        c = mfma(k.h, f[cc].m, c);
+        if constexpr (!kSwap) {
+            c = mfma(k.l, f[cc].h, c);
+            c = mfma(k.h, f[cc].l, c);
+            c = mfma(k.m, f[cc].m, c);
+            c = mfma(k.m, f[cc].h, c);
+            c = mfma(k.h, f[cc].m, c);
+        } else {
+            c = mfma(k.h, f[cc].l, c);
+            c = mfma(k.l, f[cc].h, c);
+            c = mfma(k.m, f[cc].m, c);
+            c = mfma(k.h, f[cc].m, c);
+            c = mfma(k.m, f[cc].h, c);
+        }
         ride(CC);
         DT_BUNDLE_END;
     });
@@ -744,13 +753,13 @@ __device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int 
         floatx16 sc, dp;
         Words3 dw;
         if (visible) {
-            sc = dot_rows(kt, LA, qf, [&](auto I) {  // S^T = K Q^T
+            sc = dot_rows<true>(kt, LA, qf, [&](auto I) {  // S^T = K Q^T
                 constexpr int i = decltype(I)::value;
                 if constexpr (G == 2 && i < 8) move_k(i);
                 if constexpr (G == 1 && i < 8 && (i & 1)) move_k(i / 2);
             });
             const int emask = lim - (k0 + 4 * hh);  // element i (key k0 + 8*(i/4) + 4*hh + i%4) is masked past it
-            dp = dot_rows(my.b, LA, gf, [&](auto I) {  // dP^T = V dO^T; P^T in place of S^T
+            dp = dot_rows<true>(my.b, LA, gf, [&](auto I) {  // dP^T = V dO^T; P^T in place of S^T
                 constexpr int i = decltype(I)::value;
                 if constexpr (i < 8) {
 #pragma unroll
