@@ -111,6 +111,20 @@ struct BwdDsLayout {
 inline size_t flash_bwd_ds_bytes(int B, int H, int T, int causal, int elem_bytes) {
     return (size_t)B * H * (size_t)BwdDsLayout(T, causal).per_head() * (size_t)(128 * 64 * elem_bytes);
 }
+// Whether a backward runs workgroups of two groups, which own 64 rows and split the tiles, instead of one group that owns 128.
+// Half the longest chain of tiles, for twice the workgroups and an addition at the end:
+// - where both passes' 64-row blocks fit one round of the CUs, that is half the time (bf16 H = 16, T = 512 24.3 -> 17.9 us per
+//   call, full attention 24.4 -> 18.0; fp32 78.4 -> 51.4);
+// - past that a second round follows, which costs as much as was saved where all blocks are equally long (full attention, H =
+//   16, T = 777: bf16 33.2 -> 41.2, fp32 117 -> 145; causal, 96 heads, T = 128: bf16 16.0 -> 18.7, fp32 36 -> 40) but
+//   not where causal blocks differ, as long as the 128-row blocks would leave CUs idle (H = 16, T = 1000: bf16 38 -> 33, fp32
+//   142 -> 108; 24 heads, T = 512: 25.2 -> 23.0 and 81 -> 57; with more blocks, 32 heads, T = 640: 29.6 -> 35.7). min_rows: from
+//   where on the saving outweighs the addition (bf16, 64 heads: T = 256 19.5 -> 21.6; fp32, 64 heads, T = 192 42.7 -> 40.5).
+inline bool flash_bwd_two_groups(int64_t BH, int T, int causal, int cus, int min_rows) {
+    const int64_t n64 = (T + 63) / 64, n128 = (T + 127) / 128;
+    return 2 * BH * n64 <= cus || (causal && T > min_rows && 2 * BH * n128 <= cus);
+}
+constexpr int kBwdGroupRowsBf16 = 256, kBwdGroupRowsF32 = 128;
 int launch_flash_bwd_bf16(const FlashBwdArgs& a, hipStream_t stream);
 int launch_flash_bwd_f32(const FlashBwdArgs& a, hipStream_t stream);
 

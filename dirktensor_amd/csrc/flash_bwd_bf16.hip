@@ -967,10 +967,8 @@ int launch_flash_bwd_bf16(const FlashBwdArgs& a, hipStream_t stream) {
     if (2 * blocks > 0x7fffffff) return set_error(DT_ERR_UNSUPPORTED, "too many workgroups");
     int cus = 0;
     DT_TRY(persistent_grid(0x7fffffff, &cus));
-    // Two groups per workgroup where both passes' 128-row blocks together are at most one per CU (B*H = 16, us per call,
-    // two groups / one: T = 512 18.7 / 24.7, T = 1000 34.4 / 39.1); past that the CUs are busy and the smaller blocks
-    // fetch every tile for fewer rows (T = 1280 51.9 / 46.6, T = 2048 97.5 / 80.6; B*H = 32, T = 777 50.1 / 40.9).
-    return 2 * blocks <= cus ? launch<2>(a, blocks, cus, stream) : launch<1>(a, blocks, cus, stream);
+    return flash_bwd_two_groups((int64_t)a.B * a.H, a.T, a.causal, cus, kBwdGroupRowsBf16) ? launch<2>(a, blocks, cus, stream)
+                                                                                   : launch<1>(a, blocks, cus, stream);
 }
 
 }  // namespace dt

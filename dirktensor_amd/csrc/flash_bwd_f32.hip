@@ -20,7 +20,7 @@
 //
 // A workgroup is 4 waves in G groups; the groups hold the same block and take alternate tiles, each with LDS of its
 // own, and add up their partial gradients at the end. G = 1: blocks of 128 rows; G = 2: blocks of 64, twice as many
-// of half the length, where 128-row blocks would leave the longest one to set the time (the rule is at the launch).
+// of half the length, where 128-row blocks would leave the longest one to set the time (flash_bwd_two_groups).
 //
 // A streamed tile passes through registers: a thread loads four floats of a row at a time, a phase or two ahead,
 // splits them and writes the three planes under the MFMAs of another product. Per tile and wave (dK/dV):
@@ -1002,11 +1002,8 @@ int launch_flash_bwd_f32(const FlashBwdArgs& a, hipStream_t stream) {
     if (2 * blocks > 0x7fffffff) return set_error(DT_ERR_UNSUPPORTED, "too many workgroups");
     int cus = 0;
     DT_TRY(persistent_grid(0x7fffffff, &cus));
-    // Two groups per workgroup where both passes' 128-row blocks together are at most one per CU: there the longest
-    // block sets the time (B*H = 16, us per call, two groups / one: T = 1000, 128 blocks per pass, 112 / 143; T = 1280,
-    // 160 blocks, 176 / 179). With more blocks the CUs are busy, and the smaller blocks split every tile for fewer rows
-    // (B*H = 48, T = 400, 192 blocks: 88 / 79; T = 2048, 256 blocks: 383 / 335).
-    return 2 * blocks <= cus ? launch<2>(a, blocks, cus, stream) : launch<1>(a, blocks, cus, stream);
+    return flash_bwd_two_groups((int64_t)a.B * a.H, a.T, a.causal, cus, kBwdGroupRowsF32) ? launch<2>(a, blocks, cus, stream)
+                                                                                   : launch<1>(a, blocks, cus, stream);
 }
 
 }  // namespace dt

@@ -1,5 +1,5 @@
-"""bf16 backward on both sides of the rule that picks one or two groups per workgroup (128-row blocks of one pass against
-half the CUs), at edges of the 64-row blocks and tiles, against gradients in 64 bits from the same inputs."""
+"""bf16 backward on both sides of the rule that picks one or two groups per workgroup (flash_bwd_two_groups), at edges of the
+64-row blocks and tiles, against gradients in 64 bits from the same inputs."""
 
 import math
 
