@@ -71,7 +71,6 @@ constexpr int kPlanes = 3 * kPlane;              // h, m, l
 constexpr int kBlk = 128;                        // rows owned by a workgroup of one group
 constexpr int kThreads = 256;
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kNegInf = -__builtin_huge_valf();
 constexpr float kUp = 0x1p24f;      // the operands' factor
 constexpr float kDown2 = 0x1p-48f;  // takes it out of a product
 constexpr int kBufferDword3 = 0x00020000;  // raw buffer, 32-bit data format (gfx9 family)
@@ -498,7 +497,7 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
     Frag3 kf[8], vf[8];
     load_frags(kf, Kg, key, T, a.ld_qkv, hh);
     load_frags(vf, Vg, key, T, a.ld_qkv, hh);
-    float s_min = 0.0f;  // the lowest score
+    uint32_t s_low = 0;  // the lowest score, as the largest bit pattern (-inf: 0xff800000; without a sign: any)
     KvAcc A;
 #pragma unroll
     for (int db = 0; db < 4; ++db) A.dv[db] = A.dk[db] = zero16();
@@ -577,7 +576,7 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
                 if constexpr (i < 4) {
 #pragma unroll
                     for (int e = 4 * i; e < 4 * i + 4; ++e) {
-                        s_min = fminf(s_min, sc[e]);
+                        s_low = max(s_low, __float_as_uint(sc[e]));
                         const float p = __builtin_amdgcn_exp2f(fmaf(sc[e], c * kDown2, -L[e]));
                         sc[e] = dmask > 8 * (e / 4) + (e % 4) ? 0.0f : p;
                     }
@@ -623,7 +622,7 @@ __device__ __forceinline__ void dkdv_block(const FlashBwdArgs& a, int kb_own, in
     {
         const int lane = lane_here(), hh = lane >> 5, key = kw + (lane & 31);
         const float z = finite_probe(A.dv) + finite_probe(A.dk);
-        const bool bad = key < T && (!(z == 0.0f) || s_min == kNegInf || !scale_fits(a.scale));
+        const bool bad = key < T && (!(z == 0.0f) || s_low >= 0xff800000u || !scale_fits(a.scale));
         float f = kDown2;  // takes the operands' factors out
         if (__builtin_amdgcn_ballot_w64(bad) != 0) {
             KvAcc S;
@@ -716,7 +715,7 @@ __device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int 
     Frag3 qf[8], gf[8];
     load_frags(qf, static_cast<const float*>(a.q) + qkv, q, T, a.ld_qkv, hh);
     load_frags(gf, Gg, q, T, a.ld_o, hh);
-    float s_min = 0.0f;  // the lowest score
+    uint32_t s_low = 0;  // the lowest score, as the largest bit pattern (-inf: 0xff800000; without a sign: any)
     const float lse2 = q < T ? a.lse2[(int64_t)bh * T + q] : 0.0f;
     const float delta = q < T ? a.delta[(int64_t)bh * T + q] : 0.0f;
     const int lim = a.causal ? min(q, T - 1) : T - 1;  // keys > lim are masked
@@ -764,7 +763,7 @@ __device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int 
                 if constexpr (i < 8) {
 #pragma unroll
                     for (int e = 2 * i; e < 2 * i + 2; ++e) {
-                        s_min = fminf(s_min, sc[e]);
+                        s_low = max(s_low, __float_as_uint(sc[e]));
                         const float p = __builtin_amdgcn_exp2f(fmaf(sc[e], c * kDown2, -lse2));
                         sc[e] = 8 * (e / 4) + (e % 4) > emask ? 0.0f : p;
                     }
@@ -796,7 +795,7 @@ __device__ __forceinline__ void dq_block(const FlashBwdArgs& a, int qb_own, int 
         lds_barrier();  // the next tile's planes are written
     }
 
-    const bool bad = q < T && (!(finite_probe(A.dq) == 0.0f) || s_min == kNegInf || !scale_fits(a.scale));
+    const bool bad = q < T && (!(finite_probe(A.dq) == 0.0f) || s_low >= 0xff800000u || !scale_fits(a.scale));
     float f = kDown2;  // takes the operands' factors out
     if (__builtin_amdgcn_ballot_w64(bad) != 0) {
         QAcc S;

@@ -374,7 +374,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
         A.m_t = kNegInf;
         A.m_s = kNegInf;
         A.l = 0.0f;
-        float s_min = 0.0f;  // the lowest score
+        uint64_t low = 0;  // the lanes that had a score of -inf
 
         lds_barrier();
 
@@ -431,8 +431,15 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
                     DT_BUNDLE_END;
                 });
 
+                {  // (as bit patterns: below 0 a lower score is a larger one, -inf 0xff800000)
+                    uint32_t u0 = __float_as_uint(st[0]), u1 = __float_as_uint(st[1]);
 #pragma unroll
-                for (int i = 0; i < 16; ++i) s_min = fminf(s_min, st[i]);
+                    for (int i = 2; i < 16; i += 2) {
+                        u0 = max(u0, __float_as_uint(st[i]));
+                        u1 = max(u1, __float_as_uint(st[i + 1]));
+                    }
+                    low |= __builtin_amdgcn_ballot_w64(max(u0, u1) >= 0xff800000u);
+                }
                 if (k0 + kBN > L || (a.causal && k0 + kBN - 1 > qw0)) {  // diagonal / ragged tail only
                     asm volatile("");  // keeps this block a branch
 #pragma unroll
@@ -531,9 +538,9 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a,
             for (int db = 0; db < 4; ++db)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) z = fmaf(A.o[db][i], 0.0f, z);
-            const bool keys = grp * kBN <= lim;
-            const bool bad = qrow < L && keys && (!(z == 0.0f) || !(sum_halves(A.l) > 0.0f) || s_min == kNegInf || !scale_fits);
-            if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+            const bool keys = qrow < L && grp * kBN <= lim;
+            const bool bad = keys && (!(z == 0.0f) || !(sum_halves(A.l) > 0.0f) || !scale_fits);
+            if ((__builtin_amdgcn_ballot_w64(bad) | (low & __builtin_amdgcn_ballot_w64(keys))) != 0) {
                 slow_keys(A, Qg + (int64_t)min(qrow, T - 1) * a.ldq, rk, rv, a.ldk, a.ldv, grp, n_tiles, qw0, lim, a.causal,
                           scale_here(a.scale) * kLog2e);
                 f = fm = 1.0f;
