@@ -581,6 +581,13 @@ int launch_ce_loss(const float* logits, const int32_t* target, float* term, floa
     const float inv = count > 0 ? 1.0f / (float)count : __builtin_nanf("");  // 0 / 0 as in the reference
     // the smallest form that holds the row; longer rows are read twice
     const bool vec = V % 4 == 0 && ((uintptr_t)logits | (uintptr_t)grad) % 16 == 0;
+    // Without a gradient every form reads a row once, and the one with LDS, of which a CU holds a single workgroup, loses
+    // against 256 threads a row from about two rows per CU on (V = 120000, us per call: 2047 rows 334 against 203, 1024 187
+    // against 135, 512 95 against 91, 400 86 against 89, 256 62 against 84). Unaligned rows, read in single floats there, stay
+    // (V = 110001: 2047 rows 320 against 321, 1024 180 against 283).
+    int cus = 0;
+    DT_TRY(persistent_grid(0x7fffffff, &cus));
+    const bool lds = grad || !vec || rows < 2 * cus;
     auto reg = [&](auto kernel, int threads) {
         hipLaunchKernelGGL(kernel, dim3(rows), dim3(threads), 0, s, logits, target, term, grad, V, inv);
     };
@@ -593,7 +600,7 @@ int launch_ce_loss(const float* logits, const int32_t* target, float* term, floa
     else if (n <= 4 * 13) reg(ce_rows_reg_kernel<1024, 13, 0>, 1024);
     else if (n <= 4 * 19) reg(ce_rows_reg_kernel<1024, 19, 0>, 1024);
     else if (n <= 4 * 25) reg(ce_rows_reg_kernel<1024, 25, 0>, 1024);
-    else if (n <= 4 * 32) reg(ce_rows_reg_kernel<1024, 23, 9>, 1024);
+    else if (n <= 4 * 32 && lds) reg(ce_rows_reg_kernel<1024, 23, 9>, 1024);
     else if (vec) hipLaunchKernelGGL(ce_rows_kernel<true>, dim3(rows), dim3(256), 0, s, logits, target, term, grad, V, inv);
     else hipLaunchKernelGGL(ce_rows_kernel<false>, dim3(rows), dim3(256), 0, s, logits, target, term, grad, V, inv);
     DT_HIP_TRY(hipGetLastError());

@@ -52,3 +52,19 @@ def test_rows_off_16_bytes():
     loss, grad = ce_loss(lg, tok, PAD, with_grad=True)
     loss2, grad2 = ce_loss(lg.clone(), tok, PAD, with_grad=True)
     assert loss == loss2 and torch.equal(grad, grad2)
+
+
+@pytest.mark.parametrize("V,offset", [(102400, 0), (102404, 0), (110001, 0), (110004, 1), (131072, 0), (131076, 0)])
+@pytest.mark.parametrize("rows", [40, 600])
+def test_loss_without_gradient(rows, V, offset):
+    """Few and many rows (the form for long rows depends on their number), aligned and not; tolerance as above."""
+    from dirktensor_amd import ce_loss
+
+    buf = 3.0 * torch.randn((rows + 1) * V + offset, generator=torch.Generator(device="cuda").manual_seed(V), device="cuda")
+    lg = buf[offset:].view(1, rows + 1, V)
+    tok = np.random.default_rng(V).integers(1, V, size=(1, rows + 1)).astype(np.int32)
+    loss = ce_loss(lg, tok, PAD)
+    z = lg[0, :-1]
+    tgt = torch.as_tensor(tok[0, 1:].astype(np.int64), device="cuda")
+    want = float(np.mean([float(torch.logsumexp(r.double(), -1) - r[t].double()) for r, t in zip(z, tgt)]))
+    assert abs(loss - want) <= 1e-6 * abs(want) + 1e-7
