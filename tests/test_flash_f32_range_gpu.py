@@ -7,6 +7,8 @@ import math
 
 import pytest
 
+from parity import attention64, attention_bwd64
+
 torch = pytest.importorskip("torch")
 
 pytestmark = pytest.mark.gpu
@@ -19,49 +21,19 @@ def _randn(shape, n, seed):
     return [torch.randn(shape, generator=g, device="cuda") for _ in range(n)]
 
 
-def _tr(t):
-    return t.transpose(-1, -2).contiguous()
-
-
-def _forward64(q, k, v, scale, causal):
-    """(o, m, l) in 64 bits, [B, H, T, D] and [B, H, T]."""
-    Q, K, V = (t.double().permute(0, 2, 1, 3).contiguous() for t in (q, k, v))
-    s = Q @ _tr(K) * scale
-    if causal:
-        T = s.shape[-1]
-        s = s.masked_fill(torch.ones(T, T, dtype=torch.bool, device=s.device).triu(1), float("-inf"))
-    m = s.amax(-1)
-    p = torch.exp(s - m[..., None])
-    l = p.sum(-1)
-    return p @ V / l[..., None], m, l
-
-
-def _backward64(do, o, m, l, q, k, v, scale, causal):
-    """(dq, dk, dv) in 64 bits, [B, H, T, D], from the forward's results as fp32 ([B, T, H, D] and [B, T, H])."""
-    Q, K, V, G, O = (t.double().permute(0, 2, 1, 3).contiguous() for t in (q, k, v, do, o))
-    M, L = (t.double().permute(0, 2, 1) for t in (m, l))
-    s = Q @ _tr(K) * scale
-    if causal:
-        T = s.shape[-1]
-        s = s.masked_fill(torch.ones(T, T, dtype=torch.bool, device=s.device).triu(1), float("-inf"))
-    p = torch.exp(s - M[..., None]) / L[..., None]
-    ds = p * (G @ _tr(V) - (G * O).sum(-1, keepdim=True)) * scale
-    return ds @ K, _tr(ds) @ Q, _tr(p) @ G
-
-
 def _bwd(do, q, k, v, scale, causal, path, q64=None, k64=None):
     """The kernel's gradients and the 64-bit ones, [B, H, T, D]. (q64, k64: rows of the same scores for the 64-bit side.)"""
     from dirktensor_amd import Context, flash_attention_backward
 
     q64, k64 = q if q64 is None else q64, k if k64 is None else k64
-    o, m, l = _forward64(q64, k64, v, scale, causal)
+    o, m, l = attention64(q64, k64, v, scale, causal)
     stats = (o.permute(0, 2, 1, 3).float().contiguous(), m.permute(0, 2, 1).float().contiguous(),
              l.permute(0, 2, 1).float().contiguous())
     ctx = Context(0)
     ctx.set_bwd_dq_path(path)
     r = flash_attention_backward(do, *stats, q, k, v, scale, causal, ctx=ctx)
     got = [t.double().permute(0, 2, 1, 3) for t in (r.d_Q, r.d_K, r.d_V)]
-    return got, _backward64(do, *stats, q64, k64, v, scale, causal)
+    return got, attention_bwd64(do, *stats, q64, k64, v, scale, causal)
 
 
 def _norm(x, dim):
@@ -84,7 +56,7 @@ def test_forward_small_and_large_columns_of_v(causal):
     for d, s in ((3, 1e-36), (40, 1e-33), (77, 1e-30), (101, 1e20)):
         v[..., d] *= s
     r = flash_attention_forward(q, k, v, SCALE, causal)
-    o, _, _ = _forward64(q, k, v, SCALE, causal)
+    o, _, _ = attention64(q, k, v, SCALE, causal)
     got = r.output.double().permute(0, 2, 1, 3)
     unit = _norm(o, ROWS)
     assert _rel(got / unit, o / unit, ROWS) < 1e-6
@@ -99,7 +71,7 @@ def test_forward_small_scores(qs, ks, scale):
     q, k, v = _randn((1, 150, 2, 128), 3, 2)
     q, k = q * qs, k * ks
     r = flash_attention_forward(q, k, v, scale, True)
-    o, m, _ = _forward64(q, k, v, scale, True)
+    o, m, _ = attention64(q, k, v, scale, True)
     m = m.permute(0, 2, 1)
     unit = m.abs().max()
     if unit > 1e-37:  # (denormal results hold fewer bits)
@@ -128,7 +100,7 @@ def test_forward_small_probability_of_a_large_value():
     v[..., 64:] = 0.0
     v[:, 5, :, 64:] = 2.0 ** 90
     r = flash_attention_forward(q, k, v, SCALE, False)
-    o, _, _ = _forward64(q, k, v, SCALE, False)
+    o, _, _ = attention64(q, k, v, SCALE, False)
     got = r.output.double().permute(0, 2, 1, 3)
     assert _rel(got[..., 64:], o[..., 64:], (0, 1, 2, 3)) < 3e-5
     assert _rel(got[..., :64], o[..., :64], (0, 1, 2, 3)) < 1e-6
@@ -205,7 +177,7 @@ def test_forward_large_values(which):
     big = 2.0 ** 110
     q, k, v = {"q": (q * big, k / big, v), "k": (q / big, k * big, v), "v": (q, k, v * big)}[which]
     r = flash_attention_forward(q, k, v, SCALE, True)
-    o, m, l = _forward64(q, k, v, SCALE, True)
+    o, m, l = attention64(q, k, v, SCALE, True)
     unit = o.abs().max()
     assert _rel(r.output.double().permute(0, 2, 1, 3) / unit, o / unit, (0, 1, 2, 3)) < 1e-6
 
@@ -224,7 +196,7 @@ def test_scores_that_overflow_on_the_way(H):
     for d, s in ((0, -1.0), (2, -1.0), (16, 1.0), (18, 1.0)):
         q[..., d], k[..., d] = 2.0 ** 39, s * 0.75 * 2.0 ** 41
     r = flash_attention_forward(q, k, v, SCALE, True)
-    o, _, _ = _forward64(q0, k0, v, SCALE, True)
+    o, _, _ = attention64(q0, k0, v, SCALE, True)
     assert _rel(r.output.double().permute(0, 2, 1, 3), o, (0, 1, 2, 3)) < 1e-6
     got, want = _bwd(do, q, k, v, SCALE, True, "recompute", q0, k0)
     assert _rel(got[2], want[2], (0, 1, 2, 3)) < 3e-6
